@@ -499,8 +499,8 @@ struct HamProducer final : KeyProducer {
     const uint32_t* q;
     const uint32_t* x;
     uint32_t Q, N, W;
-    va_status fallback_pass(const FbArgs& a, int pass) override {
-        return fb_launch_pass(ctx, FbHam{q, x, N, W}, a, pass);
+    va_status fallback(const FbArgs& a, const SelectArgs& sel) override {
+        return fb_launch(ctx, FbHam{q, x, N, W}, a, sel);
     }
     // distances are at most 32 W
     uint32_t key_bits() const override { return 32u - uint32_t(__builtin_clz(32u * W)); }

@@ -3,25 +3,39 @@
 //
 // A scan that selects from per-query candidate lists lists the queries whose list outgrew its
 // capacity (a device count and a device list of query ids).  The fallback finds their exact
-// top-k in a fixed number of launches whose work follows that device count; with no overflowed
-// query every workgroup exits at once.  Each pass recomputes the keys of (overflowed query,
-// database row) pairs with the producer's own arithmetic — bit-identical to its scan:
+// top-k in one launch whose work follows that device count; with no overflowed query every
+// workgroup exits at once.  Its phases recompute the keys of (overflowed query, database row)
+// pairs with the producer's own arithmetic — bit-identical to its scan:
+//   clear        the listed queries' histograms, state and list lengths;
 //   pass 0 .. 2  histograms of key bits 31:21, 20:10 and 9:0 of the keys in the bucket chosen so
 //                far: after pass 2 the k-th smallest key K and how many keys equal to K the
 //                top-k takes ("need") are known;
 //   pass 3       collects every (key, id) with key <= K, and a histogram of the ids of the ties;
 //   pass 4       (rows whose ties overflowed the list) collects key < K, and the ties whose id is
 //                below the first id-histogram edge that holds `need` of them;
-//   then the selection kernel orders each row's list by (key, id) and writes the top-k.
-// Between passes the last workgroup to finish (a completion ticket, no waiting) turns the
-// histograms into the next pass's bucket.  Work items are 32 queries x 32 database rows in the
-// 32x32 MFMA output layout: lane (l, h) holds query slot l % 32 and rows 8j + 4h + e.
+//   select       each row's list ordered by (key, id): its top-k.
+// After each pass 0 .. 3 a resolve phase turns each slot's histograms into the next pass's bucket.
+// The last workgroup to finish a phase publishes it.  Work items of a pass are 32 queries x 32
+// database rows in the 32x32 MFMA output layout: lane (l, h) holds query slot l % 32 and rows
+// 8j + 4h + e.
+//
+// One launch instead of seven (clear, five passes, selection; the screened searches also forked
+// them onto another stream and joined it): a search that overflows nothing, which is nearly every
+// search, paid their dispatches on its critical path.  Measured per search: 5,000 x 128, Q = 1
+// 106 -> 54 us; 100,003 x 768, Q = 100 183 -> 164; 10M int8 rows, Q = 32 1,480 -> 1,468.  With
+// every query overflowing: 200,000 x 128, Q = 64 6.0 -> 3.3 ms; 100,000 x 96, Q = 256 7.4 -> 2.9
+// (the resolve was one workgroup's for all slots); Q = 1 1.87 -> 1.86.  Phases are ordered by tickets, not by a barrier of the whole
+// grid: a workgroup takes the next (phase, share) ticket and waits until the phase before it is
+// published.  Every ticket of an earlier phase was taken earlier, by a workgroup that is running
+// and waits only on phases earlier still, so the wait ends whether or not the whole grid is
+// resident at once (other streams and contexts may hold the rest of the chip).
 #pragma once
 
 #include <algorithm>
 
 #include "va_distop.hpp"
 #include "va_internal.hpp"
+#include "va_select.hpp"
 
 namespace va {
 
@@ -38,11 +52,17 @@ struct FbArgs {
     uint32_t* cnt = nullptr;           // [rmax] list lengths
     uint32_t* lkey = nullptr;          // [rmax][cap]
     uint32_t* lid = nullptr;           // [rmax][cap]
-    uint32_t* done = nullptr;          // [8] completion tickets, one per pass
-    uint32_t grid = kFbGrid;           // workgroups per pass (fewer for a few rows: each launch that
-                                       // finds nothing overflowed still costs its dispatch)
+    uint32_t* done = nullptr;          // [8] shares of each pass done
+    uint32_t* sync = nullptr;          // phase words (FbSync), cleared before the scan
+    uint32_t grid = kFbGrid;           // workgroups (fewer for a few rows: a launch that finds
+                                       // nothing overflowed still costs its dispatch)
     const uint8_t* skip = nullptr;     // excluded rows: their keys are kAbsentKey
 };
+// tickets taken; shares of the clear done; whether a slot's ties overflowed its list (pass 4 runs);
+// shares of pass p's resolve done (FBS_RESOLVED + p); phase p published (FBS_READY + p)
+enum FbSync : int { FBS_TICKET = 0, FBS_CLEARED = 1, FBS_TIES = 2, FBS_RESOLVED = 4, FBS_READY = 8 };
+constexpr uint32_t kFbPhases = 2 * kFbPasses + 1;  // clear, then pass p and its resolve (pass 4: none), select
+static_assert(kFbSync + FBS_READY + kFbPhases <= kZeroWords, "the phase words fit the overflow words");
 enum FbState : int { FB_PREFIX = 0, FB_NEED = 1, FB_K = 2, FB_EDGE = 3, FB_OVF = 4 };
 static_assert(kFbKeyBins == 2048, "the passes' key histograms have 2048 bins");
 // (the pass count, grid, bins and buffer sizes: fb_geometry / fb_bytes in va_plan.hpp)
@@ -415,41 +435,39 @@ __device__ inline void fb_find_bin(const uint32_t* h, uint32_t bins, uint32_t ne
     __syncthreads();
 }
 
-// The last workgroup of a pass: the histograms of every slot -> the next pass's state.
-__device__ inline void fb_resolve(const FbArgs& a, int pass, uint32_t n) {
+// After pass 0 .. 3: a slot's histograms -> the next pass's state (one workgroup).
+__device__ inline void fb_resolve(const FbArgs& a, int pass, uint32_t s) {
     __shared__ uint32_t sh[258];
-    for (uint32_t s = 0; s < n; ++s) {
-        uint32_t* st = a.st + int64_t(s) * 8;
-        uint32_t* h = a.hist + int64_t(s) * 2048;
-        if (pass <= 2) {
-            const uint32_t bins = pass == 2 ? 1024u : 2048u;
-            const uint32_t need = pass == 0 ? a.k : st[FB_NEED];
-            uint32_t b, before;
-            fb_find_bin(h, bins, need, sh, b, before);
-            for (uint32_t i = threadIdx.x; i < 2048; i += 256) h[i] = 0;  // ready for the next pass
-            if (threadIdx.x == 0) {
-                st[FB_NEED] = need - before;
-                if (pass == 0) st[FB_PREFIX] = b;
-                else if (pass == 1) st[FB_PREFIX] = (st[FB_PREFIX] << 11) | b;
-                else st[FB_K] = (st[FB_PREFIX] << 10) | b;
-            }
-        } else if (pass == 3) {
-            if (a.cnt[s] > a.cap) {
-                // too many ties for the list: keep those below the id edge that holds `need`
-                uint32_t b, before;
-                fb_find_bin(a.tidh + int64_t(s) * kFbTieBins, kFbTieBins, st[FB_NEED], sh, b, before);
-                if (threadIdx.x == 0) {
-                    const uint64_t edge = uint64_t(b + 1) << a.ishift;
-                    st[FB_EDGE] = edge > 0xFFFFFFFFull ? 0xFFFFFFFFu : uint32_t(edge);
-                    st[FB_OVF] = 1;
-                    a.cnt[s] = 0;
-                }
-            } else if (threadIdx.x == 0) {
-                st[FB_OVF] = 0;
-            }
+    uint32_t* st = a.st + int64_t(s) * 8;
+    uint32_t* h = a.hist + int64_t(s) * 2048;
+    if (pass <= 2) {
+        const uint32_t bins = pass == 2 ? 1024u : 2048u;
+        const uint32_t need = pass == 0 ? a.k : st[FB_NEED];
+        uint32_t b, before;
+        fb_find_bin(h, bins, need, sh, b, before);
+        for (uint32_t i = threadIdx.x; i < 2048; i += 256) h[i] = 0;  // ready for the next pass
+        if (threadIdx.x == 0) {
+            st[FB_NEED] = need - before;
+            if (pass == 0) st[FB_PREFIX] = b;
+            else if (pass == 1) st[FB_PREFIX] = (st[FB_PREFIX] << 11) | b;
+            else st[FB_K] = (st[FB_PREFIX] << 10) | b;
         }
-        __syncthreads();
+    } else if (a.cnt[s] > a.cap) {
+        // too many ties for the list: keep those below the id edge that holds `need`
+        uint32_t b, before;
+        fb_find_bin(a.tidh + int64_t(s) * kFbTieBins, kFbTieBins, st[FB_NEED], sh, b, before);
+        __syncthreads();  // (every thread has read cnt[s])
+        if (threadIdx.x == 0) {
+            const uint64_t edge = uint64_t(b + 1) << a.ishift;
+            st[FB_EDGE] = edge > 0xFFFFFFFFull ? 0xFFFFFFFFu : uint32_t(edge);
+            st[FB_OVF] = 1;
+            a.sync[FBS_TIES] = 1;
+            a.cnt[s] = 0;
+        }
+    } else if (threadIdx.x == 0) {
+        st[FB_OVF] = 0;
     }
+    __syncthreads();
 }
 
 // Adds c to bin b of slot s's histogram, combining runs of one bin within the lane.
@@ -507,65 +525,109 @@ __device__ inline void fb_consume(const FbArgs& a, int pass, FbSlot& sl, uint32_
         }
     }
 }
-// End of a pass kernel (every thread of every workgroup): the last workgroup to finish (a
-// completion ticket, nobody waits) resolves the pass.
-__device__ inline void fb_pass_done(const FbArgs& a, int pass, uint32_t n) {
-    __shared__ uint32_t s_last;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        __threadfence();
-        s_last = atomicAdd(a.done + pass, 1u) == gridDim.x - 1 ? 1u : 0u;
+// The phases of a fallback kernel: pass(p, share) runs the workgroup's share of pass p (work items
+// share, share + gridDim.x, ... of the launch; no barrier inside).
+template <class Pass>
+__device__ inline void fb_phases(const FbArgs& a, const SelectArgs& sel, uint32_t n, Pass&& pass) {
+    __shared__ uint32_t s_word;
+    const uint32_t G = gridDim.x;
+    for (;;) {
+        if (threadIdx.x == 0) s_word = atomicAdd(a.sync + FBS_TICKET, 1u);
+        __syncthreads();
+        const uint32_t phase = s_word / G, share = s_word % G;
+        if (phase >= kFbPhases) return;
+        if (phase > 0) {
+            if (threadIdx.x == 0) {
+                while (!__hip_atomic_load(a.sync + FBS_READY + phase - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                    __builtin_amdgcn_s_sleep(1);
+                __threadfence();  // what the phase before wrote is visible to the workgroup
+            }
+            __syncthreads();
+        }
+        if (phase == kFbPhases - 1) {
+            for (uint32_t s = share; s < n; s += G) {
+                select_row<false, false>(sel, s, nullptr);
+                __syncthreads();
+            }
+            continue;
+        }
+        const int p = int(phase - 1) / 2;  // of phases past the clear
+        uint32_t* done;                    // shares of the phase done
+        if (phase == 0) {
+            const uint64_t step = uint64_t(G) * 256, i0 = uint64_t(share) * 256 + threadIdx.x;
+            for (uint64_t i = i0; i < uint64_t(n) * kFbKeyBins; i += step) a.hist[i] = 0;
+            for (uint64_t i = i0; i < uint64_t(n) * kFbTieBins; i += step) a.tidh[i] = 0;
+            for (uint64_t i = i0; i < uint64_t(n) * 8; i += step) a.st[i] = 0;
+            for (uint64_t i = i0; i < n; i += step) a.cnt[i] = 0;
+            if (i0 < 8) a.done[i0] = 0;
+            done = a.sync + FBS_CLEARED;
+        } else if (phase & 1) {
+            if (p < 4 || a.sync[FBS_TIES]) pass(p, share);
+            done = a.done + p;
+        } else {
+            for (uint32_t s = share; s < n; s += G) fb_resolve(a, p, s);
+            done = a.sync + FBS_RESOLVED + p;
+        }
+        // the last workgroup to finish the phase publishes it (nobody waits here)
+        wait_vmcnt<0>();  // every wave's stores and atomics have reached L2 before thread 0's release
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            __threadfence();
+            if (atomicAdd(done, 1u) == G - 1)
+                __hip_atomic_store(a.sync + FBS_READY + phase, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
-    __syncthreads();
-    if (!s_last) return;
-    __threadfence();
-    fb_resolve(a, pass, n);
 }
 
 template <class P>
-__global__ __launch_bounds__(256) void fb_pass_kernel(P p, FbArgs a, int pass) {
+__global__ __launch_bounds__(256) void fb_kernel(P p, FbArgs a, SelectArgs sel) {
     const uint32_t n = fb_count(a);
     if (n == 0) return;  // nothing overflowed: every workgroup leaves at once
     const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5;
     const uint32_t ngr = (n + 31) / 32, ntl = (a.N + 31) / 32;
     const uint64_t items = uint64_t(ngr) * ntl;
     const uint32_t nw = gridDim.x * 4;
-    for (uint64_t it = blockIdx.x * 4 + (threadIdx.x >> 6); it < items; it += nw) {
-        const uint32_t g = uint32_t(it / ntl), t = uint32_t(it % ntl);
-        const uint32_t s = g * 32 + l32;
-        uint32_t keys[16];
-        p.keys16(a.rows, g * 32, n, t * 32, lane, keys);
-        FbSlot sl;
-        if (s >= n || !fb_slot_begin(a, pass, s, sl)) continue;
+    fb_phases(a, sel, n, [&](int pass, uint32_t share) {
+        for (uint64_t it = uint64_t(share) * 4 + (threadIdx.x >> 6); it < items; it += nw) {
+            const uint32_t g = uint32_t(it / ntl), t = uint32_t(it % ntl);
+            const uint32_t s = g * 32 + l32;
+            uint32_t keys[16];
+            p.keys16(a.rows, g * 32, n, t * 32, lane, keys);
+            FbSlot sl;
+            if (s >= n || !fb_slot_begin(a, pass, s, sl)) continue;
 #pragma unroll 1
-        for (int i = 0; i < 16; ++i) {
-            const uint32_t r = t * 32 + 8 * (i >> 2) + 4 * hh + (i & 3);
-            if (r >= a.N) continue;
-            fb_consume(a, pass, sl, (a.skip && a.skip[r]) ? kAbsentKey : keys[i], r);
+            for (int i = 0; i < 16; ++i) {
+                const uint32_t r = t * 32 + 8 * (i >> 2) + 4 * hh + (i & 3);
+                if (r >= a.N) continue;
+                fb_consume(a, pass, sl, (a.skip && a.skip[r]) ? kAbsentKey : keys[i], r);
+            }
+            sl.run.flush();
         }
-        sl.run.flush();
-    }
-    fb_pass_done(a, pass, n);
+    });
 }
 
-__global__ __launch_bounds__(256) void fb_init_kernel(FbArgs a);
-
 template <class P>
-va_status fb_launch_pass(va_context* ctx, const P& p, const FbArgs& a, int pass) {
-    fb_pass_kernel<P><<<dim3(a.grid), dim3(256), 0, ctx->stream>>>(p, a, pass);
+va_status fb_launch(va_context* ctx, const P& p, const FbArgs& a, const SelectArgs& sel) {
+    fb_kernel<P><<<dim3(a.grid), dim3(256), 0, ctx->stream>>>(p, a, sel);
     VA_CHECK_LAUNCH(ctx);
     return VA_OK;
 }
 
-// Enqueues the whole fallback (clear, five passes, selection) for the producer's keys; base
-// carries the outputs and the key kind of the scan's selection.
-va_status fb_run(va_context* ctx, KeyProducer& kp, const FbArgs& a, const SelectArgs& base);
-// fb_run without the selection: the clear and the passes, which write only a's buffers (a caller
-// may run them on another stream and select after joining it).
-va_status fb_passes(va_context* ctx, KeyProducer& kp, const FbArgs& a);
-// The clear before the first pass and the selection after the last, for callers with their own
-// pass kernels (the IVF list scan).
-va_status fb_init(va_context* ctx, const FbArgs& a);
-va_status fb_select(va_context* ctx, const FbArgs& a, const SelectArgs& base, uint32_t key_bits);
+// The selection of the fallback's lists: base carries the outputs and the key kind of the scan's
+// own selection.
+inline SelectArgs fb_select_args(const FbArgs& a, const SelectArgs& base, uint32_t key_bits) {
+    SelectArgs s = base;
+    s.keys = a.lkey;
+    s.ids = a.lid;
+    s.counts = a.cnt;
+    s.ld = a.cap;
+    s.n = a.cap;
+    s.rows = a.rmax;
+    s.row_map = a.rows;
+    s.overflow_count = nullptr;
+    s.overflow_rows = nullptr;
+    s.key_bits = key_bits;
+    return s;
+}
 
 }  // namespace va

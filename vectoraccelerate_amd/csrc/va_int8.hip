@@ -1286,8 +1286,8 @@ struct I8Producer final : KeyProducer {
     const int8_t* q;
     const int8_t* x;
     uint32_t Q, N, D;
-    va_status fallback_pass(const FbArgs& a, int pass) override {
-        return fb_launch_pass(ctx, FbI8{q, int64_t(D), x, int64_t(D), N, D}, a, pass);
+    va_status fallback(const FbArgs& a, const SelectArgs& sel) override {
+        return fb_launch(ctx, FbI8{q, int64_t(D), x, int64_t(D), N, D}, a, sel);
     }
     va_status dense(const uint32_t* qrow, uint32_t q0, uint32_t nq, uint32_t c0, uint32_t cols, uint32_t stride,
                     uint32_t* out_k, int64_t ldo) override {

@@ -84,36 +84,6 @@ va_status aux_fork(va_context* ctx, int n = va_context::kAux);
 // Makes ctx->stream wait for the work queued so far on ctx->aux[0 .. n).
 va_status aux_join(va_context* ctx, int n = va_context::kAux);
 
-// Joins ctx->aux[0 .. n) into ctx->stream when it leaves scope unless join() ran first, so an
-// error return between a fork and its join still orders the aux work before anything the caller
-// queues next (scratch buffers the aux work writes are reused by later calls).
-struct AuxJoinGuard {
-    va_context* ctx;
-    int n;
-    bool armed = true;
-    AuxJoinGuard(va_context* c, int k) : ctx(c), n(k) {}
-    va_status join() {
-        armed = false;
-        return aux_join(ctx, n);
-    }
-    ~AuxJoinGuard() {
-        if (armed) (void)aux_join(ctx, n);
-    }
-    AuxJoinGuard(const AuxJoinGuard&) = delete;
-    AuxJoinGuard& operator=(const AuxJoinGuard&) = delete;
-};
-
-// Sends what the code in the scope queues on ctx->stream to another stream (an aux stream, forked
-// from ctx->stream before the scope and joined after it).
-struct StreamScope {
-    va_context* ctx;
-    hipStream_t prev;
-    StreamScope(va_context* c, hipStream_t s) : ctx(c), prev(c->stream) { c->stream = s; }
-    ~StreamScope() { ctx->stream = prev; }
-    StreamScope(const StreamScope&) = delete;
-    StreamScope& operator=(const StreamScope&) = delete;
-};
-
 // Makes `ctx->device` current for the lifetime of the guard.
 struct DeviceGuard {
     int prev = -1;
@@ -495,8 +465,6 @@ struct SelectArgs {
     uint32_t k = 0;
     uint32_t id_offset = 0;        // added to output ids
     const uint32_t* row_map = nullptr;  // output row for each input row (nullptr: identity)
-    // device row count (rows past it are skipped; rows is then the host bound), or nullptr
-    const uint32_t* rows_dev = nullptr;
     // outputs (row stride out_ld, default k)
     int64_t out_ld = 0;
     uint32_t* out_idx = nullptr;   // [rows x k]
@@ -514,7 +482,15 @@ struct SelectArgs {
     // every key is below 2^key_bits (Hamming distances: a few bits); up to 11 bits the k-th
     // smallest key comes from one histogram pass instead of four byte passes
     uint32_t key_bits = 32;
+    // cleared on the side, so that the scan behind a threshold selection needs no fill launch:
+    // zero_cnt[row] and the kZeroWords words at zero_words (by row 0)
+    uint32_t* zero_cnt = nullptr;
+    uint32_t* zero_words = nullptr;
 };
+// Overflow words of a scan (one carve): [0] queries listed for the fallback, [1] longest rerank
+// list, [kFbSync ..) the fallback's phase words (va_fallback.hpp).  Cleared before the scan.
+constexpr uint32_t kZeroWords = 64;
+constexpr uint32_t kFbSync = 8;
 va_status launch_select(va_context* ctx, const SelectArgs& a);
 
 // assign[i] = the nearest centroid of row i by L2^2 (ties -> lower centroid) on the fp32 MFMA
@@ -549,8 +525,9 @@ struct KeyProducer {
     virtual va_status filter(const uint32_t* thr, uint32_t* cnt, uint32_t* ckey, uint32_t* cid, uint32_t cap) = 0;
     // every key the producer makes is below 2^key_bits()
     virtual uint32_t key_bits() const { return 32; }
-    // one pass of the device-side overflow fallback (fb_pass_kernel over the producer's keys)
-    virtual va_status fallback_pass(const FbArgs& a, int pass) = 0;
+    // the device-side overflow fallback over the producer's keys (fb_kernel); sel carries the
+    // outputs of its selection (fb_select_args)
+    virtual va_status fallback(const FbArgs& a, const SelectArgs& sel) = 0;
     virtual ~KeyProducer() = default;
 };
 

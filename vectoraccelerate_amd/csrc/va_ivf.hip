@@ -149,8 +149,8 @@ struct F32Keys final : KeyProducer {
     const float* q;
     const float* x;
     uint32_t Q, N, D;
-    va_status fallback_pass(const FbArgs& a, int pass) override {
-        return fb_launch_pass(ctx, FbF32{q, int64_t(D), x, int64_t(D), N, D, int(OP_L2SQ)}, a, pass);
+    va_status fallback(const FbArgs& a, const SelectArgs& sel) override {
+        return fb_launch(ctx, FbF32{q, int64_t(D), x, int64_t(D), N, D, int(OP_L2SQ)}, a, sel);
     }
     va_status dense(const uint32_t* qrow, uint32_t q0, uint32_t nq, uint32_t c0, uint32_t cols, uint32_t stride,
                     uint32_t* out_k, int64_t ldo) override {
@@ -1729,60 +1729,61 @@ struct FbIvf {
 // keys with the arithmetic of the kernel that scanned the list in the full pass, then the
 // fallback pass's action for each.
 template <bool VEC>
-__global__ __launch_bounds__(256) void fb_ivf_pass_kernel(FbIvf v, FbArgs a, int pass) {
+__global__ __launch_bounds__(256) void fb_ivf_kernel(FbIvf v, FbArgs a, SelectArgs sel) {
     const uint32_t n = fb_count(a);
     if (n == 0) return;  // nothing overflowed: every workgroup leaves at once
     const int lane = threadIdx.x & 63;
     const uint64_t items = uint64_t(n) * v.np * v.tmax;
     const uint32_t nw = gridDim.x * 4;
-    for (uint64_t it = blockIdx.x * 4 + (threadIdx.x >> 6); it < items; it += nw) {
-        const uint32_t t = uint32_t(it % v.tmax);
-        const uint64_t sp = it / v.tmax;
-        const uint32_t p = uint32_t(sp % v.np), s = uint32_t(sp / v.np);
-        const uint32_t qi = a.rows[s];
-        const uint32_t l = v.P[int64_t(qi) * v.np + p];
-        if (l == 0xFFFFFFFFu) continue;
-        const uint32_t len = v.roff[l + 1] - v.roff[l];
-        if (t * 32 >= len) continue;  // (uniform)
-        FbSlot sl;
-        if (!fb_slot_begin(a, pass, s, sl)) continue;
-        const uint32_t base = v.roff[l] + t * 32, rc = min(32u, len - t * 32);
-        const float* qrow = v.q + int64_t(qi) * v.D;
-        if (v.small_ok && v.qcnt[l] <= kSmallListQueries) {
-            const int j = lane & 15, g = lane >> 4;
-            uint32_t keys[8];
-            small_keys32(j == 0 ? qrow : nullptr, uint32_t(j) < rc ? v.x + int64_t(base + j) * v.D : nullptr,
-                         uint32_t(16 + j) < rc ? v.x + int64_t(base + 16 + j) * v.D : nullptr, v.D, lane, keys);
-            if (j == 0) {
+    fb_phases(a, sel, n, [&](int pass, uint32_t share) {
+        for (uint64_t it = uint64_t(share) * 4 + (threadIdx.x >> 6); it < items; it += nw) {
+            const uint32_t t = uint32_t(it % v.tmax);
+            const uint64_t sp = it / v.tmax;
+            const uint32_t p = uint32_t(sp % v.np), s = uint32_t(sp / v.np);
+            const uint32_t qi = a.rows[s];
+            const uint32_t l = v.P[int64_t(qi) * v.np + p];
+            if (l == 0xFFFFFFFFu) continue;
+            const uint32_t len = v.roff[l + 1] - v.roff[l];
+            if (t * 32 >= len) continue;  // (uniform)
+            FbSlot sl;
+            if (!fb_slot_begin(a, pass, s, sl)) continue;
+            const uint32_t base = v.roff[l] + t * 32, rc = min(32u, len - t * 32);
+            const float* qrow = v.q + int64_t(qi) * v.D;
+            if (v.small_ok && v.qcnt[l] <= kSmallListQueries) {
+                const int j = lane & 15, g = lane >> 4;
+                uint32_t keys[8];
+                small_keys32(j == 0 ? qrow : nullptr, uint32_t(j) < rc ? v.x + int64_t(base + j) * v.D : nullptr,
+                             uint32_t(16 + j) < rc ? v.x + int64_t(base + 16 + j) * v.D : nullptr, v.D, lane, keys);
+                if (j == 0) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const uint32_t m = uint32_t(16 * (i >> 2) + 4 * g + (i & 3));
-                    if (m < rc) {
-                        const uint32_t id = v.ids[base + m];
-                        fb_consume(a, pass, sl, (a.skip && a.skip[id]) ? kAbsentKey : keys[i], id);
+                    for (int i = 0; i < 8; ++i) {
+                        const uint32_t m = uint32_t(16 * (i >> 2) + 4 * g + (i & 3));
+                        if (m < rc) {
+                            const uint32_t id = v.ids[base + m];
+                            fb_consume(a, pass, sl, (a.skip && a.skip[id]) ? kAbsentKey : keys[i], id);
+                        }
+                    }
+                }
+            } else {
+                const int l32 = lane & 31, hh = lane >> 5;
+                uint32_t keys[16];
+                f32_block_keys<VEC>(l32 == 0 ? qrow : nullptr,
+                                    uint32_t(l32) < rc ? v.x + int64_t(base + l32) * v.D : nullptr, v.D, int(OP_L2SQ),
+                                    lane, keys);
+                if (l32 == 0) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        const uint32_t m = uint32_t(8 * (i >> 2) + 4 * hh + (i & 3));
+                        if (m < rc) {
+                            const uint32_t id = v.ids[base + m];
+                            fb_consume(a, pass, sl, (a.skip && a.skip[id]) ? kAbsentKey : keys[i], id);
+                        }
                     }
                 }
             }
-        } else {
-            const int l32 = lane & 31, hh = lane >> 5;
-            uint32_t keys[16];
-            f32_block_keys<VEC>(l32 == 0 ? qrow : nullptr,
-                                uint32_t(l32) < rc ? v.x + int64_t(base + l32) * v.D : nullptr, v.D, int(OP_L2SQ),
-                                lane, keys);
-            if (l32 == 0) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const uint32_t m = uint32_t(8 * (i >> 2) + 4 * hh + (i & 3));
-                    if (m < rc) {
-                        const uint32_t id = v.ids[base + m];
-                        fb_consume(a, pass, sl, (a.skip && a.skip[id]) ? kAbsentKey : keys[i], id);
-                    }
-                }
-            }
+            sl.run.flush();
         }
-        sl.run.flush();
-    }
-    fb_pass_done(a, pass, n);
+    });
 }
 
 // ---- exact keys of the screened scan's rerank lists ------------------------------------------
@@ -1847,12 +1848,9 @@ __global__ __launch_bounds__(256) void ivf_rerank_kernel(const float* __restrict
 }
 
 // Exact top-k, on the device, of the queries listed in fb (their candidates outgrew a list):
-// their probed lists walked with the arithmetic of the kernel that scans each list.  The passes
-// read only the queries, the lists, the plan and fb's list of queries, and write only fb's
-// buffers; the selection writes the listed queries' results.
-va_status ivf_fallback_passes(va_context* ctx, const va_ivf* ivf, const float* queries, const DevPlan& dp, uint32_t np,
-                              const FbArgs& fb) {
-    VA_CHECK_STATUS(fb_init(ctx, fb));
+// their probed lists walked with the arithmetic of the kernel that scans each list.
+va_status ivf_fallback(va_context* ctx, const va_ivf* ivf, const float* queries, const DevPlan& dp, uint32_t np,
+                       const FbArgs& fb, const SelectArgs& base) {
     FbIvf v;
     v.q = queries;
     v.x = ivf->list_vectors;
@@ -1866,19 +1864,13 @@ va_status ivf_fallback_passes(va_context* ctx, const va_ivf* ivf, const float* q
     v.small_ok = dp.small_ok;
     const bool vec = ivf->D % 4 == 0 && (reinterpret_cast<uintptr_t>(queries) & 15) == 0 &&
                      (reinterpret_cast<uintptr_t>(ivf->list_vectors) & 15) == 0;
-    for (int pass = 0; pass < kFbPasses; ++pass) {
-        if (vec)
-            fb_ivf_pass_kernel<true><<<dim3(fb.grid), dim3(256), 0, ctx->stream>>>(v, fb, pass);
-        else
-            fb_ivf_pass_kernel<false><<<dim3(fb.grid), dim3(256), 0, ctx->stream>>>(v, fb, pass);
-        VA_CHECK_LAUNCH(ctx);
-    }
+    const SelectArgs sel = fb_select_args(fb, base, 32);
+    if (vec)
+        fb_ivf_kernel<true><<<dim3(fb.grid), dim3(256), 0, ctx->stream>>>(v, fb, sel);
+    else
+        fb_ivf_kernel<false><<<dim3(fb.grid), dim3(256), 0, ctx->stream>>>(v, fb, sel);
+    VA_CHECK_LAUNCH(ctx);
     return VA_OK;
-}
-va_status ivf_fallback(va_context* ctx, const va_ivf* ivf, const float* queries, const DevPlan& dp, uint32_t np,
-                       const FbArgs& fb, const SelectArgs& base) {
-    VA_CHECK_STATUS(ivf_fallback_passes(ctx, ivf, queries, dp, np, fb));
-    return fb_select(ctx, fb, base, 32);
 }
 
 // A list takes 16-query tiles when few queries probe it (decided once per search from the
@@ -1962,7 +1954,7 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     uint32_t* ubound = s.carve<uint32_t>(Q);
     uint32_t* rcount = s.carve<uint32_t>(Q);
     uint32_t* ovf_rows = s.carve<uint32_t>(Q);
-    uint32_t* ovf_cnt = s.carve<uint32_t>(64);
+    uint32_t* ovf_cnt = s.carve<uint32_t>(va::kZeroWords);
     float4* qinfo = s.carve<float4>(Q);
     float* qerr = s.carve<float>(Q);
     _Float16* qh = s.carve<_Float16>(uint64_t(Q) * Dp);
@@ -1999,6 +1991,7 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     FbArgs fb = fb_carve(s, Q, id_span, k, ivf->N);
     fb.n_rows = ovf_cnt;
     fb.rows = ovf_rows;
+    fb.sync = ovf_cnt + va::kFbSync;
     fb.skip = skip;
     float4* gpt = dp.big_tq ? s.carve<float4>(pairs) : nullptr;
     float2* gqv = dp.big_tq ? s.carve<float2>(pairs) : nullptr;
@@ -2018,7 +2011,7 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     VA_CHECK_STATUS(pm.mark(0));
     // ---- 0. plan and queries --------------------------------------------------------------------
     VA_CHECK_STATUS(plan_on_device(ctx, dp));
-    VA_CHECK_STATUS(screen_prepare_queries(ctx, queries, Q, D, qh, qinfo, bnd.c0, qerr, cnt2, 2 * Q, ovf_cnt, 2));
+    VA_CHECK_STATUS(screen_prepare_queries(ctx, queries, Q, D, qh, qinfo, bnd.c0, qerr, cnt2, 2 * Q, ovf_cnt, kZeroWords));
     Ivf16Args a;
     a.qh = qh;
     a.nq = Q;
@@ -2083,15 +2076,6 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     // ---- 4. rerank lists, 5. exact keys ----------------------------------------------------------
     VA_CHECK_STATUS(screen_compact(ctx, cnt, clo, cpos, ubound, uint32_t(cap), Q, rr, rcount, uint32_t(rcap), ovf_cnt,
                                    ovf_rows));
-    // ---- 7a. the overflowed queries (listed by the U_q selection and the compaction) take the
-    // device fallback's passes on an aux stream, beside the rerank and the selection (a search
-    // with none still pays their launches, off the critical path here)
-    VA_CHECK_STATUS(aux_fork(ctx, 1));
-    AuxJoinGuard fb_join(ctx, 1);
-    {
-        StreamScope on_aux(ctx, ctx->aux[0]);
-        VA_CHECK_STATUS(ivf_fallback_passes(ctx, ivf, queries, dp, np, fb));
-    }
     {
         const uint64_t items = uint64_t(Q) * ((rcap + 63) / 64);
         const uint32_t blocks = uint32_t(std::min<uint64_t>(2048, (items + 3) / 4));
@@ -2122,9 +2106,9 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     VA_CHECK_STATUS(pm.count_sum(rcount, Q));
     VA_CHECK_STATUS(pm.count_overflow(ovf_cnt));
     VA_CHECK_STATUS(pm.mark(3));
-    // ---- 7b. their exact top-k over the rows the selection wrote
-    VA_CHECK_STATUS(fb_join.join());
-    VA_CHECK_STATUS(fb_select(ctx, fb, base, 32));
+    // ---- 7. exact top-k of the overflowed queries (listed by the U_q selection and the
+    // compaction), over the rows the selection wrote
+    VA_CHECK_STATUS(ivf_fallback(ctx, ivf, queries, dp, np, fb, base));
     return pm.finish(true, true);
 }
 }  // namespace
@@ -2354,7 +2338,7 @@ va_status ivf_scan_masked(va_context* ctx, const va_ivf* ivf, const float* queri
     uint32_t* thr = s.carve<uint32_t>(Q);
     uint32_t* cnt = s.carve<uint32_t>(Q);
     uint32_t* ovf_rows = s.carve<uint32_t>(Q);
-    uint32_t* ovf_cnt = s.carve<uint32_t>(64);
+    uint32_t* ovf_cnt = s.carve<uint32_t>(va::kZeroWords);
     va::DevPlan dp;
     dp.probes = probes;
     dp.Q = Q;
@@ -2374,6 +2358,7 @@ va_status ivf_scan_masked(va_context* ctx, const va_ivf* ivf, const float* queri
     va::FbArgs fb = va::fb_carve(s, Q, id_span, k, ivf->N);
     fb.n_rows = ovf_cnt;
     fb.rows = ovf_rows;
+    fb.sync = ovf_cnt + va::kFbSync;
     fb.skip = skip;
     VA_CHECK_STATUS(s.verify(need));
 
@@ -2401,7 +2386,7 @@ va_status ivf_scan_masked(va_context* ctx, const va_ivf* ivf, const float* queri
     }
     // ---- 2. full pass with the thresholds, 3. exact selection -----------------------------------
     VA_CHECK_STATUS(va::fill_u32(ctx, cnt, Q, 0));
-    VA_CHECK_STATUS(va::fill_u32(ctx, ovf_cnt, 1, 0));
+    VA_CHECK_STATUS(va::fill_u32(ctx, ovf_cnt, va::kZeroWords, 0));
     VA_CHECK_STATUS(pm.mark(1));
     VA_CHECK_STATUS(va::run_planned_pass(ctx, dp, 1, queries, ivf, thr, cnt, ckey, cid, uint32_t(cap)));
     VA_CHECK_STATUS(pm.mark(2));

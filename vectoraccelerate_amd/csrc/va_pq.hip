@@ -680,8 +680,8 @@ struct AdcProducer final : KeyProducer {
     // fp16 pair tables and scales of the screened filter (nullptr: the fp32 filter)
     const uint32_t* packed = nullptr;
     const float* scale = nullptr;
-    va_status fallback_pass(const FbArgs& a, int pass) override {
-        return fb_launch_pass(ctx, FbAdc{codes, tables, N, M, K}, a, pass);
+    va_status fallback(const FbArgs& a, const SelectArgs& sel) override {
+        return fb_launch(ctx, FbAdc{codes, tables, N, M, K}, a, sel);
     }
     va_status dense(const uint32_t* qrow, uint32_t q0, uint32_t nq, uint32_t c0, uint32_t cols, uint32_t stride,
                     uint32_t* out_k, int64_t ldo) override {

@@ -222,13 +222,14 @@ va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t
     uint32_t* ovf_rows = s.carve<uint32_t>(Q);
     uint32_t* ckey = s.carve<uint32_t>(uint64_t(Q) * cap);
     uint32_t* cid = s.carve<uint32_t>(uint64_t(Q) * cap);
-    uint32_t* ovf_cnt = s.carve<uint32_t>(64);
+    uint32_t* ovf_cnt = s.carve<uint32_t>(kZeroWords);
     uint32_t* skeys = s.carve<uint32_t>(uint64_t(qs) * S);
     FbArgs fb;
     if (device_fb) {
         fb = fb_carve(s, Q, N, k);
         fb.n_rows = ovf_cnt;
         fb.rows = ovf_rows;
+        fb.sync = ovf_cnt + kFbSync;
         fb.skip = out.skip;
     }
     VA_CHECK_STATUS(s.verify(need));
@@ -246,11 +247,11 @@ va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t
         a.k = rank;
         a.out_kth = thr + q0;
         a.key_bits = kp.key_bits();
+        a.zero_cnt = cnt + q0;  // the filter's list lengths and overflow words
+        a.zero_words = ovf_cnt;
         VA_CHECK_STATUS(launch_select(ctx, a));
     }
     // ---- 2. filter --------------------------------------------------------------------
-    VA_CHECK_STATUS(fill_u32(ctx, cnt, Q, 0));
-    VA_CHECK_STATUS(fill_u32(ctx, ovf_cnt, 1, 0));
     VA_CHECK_STATUS(pm.mark(1));
     VA_CHECK_STATUS(kp.filter(thr, cnt, ckey, cid, uint32_t(cap)));
     VA_CHECK_STATUS(pm.mark(2));
@@ -276,7 +277,7 @@ va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t
     VA_CHECK_STATUS(pm.mark(3));
     if (device_fb) {
         // ---- 4. exact top-k of the overflowed rows, on the device ------------------------------
-        VA_CHECK_STATUS(fb_run(ctx, kp, fb, base));
+        VA_CHECK_STATUS(kp.fallback(fb, fb_select_args(fb, base, kp.key_bits())));
         return pm.finish(true, true);
     }
     VA_CHECK_HIP(ctx, hipMemcpyAsync(ctx->host_word, ovf_cnt, 4, hipMemcpyDeviceToHost, ctx->stream));

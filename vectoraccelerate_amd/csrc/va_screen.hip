@@ -1697,7 +1697,7 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
     uint32_t* ubound = s.carve<uint32_t>(Q);
     uint32_t* rcount = s.carve<uint32_t>(Q);
     uint32_t* ovf_rows = s.carve<uint32_t>(Q);
-    uint32_t* ovf_cnt = s.carve<uint32_t>(64);
+    uint32_t* ovf_cnt = s.carve<uint32_t>(kZeroWords);
     float4* qinfo = s.carve<float4>(Q);
     float4* ptc = s.carve<float4>(Q);
     float* qerr = s.carve<float>(Q);
@@ -1714,17 +1714,17 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
         fb = fb_carve(s, Q, N, k);
         fb.n_rows = ovf_cnt;
         fb.rows = ovf_rows;
+        fb.sync = ovf_cnt + kFbSync;
         fb.skip = out.skip;
     }
     VA_CHECK_STATUS(s.verify(need));
 
     // ---- 1. queries -> scaled fp16 ---------------------------------------------------------
-    // (also clears the scan's list counters and the overflow words: [0] overflowed queries, [1]
-    // longest rerank list)
+    // (also clears the scan's list counters and the overflow words)
     const bool measured = in.xh && in.xe;  // the candidates' intervals from measured rounding errors
     screen_prep_kernel<<<dim3((Q + 3) / 4), dim3(256), 0, ctx->stream>>>(in.q, int64_t(D), Q, D, Dp, qh, qinfo,
                                                                        bnd.c0, measured ? qerr : nullptr, 1, cnt, Q,
-                                                                       ovf_cnt, 2u);
+                                                                       ovf_cnt, kZeroWords);
     VA_CHECK_LAUNCH(ctx);
 
     ScreenArgs sa;
@@ -1865,15 +1865,6 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
                                                                  rcount, uint32_t(rcap), ovf_cnt, ovf_rows,
                                                                  ovf_cnt + 1);
     VA_CHECK_LAUNCH(ctx);
-    AuxJoinGuard fb_join(ctx, device_fb ? 1 : 0);
-    if (device_fb) {
-        // ---- 8a. the overflowed queries (listed by steps 4 and 5) take the device fallback's
-        // passes on an aux stream, beside the rerank and the selection (a search with none still
-        // pays their launches, off the critical path here)
-        VA_CHECK_STATUS(aux_fork(ctx, 1));
-        StreamScope on_aux(ctx, ctx->aux[0]);
-        VA_CHECK_STATUS(fb_passes(ctx, exact, fb));
-    }
     // Without the device fallback the overflow count is read back (one synchronisation).
     uint32_t n_ovf = 0;
     if (!device_fb) {
@@ -1915,9 +1906,9 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
     if (device_fb) VA_CHECK_STATUS(pm.count_overflow(ovf_cnt));
     VA_CHECK_STATUS(pm.mark(3));
     if (device_fb) {
-        // ---- 8b. their exact top-k, over the rows step 7 wrote ----------------------------------
-        VA_CHECK_STATUS(fb_join.join());
-        VA_CHECK_STATUS(fb_select(ctx, fb, base, exact.key_bits()));
+        // ---- 8. exact top-k of the overflowed queries (listed by steps 4 and 5), over the rows
+        // step 7 wrote
+        VA_CHECK_STATUS(exact.fallback(fb, fb_select_args(fb, base, exact.key_bits())));
         return pm.finish(true, true);
     }
     ctx->last_scan.overflow_rows = n_ovf;
