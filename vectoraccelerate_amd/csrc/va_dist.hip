@@ -482,6 +482,180 @@ va_status launch_shape(va_context* ctx, const DistArgs& a, bool vec) {
     return vec ? launch_tile<WQ, WN, true, OUT, false>(ctx, a) : launch_tile<WQ, WN, false, OUT, false>(ctx, a);
 }
 
+// ---------------------------------------------------------------------------------------
+// Few queries: rows streamed into registers
+// ---------------------------------------------------------------------------------------
+// A batch of at most 32 queries is bound by reading the rows, and a launch of few tiles by the
+// latency of each tile's chain of stages (one stage ahead: 1.4 us per 16 values of a row, 104 us for
+// 20,000 x 768).  Here every wave is an independent worker without LDS or barriers: a tile of 32
+// rows x 32 queries, both operands loaded straight into registers in chunks of 32 values (whole
+// 128-byte lines per row), a ring of R chunks with R - 1 in flight.  (Two query blocks per wave
+// spilled; the blocks of a batch past 32 are neighbouring tiles instead, which share the rows
+// through L2.)  The values of a key are formed
+// in dist_tile's order (32x32x2 MFMA steps over d = 8g + e and 8g + 4 + e, exactly ceil(D / 16)
+// stages of 16, the norms as two half chains), so the keys are the same bits.  The distance is a
+// template parameter: sixteen copies of its switch would be most of the kernel's code.
+// Measured against one-wave GEMM tiles, whole searches, top-10: 20,000 x 768, Q = 1 104 -> 38 us;
+// 200,000 x 768, Q = 8 189 -> 186; 500,000 x 768, Q = 1 390 -> 353 (1.5 GB: 4.4 TB/s).
+// TAIL: D % 4 != 0 (a lane's four values may run into the next row: cleared past D).
+template <int R, bool TAIL, int OUT, int OP>
+__global__ __launch_bounds__(256, 2) void dist_stream_kernel(DistArgs a) {
+    const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t D = a.D, nch = (D + 31) / 32, nqb = (a.Q + 31) / 32;
+    const uint32_t ntiles = (a.N + 31) / 32 * nqb;
+    struct Slot {
+        f32x4v x[4], q[4];
+    };
+    for (uint32_t tile = blockIdx.x * 4 + wave; tile < ntiles; tile += gridDim.x * 4) {
+        const uint32_t rt = nqb == 1 ? tile : tile / nqb;
+        const uint32_t q0 = (tile - rt * nqb) * 32, qn = min(32u, a.Q - q0);
+        const __amdgpu_buffer_rsrc_t qres =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.q + int64_t(q0) * a.ldq), 0,
+                                              int((uint64_t(qn - 1) * uint64_t(a.ldq) + D) * 4u), 0x00020000);
+        const uint32_t qoff = uint32_t(l32) < qn ? uint32_t(l32 * uint64_t(a.ldq) * 4) : kDmaSkip;
+        const uint32_t rs = rt * 32, rc = min(32u, a.N - rs);
+        const __amdgpu_buffer_rsrc_t xres =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.x + int64_t(rs) * a.ldx), 0,
+                                              int((uint64_t(rc - 1) * uint64_t(a.ldx) + D) * 4u), 0x00020000);
+        const uint32_t xoff = uint32_t(l32) < rc ? uint32_t(l32 * uint64_t(a.ldx) * 4) : kDmaSkip;
+        Slot ring[R];
+        auto load = [&](uint32_t c, Slot& s) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const uint32_t d = 32 * c + 8 * g + 4 * hh;
+                const bool in = d < D;
+                auto one = [&](const __amdgpu_buffer_rsrc_t& r, uint32_t off) {
+                    f32x4v v = __builtin_bit_cast(
+                        f32x4v, __builtin_amdgcn_raw_buffer_load_b128(r, in && off != kDmaSkip ? off + 4 * d : kDmaSkip, 0, 0));
+                    return v;
+                };
+                s.x[g] = one(xres, xoff);
+                s.q[g] = one(qres, qoff);
+            }
+        };
+        f32x16 acc;
+        float qss = 0.0f, xss = 0.0f;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+        auto stage = [&](Slot& s, uint32_t c, int h, bool last) {
+#pragma unroll
+            for (int g = 2 * h; g < 2 * h + 2; ++g) {
+                if (TAIL && last) {
+                    const uint32_t d = 32 * c + 8 * g + 4 * hh;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (d + e >= D) {
+                            s.x[g][e] = 0.0f;
+                            s.q[g][e] = 0.0f;
+                        }
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) xss = fmaf(s.x[g][e], s.x[g][e], xss);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) qss = fmaf(s.q[g][e], s.q[g][e], qss);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(s.x[g][e], s.q[g][e], acc, 0, 0, 0);
+            }
+        };
+#pragma unroll
+        for (int r = 0; r < R - 1; ++r) load(uint32_t(r), ring[r]);
+        const uint32_t nfull = (nch - 1) / R * R;  // chunks of the rolled loop: none is the last
+        for (uint32_t c = 0; c < nfull; c += R) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                load(c + uint32_t(r + R - 1), ring[(r + R - 1) % R]);  // (past the end: zeros, unused)
+                stage(ring[r], c + r, 0, false);
+                stage(ring[r], c + r, 1, false);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (nfull + R - 1 < nch) load(nfull + R - 1, ring[R - 1]);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const uint32_t c = nfull + r;
+            if (c < nch) {
+                stage(ring[r], c, 0, true);
+                if (32 * c + 16 < D) stage(ring[r], c, 1, true);
+            }
+        }
+        // lane (l32, hh): query q0 + l32 against rows 8j + 4hh + e in acc[4j + e]
+        const float xt = xss + __shfl_xor(xss, 32);
+        const float qq = qss + __shfl_xor(qss, 32);
+        const uint32_t qi = q0 + uint32_t(l32);
+        uint32_t key[16];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                key[4 * j + e] = key_of_float(apply_op(OP, acc[4 * j + e], qq, __shfl(xt, 8 * j + 4 * hh + e)));
+        if (uint32_t(l32) >= qn) continue;
+        if (OUT == OUT_KEYS) {
+            uint32_t* o = a.out_k + int64_t(qi) * a.ldo + rs;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t r = 8 * j + 4 * hh + e;
+                    if (r < rc) o[r] = key[4 * j + e];
+                }
+        } else {
+            const uint32_t thr = a.thr[qi];
+            uint32_t pass = 0;
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                pass |= uint32_t((8u * (v >> 2) + 4u * hh + (v & 3) < rc) & (key[v] <= thr)) << v;
+            if (!pass) continue;
+            uint32_t pos = atomicAdd(a.cnt + qi, uint32_t(__popc(pass)));
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                if (!((pass >> v) & 1)) continue;
+                if (pos < a.cap) {
+                    const int64_t o = int64_t(qi) * a.cap + pos;
+                    a.cand_key[o] = key[v];
+                    a.cand_id[o] = a.id_base + rs + 8 * (v >> 2) + 4 * hh + (v & 3);
+                }
+                ++pos;
+            }
+        }
+    }
+}
+
+// The launches dist_stream_kernel takes: keys or a filter over dense query rows, at most 32 queries
+// or so few GEMM tiles that the chip would be mostly idle (past that the GEMM's tiles read the rows
+// once for up to 128 queries: 500,000 x 768, Q = 40 595 us on them, 810 streamed), every offset
+// within a tile below 2^31.
+bool stream_ok(const va_context* ctx, const DistArgs& a, int wq, int wn) {
+    if (a.wq || a.wn || a.plan.pre || a.gather || a.qrow || a.ids || (a.out != OUT_KEYS && a.out != OUT_FILTER)) return false;
+    if (a.op != OP_L2SQ && a.op != OP_L2 && a.op != OP_COS_DIST && a.op != OP_NEG_DOT) return false;
+    if (uint64_t(ceil_div(a.N, 32)) * ceil_div(a.Q, 32) >= (1ull << 31)) return false;
+    if (uint64_t(31) * uint64_t(a.ldq) * 4 + uint64_t(a.D) * 4 > kDmaMaxBytes ||
+        uint64_t(31) * uint64_t(a.ldx) * 4 + uint64_t(a.D) * 4 > kDmaMaxBytes)
+        return false;
+    return a.Q <= 32 || uint64_t(ceil_div(a.Q, 32 * wq)) * ceil_div(a.N, 128 * wn) < 2ull * uint64_t(ctx->num_cus);
+}
+
+template <int OUT, int OP>
+void launch_stream_op(va_context* ctx, const DistArgs& a) {
+    const uint32_t tiles = ceil_div(a.N, 32) * ceil_div(a.Q, 32);
+    const uint32_t grid = std::min((tiles + 3) / 4, 8 * uint32_t(ctx->num_cus));
+    if (a.D % 4)
+        dist_stream_kernel<4, true, OUT, OP><<<dim3(grid), dim3(256), 0, ctx->stream>>>(a);
+    else
+        dist_stream_kernel<4, false, OUT, OP><<<dim3(grid), dim3(256), 0, ctx->stream>>>(a);
+}
+template <int OUT>
+va_status launch_stream(va_context* ctx, const DistArgs& a) {
+    switch (a.op) {
+        case OP_L2SQ: launch_stream_op<OUT, OP_L2SQ>(ctx, a); break;
+        case OP_L2: launch_stream_op<OUT, OP_L2>(ctx, a); break;
+        case OP_COS_DIST: launch_stream_op<OUT, OP_COS_DIST>(ctx, a); break;
+        default: launch_stream_op<OUT, OP_NEG_DOT>(ctx, a);
+    }
+    VA_CHECK_LAUNCH(ctx);
+    return VA_OK;
+}
+
 }  // namespace
 
 va_status launch_dist(va_context* ctx, const DistArgs& a) {
@@ -496,6 +670,8 @@ va_status launch_dist(va_context* ctx, const DistArgs& a) {
     }
     const int wq = a.wq ? a.wq : (a.Q <= 32 ? 1 : (a.Q <= 64 ? 2 : 4));
     const int wn = a.wn ? a.wn : 4 / wq;
+    if (stream_ok(ctx, a, wq, wn))
+        return a.out == OUT_KEYS ? launch_stream<OUT_KEYS>(ctx, a) : launch_stream<OUT_FILTER>(ctx, a);
 #define VA_DIST_CASE(W, N, O) \
     if (wq == W && wn == N && a.out == O) return launch_shape<W, N, O>(ctx, a, vec);
     VA_DIST_CASE(1, 4, OUT_VALUES) VA_DIST_CASE(1, 4, OUT_KEYS) VA_DIST_CASE(1, 4, OUT_FILTER)

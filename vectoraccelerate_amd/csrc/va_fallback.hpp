@@ -530,6 +530,7 @@ __device__ inline void fb_consume(const FbArgs& a, int pass, FbSlot& sl, uint32_
 template <class Pass>
 __device__ inline void fb_phases(const FbArgs& a, const SelectArgs& sel, uint32_t n, Pass&& pass) {
     __shared__ uint32_t s_word;
+    __shared__ SelectLds<false> s_sel;
     const uint32_t G = gridDim.x;
     for (;;) {
         if (threadIdx.x == 0) s_word = atomicAdd(a.sync + FBS_TICKET, 1u);
@@ -546,7 +547,7 @@ __device__ inline void fb_phases(const FbArgs& a, const SelectArgs& sel, uint32_
         }
         if (phase == kFbPhases - 1) {
             for (uint32_t s = share; s < n; s += G) {
-                select_row<false, false>(sel, s, nullptr);
+                select_row<256, false, false>(sel, s, s_sel, nullptr);
                 __syncthreads();
             }
             continue;

@@ -74,6 +74,23 @@ va_status mask_list_keys(va_context* ctx, uint32_t* keys, uint32_t* keys2, const
     return VA_OK;
 }
 
+// gmin[r * G + g] = the smallest of the keys r * ld + g + j G, j < kGroupKeys (columns past S
+// absent).  Any partition of the sample into groups will do; this one reads whole lines.
+constexpr uint32_t kGroupKeys = 32;
+__global__ __launch_bounds__(256) void group_min_kernel(const uint32_t* __restrict__ keys, int64_t ld, uint32_t S,
+                                                        uint32_t G, uint32_t* __restrict__ gmin) {
+    const uint32_t g = blockIdx.x * 256 + threadIdx.x;
+    if (g >= G) return;
+    const uint32_t* row = keys + int64_t(blockIdx.y) * ld;
+    uint32_t v[kGroupKeys];
+#pragma unroll
+    for (uint32_t j = 0; j < kGroupKeys; ++j) v[j] = g + j * G < S ? row[g + j * G] : 0xFFFFFFFFu;
+    uint32_t m = v[0];
+#pragma unroll
+    for (uint32_t j = 1; j < kGroupKeys; ++j) m = min(m, v[j]);
+    gmin[int64_t(blockIdx.y) * G + g] = m;
+}
+
 bool fb_fits(const va_context* ctx, size_t need, uint32_t rows, uint32_t N, uint32_t k) {
     return fb_fits_in(ctx->fixed_scratch ? ctx->fixed_scratch_bytes : 0, need, rows, N, k);
 }
@@ -162,6 +179,12 @@ uint32_t sample_rank(const va_context* ctx, uint32_t k, uint64_t S, uint32_t N, 
     return sample_rank_for(ctx->opt_sample_rank, k, S, N, masked);
 }
 
+// Up to this many (query, row) pairs a search writes every key and selects from them: two or three
+// launches instead of the sampled scan's five or six and its second pass over part of the rows.
+// Measured per search, k = 10, dense against sampled: fp32 768-d, 50,000 rows, Q = 8 57 / 83 us,
+// Q = 40 (2M pairs) 107 / 129, 200,000 rows, Q = 40 (8M) 290 / 286; int8 512-d, 20,000 rows, Q = 160
+// (3.2M) 53 / 56, 50,000 rows, Q = 160 (8M) 89 / 68; PQ, 500,000 rows, Q = 8 (4M) 80 / 83.
+constexpr uint64_t kDensePairs = 4ull << 20;
 va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t N, uint32_t k,
                           const ScanOutputs& out) {
     SelectArgs base;
@@ -174,9 +197,11 @@ va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t
     base.key_bits = kp.key_bits();
 
     // ---- plan ------------------------------------------------------------------------
+    const bool automatic = !ctx->opt_candidate_cap && !ctx->opt_sample_rows && !ctx->opt_sample_rank;
     const ScanPlan plan = plan_scan(ctx, Q, N, k);
     const uint64_t S = plan.S;
-    const bool direct = plan.direct;
+    const bool direct = plan.direct || (automatic && uint64_t(Q) * N <= kDensePairs &&
+                                        uint64_t(Q) * N * 4 <= dense_budget(ctx));
     ScanPhaseMarks pm(ctx);
     ctx->last_scan = va_scan_timings{};
     VA_CHECK_STATUS(pm.mark(0));
@@ -185,9 +210,12 @@ va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t
         // small database: dense keys in query chunks + select
         const uint64_t per_q = uint64_t(N) * 4;
         uint32_t qc = uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(Q, dense_budget(ctx) / per_q)));
+        const uint64_t win = qc * select_scratch(N, k);  // winners of the rows' segments
         Scratch s(ctx);
-        VA_CHECK_STATUS(s.reserve(Scratch::round(uint64_t(qc) * per_q)));
+        VA_CHECK_STATUS(s.reserve(Scratch::round(uint64_t(qc) * per_q) + Scratch::round(win * 4) * 2));
         uint32_t* keys = s.carve<uint32_t>(uint64_t(qc) * N);
+        uint32_t* wkey = s.carve<uint32_t>(win);
+        uint32_t* wid = s.carve<uint32_t>(win);
         for (uint32_t q0 = 0; q0 < Q; q0 += qc) {
             const uint32_t nq = std::min(qc, Q - q0);
             VA_CHECK_STATUS(kp.dense(nullptr, q0, nq, 0, N, 1, keys, N));
@@ -202,7 +230,7 @@ va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t
             if (out.f) a.out_f = out.f + int64_t(q0) * k;
             if (out.i32) a.out_i32 = out.i32 + int64_t(q0) * k;
             if (out.key) a.out_key = out.key + int64_t(q0) * k;
-            VA_CHECK_STATUS(launch_select(ctx, a));
+            VA_CHECK_STATUS(launch_select_dense(ctx, a, wkey, wid));
         }
         return pm.finish(false, false);
     }
@@ -210,6 +238,13 @@ va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t
     const uint64_t cap = plan.cap;
     const uint32_t rank = sample_rank(ctx, k, S, N, out.skip != nullptr);
     const uint32_t qs = plan.qs;
+    // The threshold may be looser than the sample's rank-th key (a rank below k is checked by the
+    // selection, rank k only needs an upper bound of the k-th key), so it is the rank-th smallest
+    // of the minima of groups of keys: one workgroup per query over the whole sample row was a
+    // serial pass of 16K-260K keys (10M int8 rows, Q = 32: 263 us on 32 workgroups, now 20).
+    // The minima sit where the candidate lists go later.
+    const uint32_t groups = ceil_div(S, kGroupKeys);
+    const bool group_min = S >= 128ull * rank && uint64_t(qs) * groups <= 2 * uint64_t(Q) * cap;
 
     Scratch s(ctx);
     size_t need = exact_scan_need(Q, plan);
@@ -224,6 +259,7 @@ va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t
     uint32_t* cid = s.carve<uint32_t>(uint64_t(Q) * cap);
     uint32_t* ovf_cnt = s.carve<uint32_t>(kZeroWords);
     uint32_t* skeys = s.carve<uint32_t>(uint64_t(qs) * S);
+    uint32_t* const gkeys = ckey;  // (ckey and cid are adjacent)
     FbArgs fb;
     if (device_fb) {
         fb = fb_carve(s, Q, N, k);
@@ -239,10 +275,17 @@ va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t
         const uint32_t nq = std::min(qs, Q - q0);
         VA_CHECK_STATUS(kp.dense(nullptr, q0, nq, 0, uint32_t(S), stride, skeys, int64_t(S)));
         VA_CHECK_STATUS(mask_dense_keys(ctx, skeys, nq, uint32_t(S), int64_t(S), 0, stride, out.skip));
+        if (group_min)
+            for (uint32_t r0 = 0; r0 < nq; r0 += 65535) {
+                const uint32_t nr = std::min<uint32_t>(65535, nq - r0);
+                group_min_kernel<<<dim3((groups + 255) / 256, nr), dim3(256), 0, ctx->stream>>>(
+                    skeys + uint64_t(r0) * S, int64_t(S), uint32_t(S), groups, gkeys + uint64_t(r0) * groups);
+                VA_CHECK_LAUNCH(ctx);
+            }
         SelectArgs a;
-        a.keys = skeys;
-        a.ld = int64_t(S);
-        a.n = uint32_t(S);
+        a.keys = group_min ? gkeys : skeys;
+        a.n = group_min ? groups : uint32_t(S);
+        a.ld = int64_t(a.n);
         a.rows = nq;
         a.k = rank;
         a.out_kth = thr + q0;

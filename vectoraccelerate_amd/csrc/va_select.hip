@@ -1,7 +1,8 @@
 // va_select.hip — exact row-wise top-k on 32-bit ordering keys.
 //
-// One workgroup per row:
-//   1. radix select (4 x 8-bit LDS histograms) finds T, the k-th smallest key;
+// One workgroup per row (or per segment of a long dense row):
+//   1. radix select (LDS histograms of 11 bits, below the bits all keys share) finds T, the k-th
+//      smallest key;
 //   2. when more items share T than are needed, a second radix select over the ids of the
 //      key == T items finds the cut id, so ties go to the lower index;
 //   3. the exactly-k winners are gathered into LDS and bitonic-sorted by (key, id).
@@ -16,14 +17,20 @@
 namespace va {
 namespace {
 
-// One workgroup per row.
-template <bool CACHED, bool KTH = false>
-__global__ __launch_bounds__(SEL_THREADS) void select_kernel(SelectArgs a) {
-    extern __shared__ uint32_t s_row[];  // CACHED: the row's keys
+// One workgroup per row.  Not CACHED (long rows, lists of a large capacity): a list that turns out
+// to hold at most kSelList keys is still copied to LDS.
+constexpr uint32_t kSelList = 4096;
+template <int NT, bool CACHED, bool KTH = false>
+__global__ __launch_bounds__(NT) void select_kernel(SelectArgs a) {
+    extern __shared__ uint32_t s_row[];  // the row's keys
+    __shared__ SelectLds<KTH> lds;
     const uint32_t row = blockIdx.x;
     if (a.zero_cnt && threadIdx.x == 0) a.zero_cnt[row] = 0;
     if (a.zero_words && row == 0 && threadIdx.x < kZeroWords) a.zero_words[threadIdx.x] = 0;
-    select_row<CACHED, KTH>(a, row, s_row);
+    if (CACHED || (a.counts && a.counts[row] <= kSelList))
+        select_row<NT, true, KTH>(a, row, lds, s_row);
+    else
+        select_row<NT, false, KTH>(a, row, lds, s_row);
 }
 
 // float values -> ordering keys (dense matrices given to va_topk_select)
@@ -62,21 +69,62 @@ va_status launch_select(va_context* ctx, const SelectArgs& a) {
     // Candidate lists are mostly far below their capacity, which sizes the LDS copy: past 8K
     // entries a large copy would leave one workgroup per CU, so such rows are read from memory
     // (L2-resident lists) by many workgroups at once instead.
-    const bool cache = a.n <= kSelCache && !((a.counts || a.out_kth) && a.n > 8192);
-    if (!cache && a.out_kth) {
-        select_kernel<false, true><<<dim3(a.rows), dim3(SEL_THREADS), 0, ctx->stream>>>(a);
-    } else if (cache) {
-        const size_t lds = size_t(std::max<uint32_t>(a.n, 1)) * 4;
-        auto kern = a.out_kth ? &select_kernel<true, true> : &select_kernel<true, false>;
+    const uint32_t n = a.nseg ? a.seg : a.n;
+    const bool cache = n <= kSelCache && !((a.counts || a.out_kth) && n > 8192);
+    const size_t lds = size_t(cache ? std::max<uint32_t>(n, 1) : (a.counts ? kSelList : 0)) * 4;
+    auto go = [&](auto kern, int threads) -> va_status {
         if (lds > 48 * 1024)
             VA_CHECK_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-        kern<<<dim3(a.rows), dim3(SEL_THREADS), lds, ctx->stream>>>(a);
-    } else {
-        select_kernel<false><<<dim3(a.rows), dim3(SEL_THREADS), 0, ctx->stream>>>(a);
-    }
+        kern<<<dim3(a.rows), dim3(threads), lds, ctx->stream>>>(a);
+        return VA_OK;
+    };
+    // A few long rows: 1,024 threads each, since a row's passes are a serial chain and the chip has
+    // room; many rows share a CU with 256.
+    const bool tall = n > 1024 && a.rows <= 2 * uint32_t(ctx->num_cus);
+    if (a.out_kth)
+        VA_CHECK_STATUS(cache ? (tall ? go(&select_kernel<1024, true, true>, 1024) : go(&select_kernel<256, true, true>, 256))
+                              : (tall ? go(&select_kernel<1024, false, true>, 1024)
+                                      : go(&select_kernel<256, false, true>, 256)));
+    else
+        VA_CHECK_STATUS(cache ? (tall ? go(&select_kernel<1024, true>, 1024) : go(&select_kernel<256, true>, 256))
+                              : (tall ? go(&select_kernel<1024, false>, 1024) : go(&select_kernel<256, false>, 256)));
     VA_CHECK_LAUNCH(ctx);
     return VA_OK;
+}
+
+// A long row is bound by its one workgroup: the passes over the row are serial, and a batch of few
+// queries leaves most of the chip idle.  Rows past kSegRow keys are cut into segments of at least
+// kSegKeys keys (16 k for large k, so that the winners are a small part of the row), each segment's
+// top-k selected by a workgroup of its own and the winners merged (20,000 keys, one query: 31 ->
+// 12 us; a whole search of 49,999 x 300, Q = 37 138 -> 59 us with the dense path).
+constexpr uint32_t kSegRow = 8192, kSegKeys = 4096;
+uint32_t select_segments(uint32_t n, uint32_t k) {
+    if (n <= kSegRow) return 0;
+    return n / std::max(kSegKeys, 16u * k);
+}
+
+va_status launch_select_dense(va_context* ctx, const SelectArgs& a, uint32_t* wkey, uint32_t* wid) {
+    const uint32_t nseg = select_segments(a.n, a.k);
+    if (nseg <= 1) return launch_select(ctx, a);
+    SelectArgs p;
+    p.keys = a.keys;
+    p.ld = a.ld;
+    p.n = a.n;
+    p.rows = a.rows * nseg;
+    p.k = a.k;
+    p.seg = (a.n + nseg - 1) / nseg;
+    p.nseg = nseg;
+    p.key_bits = a.key_bits;
+    p.out_idx = wid;
+    p.out_key = wkey;
+    VA_CHECK_STATUS(launch_select(ctx, p));
+    SelectArgs m = a;
+    m.keys = wkey;
+    m.ids = wid;
+    m.ld = int64_t(nseg) * a.k;
+    m.n = nseg * a.k;
+    return launch_select(ctx, m);
 }
 
 }  // namespace va
@@ -93,8 +141,11 @@ va_status va_topk_select(va_context* ctx, const float* values, uint32_t num_rows
     va::DeviceGuard g(ctx->device);
     const uint64_t total = uint64_t(num_rows) * num_elements;
     va::Scratch s(ctx);
-    VA_CHECK_STATUS(s.reserve(va::Scratch::round(total * 4)));
+    const uint64_t win = num_rows * va::select_scratch(num_elements, k);
+    VA_CHECK_STATUS(s.reserve(va::Scratch::round(total * 4) + va::Scratch::round(win * 4) * 2));
     uint32_t* keys = s.carve<uint32_t>(total);
+    uint32_t* wkey = s.carve<uint32_t>(win);
+    uint32_t* wid = s.carve<uint32_t>(win);
     uint64_t blocks = (total + 255) / 256;
     if (blocks > 8192) blocks = 8192;
     va::keys_from_floats<<<dim3(uint32_t(blocks)), dim3(256), 0, ctx->stream>>>(values, total, mode == VA_SELECT_MAX,
@@ -109,7 +160,7 @@ va_status va_topk_select(va_context* ctx, const float* values, uint32_t num_rows
     a.out_idx = out_idx;
     a.out_f = out_values;
     a.key_kind = mode == VA_SELECT_MAX ? 1 : 0;
-    return va::launch_select(ctx, a);
+    return va::launch_select_dense(ctx, a, wkey, wid);
 }
 
 va_status va_topk_merge(va_context* ctx, const uint32_t* a_idx, const float* a_dist, const uint32_t* b_idx,

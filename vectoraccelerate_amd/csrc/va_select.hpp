@@ -13,6 +13,8 @@ constexpr uint32_t SEL_BUF = VA_MAX_K;  // winners buffer (k <= VA_MAX_K)
 // the radix passes then read LDS instead of re-reading the row from memory once per pass with
 // one load in flight per thread, which left a short row's workgroup waiting on memory latency.
 constexpr uint32_t kSelCache = 24576;  // 96 KiB
+constexpr uint32_t SEL_FEW = 128;   // items ranked by comparing all pairs
+constexpr uint32_t SEL_BITS = 11, SEL_BINS = 1u << SEL_BITS;  // bits and bins of one histogram pass
 
 template <bool CACHED>
 struct RowView {
@@ -23,50 +25,27 @@ struct RowView {
     __device__ uint32_t id(uint32_t i) const { return ids ? ids[i] : i; }
 };
 
-// Wave 0 scans the 256-bin histogram and finds the bin holding the `need`-th item.
-// Writes digit, the count before it, and the bin count to shared memory.
-__device__ inline void find_digit(const uint32_t* hist, uint32_t need, uint32_t* s_digit, uint32_t* s_before,
-                           uint32_t* s_bin) {
-    const int lane = threadIdx.x & 63;
-    if (threadIdx.x >= 64) return;
-    uint32_t c[4];
-    uint32_t sum = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        c[i] = hist[lane * 4 + i];
-        sum += c[i];
-    }
-    uint32_t incl = sum;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        uint32_t o = __shfl_up(incl, off);
-        if (lane >= off) incl += o;
-    }
-    uint32_t excl = incl - sum;
-    if (excl < need && need <= incl) {
-        uint32_t run = excl;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if (run < need && need <= run + c[i]) {
-                *s_digit = uint32_t(lane * 4 + i);
-                *s_before = run;
-                *s_bin = c[i];
-            }
-            run += c[i];
-        }
-    }
-}
+// The LDS of a row's selection (KTH: threshold mode, without the winners).
+template <bool KTH>
+struct SelectLds {
+    uint32_t digit, before, bin, cnt, lo, hi;
+    uint32_t wsum[16];
+    uint32_t whist[SEL_BINS];
+    uint32_t okey[KTH ? 1 : SEL_BUF];
+    uint32_t oid[KTH ? 1 : SEL_BUF];
+};
 
-// The bin of a histogram of nb <= 2048 bins holding the need-th item: each thread sums eight
-// bins, a block-wide scan of the sums, then the thread whose range holds the item finds it.
-__device__ inline void find_bin_wide(const uint32_t* hist, uint32_t nb, uint32_t need, uint32_t* s_digit,
-                              uint32_t* s_before, uint32_t* s_bin) {
-    __shared__ uint32_t wsum[SEL_THREADS / 64];
+// The bin of a histogram of nb <= 2048 bins holding the need-th item: each thread sums a
+// few bins, a block-wide scan of the sums, then the thread whose range holds the item finds it.
+template <int NT>
+__device__ inline void find_bin_wide(const uint32_t* hist, uint32_t nb, uint32_t need, uint32_t* wsum,
+                                     uint32_t* s_digit, uint32_t* s_before, uint32_t* s_bin) {
+    constexpr int PER = int(SEL_BINS) / NT;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    uint32_t c[8], sum = 0;
+    uint32_t c[PER], sum = 0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const uint32_t b = uint32_t(tid) * 8 + i;
+    for (int i = 0; i < PER; ++i) {
+        const uint32_t b = uint32_t(tid) * PER + i;
         c[i] = b < nb ? hist[b] : 0u;
         sum += c[i];
     }
@@ -85,9 +64,9 @@ __device__ inline void find_bin_wide(const uint32_t* hist, uint32_t nb, uint32_t
     if (excl < need && need <= incl) {
         uint32_t run = excl;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < PER; ++i) {
             if (run < need && need <= run + c[i]) {
-                *s_digit = uint32_t(tid) * 8 + i;
+                *s_digit = uint32_t(tid) * PER + i;
                 *s_before = run;
                 *s_bin = c[i];
             }
@@ -96,40 +75,51 @@ __device__ inline void find_bin_wide(const uint32_t* hist, uint32_t nb, uint32_t
     }
 }
 
-// Adds this lane's item to the histogram when m.  Keys of one search crowd into few digits
-// (the top bytes of nearby distances are equal; Hamming distances are below 1024), and 256
-// threads incrementing one LDS bin serialise: when every active lane of the wave adds to the
-// same bin, one lane adds the wave's count.
+// Adds this lane's item to bin d of the histogram when m.  Keys of one search crowd into few bins
+// (ties, excluded rows, Hamming distances), and 64 lanes incrementing one LDS word serialise: the
+// bins of the first two lanes still waiting are each added once for all lanes that share them, the
+// rest one by one.
 __device__ __forceinline__ void hist_add(uint32_t* hist, bool m, uint32_t d) {
-    const uint32_t dd = m ? d : 0xFFFFFFFFu;
-    const uint32_t first = __builtin_amdgcn_readfirstlane(dd);
-    const uint64_t act = __ballot(1);
-    if (__ballot(dd == first) == act) {
-        if (first != 0xFFFFFFFFu && (threadIdx.x & 63) == uint32_t(__builtin_ctzll(act)))
-            atomicAdd(&hist[first], uint32_t(__popcll(act)));
-    } else if (m) {
-        atomicAdd(&hist[d], 1u);
+    uint64_t rest = __ballot(m);
+    const uint32_t lane = threadIdx.x & 63;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        if (!rest) return;
+        const int l = __builtin_ctzll(rest);
+        const uint32_t f = uint32_t(__builtin_amdgcn_readlane(int(d), l));
+        const uint64_t same = __ballot(m && d == f) & rest;
+        if (lane == uint32_t(l)) atomicAdd(&hist[f], uint32_t(__popcll(same)));
+        rest &= ~same;
     }
+    if ((rest >> lane) & 1ull) atomicAdd(&hist[d], 1u);
 }
 
-// Exact top-k of one row (every thread of a SEL_THREADS-thread workgroup calls it; a caller that
-// selects several rows in turn puts a barrier between them).  KTH: threshold mode only (a.out_kth
+// Exact top-k of one row (every thread of an NT-thread workgroup calls it; a caller that selects
+// several rows in turn puts a barrier between them).  KTH: threshold mode only (a.out_kth
 // set): no winners buffer, so a cached row of up to 16K keys leaves room for two workgroups per CU.
 // CACHED: the row's keys are copied to s_row (LDS) first.
-template <bool CACHED, bool KTH>
-__device__ void select_row(const SelectArgs& a, uint32_t row, uint32_t* s_row) {
-    __shared__ uint32_t hist[256];
-    __shared__ uint32_t s_digit, s_before, s_bin, s_cnt;
-    __shared__ uint32_t okey[KTH ? 1 : SEL_BUF];
-    __shared__ uint32_t oid[KTH ? 1 : SEL_BUF];
-    __shared__ uint32_t whist[2048];     // one-pass histogram of keys below 2^11
+template <int NT, bool CACHED, bool KTH>
+__device__ void select_row(const SelectArgs& a, uint32_t row, SelectLds<KTH>& lds, uint32_t* s_row) {
+    uint32_t &s_digit = lds.digit, &s_before = lds.before, &s_bin = lds.bin, &s_cnt = lds.cnt;
+    uint32_t &s_lo = lds.lo, &s_hi = lds.hi;
+    uint32_t *const okey = lds.okey, *const oid = lds.oid, *const whist = lds.whist;
     const int tid = threadIdx.x;
     const uint32_t orow = a.row_map ? a.row_map[row] : row;
 
     RowView<CACHED> rv;
-    rv.keys = a.keys + int64_t(row) * a.ld;
-    rv.ids = a.ids ? a.ids + int64_t(row) * a.ld : nullptr;
-    rv.n = a.n;
+    uint32_t id_offset = a.id_offset;
+    if (a.nseg) {
+        // segment row % nseg of dense row row / nseg
+        const uint32_t s0 = (row % a.nseg) * a.seg;
+        rv.keys = a.keys + int64_t(row / a.nseg) * a.ld + s0;
+        rv.ids = nullptr;
+        rv.n = min(a.seg, a.n - s0);
+        id_offset += s0;
+    } else {
+        rv.keys = a.keys + int64_t(row) * a.ld;
+        rv.ids = a.ids ? a.ids + int64_t(row) * a.ld : nullptr;
+        rv.n = a.n;
+    }
     if (a.counts) {
         const uint32_t c = a.counts[row];
         if (c > a.n || c < a.min_count) {
@@ -144,19 +134,24 @@ __device__ void select_row(const SelectArgs& a, uint32_t row, uint32_t* s_row) {
         rv.n = c;
     }
     const uint32_t n = rv.n;
+    uint32_t mn = 0xFFFFFFFFu, mx = 0;  // of this thread's keys
     if (CACHED) {
         // eight independent loads per thread per round
-        for (uint32_t i0 = 0; i0 < n; i0 += 8 * SEL_THREADS) {
+        for (uint32_t i0 = 0; i0 < n; i0 += 8 * NT) {
             uint32_t v[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                const uint32_t i = i0 + uint32_t(j * SEL_THREADS + tid);
+                const uint32_t i = i0 + uint32_t(j * NT + tid);
                 v[j] = i < n ? rv.keys[i] : 0u;
             }
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                const uint32_t i = i0 + uint32_t(j * SEL_THREADS + tid);
-                if (i < n) s_row[i] = v[j];
+                const uint32_t i = i0 + uint32_t(j * NT + tid);
+                if (i < n) {
+                    s_row[i] = v[j];
+                    mn = min(mn, v[j]);
+                    mx = max(mx, v[j]);
+                }
             }
         }
         rv.keys = s_row;
@@ -168,79 +163,122 @@ __device__ void select_row(const SelectArgs& a, uint32_t row, uint32_t* s_row) {
     auto for_keys = [&](auto&& f) {
         uint32_t i = uint32_t(tid);
         if (!CACHED)
-            for (; i + 7u * SEL_THREADS < n; i += 8u * SEL_THREADS) {
+            for (; i + 7u * NT < n; i += 8u * NT) {
                 uint32_t v[8];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) v[j] = rv.key(i + uint32_t(j) * SEL_THREADS);
+                for (int j = 0; j < 8; ++j) v[j] = rv.key(i + uint32_t(j) * NT);
 #pragma unroll
                 for (int j = 0; j < 8; ++j) f(v[j]);
             }
-        for (; i < n; i += SEL_THREADS) f(rv.key(i));
+        for (; i < n; i += NT) f(rv.key(i));
+    };
+
+    // The need-th smallest value of the items for_vals(f) runs f(value, taken) over, all within
+    // [base, base + 2^bits): histograms of up to 11 bits at a time, from the top, until the bin that
+    // holds it has at most SEL_FEW items (the tail of a spread of distances: usually after the
+    // first), which are ranked directly.  need becomes its rank among the items equal to it, eq
+    // their number.
+    auto radix = [&](auto&& for_vals, uint32_t base, uint32_t bits, uint32_t& need, uint32_t& eq) {
+        uint32_t prefix = 0;
+        uint32_t left = bits;
+        while (left) {
+            const uint32_t w = left < SEL_BITS ? left : SEL_BITS, sh = left - w, nb = 1u << w;
+            for (uint32_t b = tid; b < nb; b += NT) whist[b] = 0;
+            __syncthreads();
+            for_vals([&](uint32_t v, bool taken) {
+                const uint32_t d = v - base;
+                const bool m = taken && (left == bits || (d >> left) == prefix);
+                // (a value past the range, a sentinel above every real one, lands in the top bin)
+                const uint32_t bin = d >> sh;
+                hist_add(whist, m, left == bits ? min(bin, nb - 1u) : (bin & (nb - 1u)));
+            });
+            __syncthreads();
+            find_bin_wide<NT>(whist, nb, need, lds.wsum, &s_digit, &s_before, &s_bin);
+            __syncthreads();
+            prefix = (prefix << w) | s_digit;
+            need -= s_before;
+            eq = s_bin;
+            left = sh;
+            __syncthreads();
+            if (left && eq <= SEL_FEW) {
+                if (tid == 0) s_cnt = 0;
+                __syncthreads();
+                for_vals([&](uint32_t v, bool taken) {
+                    if (taken && ((v - base) >> left) == prefix) whist[atomicAdd(&s_cnt, 1u)] = v;
+                });
+                __syncthreads();
+                const uint32_t few = eq, want = need;
+                if (uint32_t(tid) < few) {
+                    const uint32_t v = whist[tid];
+                    uint32_t below = 0, same = 0;
+                    for (uint32_t j = 0; j < few; ++j) {
+                        const uint32_t o = whist[j];
+                        below += o < v;
+                        same += o == v;
+                    }
+                    if (below < want && want <= below + same) {  // (every item equal to the answer writes the same)
+                        s_lo = v;
+                        s_before = below;
+                        s_bin = same;
+                    }
+                }
+                __syncthreads();
+                const uint32_t t = s_lo;
+                need = want - s_before;
+                eq = s_bin;
+                __syncthreads();
+                return t;
+            }
+        }
+        return base + prefix;
     };
 
     uint32_t T = 0xFFFFFFFFu, Tid = 0xFFFFFFFFu;
     bool take_all = (n <= a.k);
     if (!take_all) {
         // ---- phase 1: k-th smallest key ---------------------------------------------
-        uint32_t prefix = 0, mask = 0, need = K;
-        uint32_t eq = 0;
-        int top = 24;  // first byte pass
-        if (a.key_bits <= 11) {
-            // small keys: one histogram over all key values
-            const uint32_t nb = 1u << a.key_bits;
-            for (uint32_t b = tid; b < nb; b += SEL_THREADS) whist[b] = 0;
+        // The histograms start below the leading bits that all keys share: nearby distances have
+        // equal top bits, and bins of those bits alone would count everything in one bin.
+        uint32_t need = K, eq = n, lo = 0, bits = a.key_bits;
+        if (a.key_bits > SEL_BITS) {
+            if (!CACHED)
+                for_keys([&](uint32_t k) {
+                    mn = min(mn, k);
+                    mx = max(mx, k);
+                });
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) {
+                mn = min(mn, uint32_t(__shfl_xor(int(mn), off)));
+                mx = max(mx, uint32_t(__shfl_xor(int(mx), off)));
+            }
+            if (tid == 0) {
+                s_lo = 0xFFFFFFFFu;
+                s_hi = 0;
+            }
             __syncthreads();
-            // (a sentinel key, above every real one, lands in the top bin)
-            for_keys([&](uint32_t k) { hist_add(whist, true, min(k, nb - 1u)); });
+            if ((tid & 63) == 0) {
+                atomicMin(&s_lo, mn);
+                atomicMax(&s_hi, mx);
+            }
             __syncthreads();
-            find_bin_wide(whist, nb, need, &s_digit, &s_before, &s_bin);
-            __syncthreads();
-            prefix = s_digit;
-            mask = 0xFFFFFFFFu;
-            need -= s_before;
-            eq = s_bin;
-            __syncthreads();
-            top = -8;  // no byte passes left
+            lo = s_lo;
+            bits = s_hi == lo ? 0u : 32u - uint32_t(__builtin_clz(s_hi - lo));
         }
-        for (int shift = top; shift >= 0; shift -= 8) {
-            hist[tid] = 0;
-            __syncthreads();
-            for_keys([&](uint32_t k) { hist_add(hist, (k & mask) == prefix, (k >> shift) & 255u); });
-            __syncthreads();
-            find_digit(hist, need, &s_digit, &s_before, &s_bin);
-            __syncthreads();
-            prefix |= s_digit << shift;
-            mask |= 255u << shift;
-            need -= s_before;
-            eq = s_bin;
-            __syncthreads();
-        }
-        T = prefix;
+        T = radix([&](auto&& f) { for_keys([&](uint32_t k) { f(k, true); }); }, lo, bits, need, eq);
         if (KTH || a.out_kth) {
             if (tid == 0) a.out_kth[orow] = T;
             return;
         }
         // ---- phase 2: among key == T take the `need` lowest ids ----------------------
-        if (need < eq) {
-            uint32_t ip = 0, im = 0, ineed = need;
-            for (int shift = 24; shift >= 0; shift -= 8) {
-                hist[tid] = 0;
-                __syncthreads();
-                for (uint32_t i = tid; i < n; i += SEL_THREADS) {
-                    const bool t = rv.key(i) == T;
-                    const uint32_t id = t ? rv.id(i) : 0u;
-                    hist_add(hist, t && (id & im) == ip, (id >> shift) & 255u);
-                }
-                __syncthreads();
-                find_digit(hist, ineed, &s_digit, &s_before, &s_bin);
-                __syncthreads();
-                ip |= s_digit << shift;
-                im |= 255u << shift;
-                ineed -= s_before;
-                __syncthreads();
-            }
-            Tid = ip;
-        }
+        if (need < eq)
+            Tid = radix(
+                [&](auto&& f) {
+                    for (uint32_t i = tid; i < n; i += NT) {
+                        const bool t = rv.key(i) == T;
+                        f(t ? rv.id(i) : 0u, t);
+                    }
+                },
+                0u, 32u, need, eq);
     } else if (a.out_kth) {
         // fewer items than k: every key passes
         if (tid == 0) a.out_kth[orow] = 0xFFFFFFFFu;
@@ -251,7 +289,7 @@ __device__ void select_row(const SelectArgs& a, uint32_t row, uint32_t* s_row) {
     if constexpr (KTH) return;  // threshold launches always have out_kth (returned above)
     if (tid == 0) s_cnt = 0;
     __syncthreads();
-    for (uint32_t i = tid; i < n; i += SEL_THREADS) {
+    for (uint32_t i = tid; i < n; i += NT) {
         const uint32_t k = rv.key(i);
         if (take_all || k < T || k == T) {
             const uint32_t id = rv.id(i);
@@ -265,17 +303,46 @@ __device__ void select_row(const SelectArgs& a, uint32_t row, uint32_t* s_row) {
         }
     }
     __syncthreads();
-    uint32_t cnt = s_cnt < SEL_BUF ? s_cnt : SEL_BUF;
+    const uint32_t cnt = s_cnt < SEL_BUF ? s_cnt : SEL_BUF;
+    // slot r of the output: winner (wk, wid), or missing
+    auto put = [&](uint32_t r, bool have, uint32_t wk, uint32_t wid) {
+        const int64_t o = int64_t(orow) * (a.out_ld ? a.out_ld : int64_t(a.k)) + r;
+        have = have && wk != kAbsentKey;
+        const uint32_t k = have ? wk : 0xFFFFFFFFu;
+        if (a.out_idx) a.out_idx[o] = have ? wid + id_offset : kSentinel;
+        if (a.out_key) a.out_key[o] = k;
+        if (a.out_f) {
+            float v;
+            if (!have) v = (a.key_kind == 1) ? -__builtin_inff() : __builtin_inff();
+            else v = (a.key_kind == 1) ? float_of_key_desc(k) : float_of_key(k);
+            a.out_f[o] = v;
+        }
+        if (a.out_i32) a.out_i32[o] = have ? (a.key_kind == 3 ? int32_t(k) : i32_of_key(k)) : INT32_MAX;
+    };
+    if (cnt <= SEL_FEW) {
+        // few winners: each finds its slot by comparing itself with all of them
+        if (uint32_t(tid) < cnt) {
+            const uint32_t wk = okey[tid], wid = oid[tid];
+            uint32_t r = 0;
+            for (uint32_t j = 0; j < cnt; ++j) {
+                const uint32_t kj = okey[j], ij = oid[j];
+                r += kj < wk || (kj == wk && (ij < wid || (ij == wid && j < uint32_t(tid))));
+            }
+            if (r < K) put(r, true, wk, wid);
+        }
+        for (uint32_t r = min(cnt, K) + tid; r < a.k; r += NT) put(r, false, 0, 0);
+        return;
+    }
     uint32_t P = 1;
     while (P < cnt) P <<= 1;
-    for (uint32_t i = cnt + tid; i < P; i += SEL_THREADS) {
+    for (uint32_t i = cnt + tid; i < P; i += NT) {
         okey[i] = 0xFFFFFFFFu;
         oid[i] = 0xFFFFFFFFu;
     }
     __syncthreads();
     for (uint32_t size = 2; size <= P; size <<= 1) {
         for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-            for (uint32_t t = tid; t < P / 2; t += SEL_THREADS) {
+            for (uint32_t t = tid; t < P / 2; t += NT) {
                 const uint32_t i = 2 * t - (t & (stride - 1));
                 const uint32_t j = i + stride;
                 const bool asc = (i & size) == 0;
@@ -291,21 +358,7 @@ __device__ void select_row(const SelectArgs& a, uint32_t row, uint32_t* s_row) {
             __syncthreads();
         }
     }
-    // ---- write k slots -----------------------------------------------------------------
-    for (uint32_t r = tid; r < a.k; r += SEL_THREADS) {
-        const int64_t o = int64_t(orow) * (a.out_ld ? a.out_ld : int64_t(a.k)) + r;
-        const bool have = r < cnt && r < K && okey[r] != kAbsentKey;
-        const uint32_t k = have ? okey[r] : 0xFFFFFFFFu;
-        if (a.out_idx) a.out_idx[o] = have ? oid[r] + a.id_offset : kSentinel;
-        if (a.out_key) a.out_key[o] = k;
-        if (a.out_f) {
-            float v;
-            if (!have) v = (a.key_kind == 1) ? -__builtin_inff() : __builtin_inff();
-            else v = (a.key_kind == 1) ? float_of_key_desc(k) : float_of_key(k);
-            a.out_f[o] = v;
-        }
-        if (a.out_i32) a.out_i32[o] = have ? (a.key_kind == 3 ? int32_t(k) : i32_of_key(k)) : INT32_MAX;
-    }
+    for (uint32_t r = tid; r < a.k; r += NT) put(r, r < cnt && r < K, okey[r < cnt ? r : 0], oid[r < cnt ? r : 0]);
 }
 
 }  // namespace va
