@@ -155,7 +155,7 @@ __global__ __launch_bounds__(256) void hamming_scan_wide_kernel(HamArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Filter scan on the fp4 MFMA (large Q, rows of 8/16/24 words)
+// Filter scan on the fp4 MFMA (rows of 4, 8, 12, 16, 24 or 32 words)
 // ---------------------------------------------------------------------------------------
 // Hamming distance as |a| + |b| - 2 a.b over {0,1} vectors: a.b is a dot product of bits,
 // which the gfx950 matrix cores compute exactly with every bit widened to an fp4 (e2m1)
@@ -163,28 +163,36 @@ __global__ __launch_bounds__(256) void hamming_scan_wide_kernel(HamArgs a) {
 // (v_mfma_scale_f32_32x32x64_f8f6f4, unit scales, fp32 sums of integers <= 1024).  fp4 runs the 32x32x64 MFMA at 8 dense TFLOP/s-equivalents per CU per clock pair
 // of the int8 rate, so the 2·Q·N·32W bit products cost a fraction of the xor + popcount
 // VALU scan, which is bound by VALU issue (two ops per word per pair).
-// Layout and pipeline follow i8_resq_kernel: a workgroup keeps 256 queries resident in LDS
+// Layout and pipeline follow i8_resq_kernel: a workgroup keeps 32 NB queries resident in LDS
 // (already widened: 16 bytes per 32-bit word, rows padded to 16W + 16 bytes, which puts the
 // 16 rows of one ds_read_b128 clock in 16 distinct bank groups) and streams a contiguous range
 // of 256-row tiles past them; each of its eight waves owns 32 rows of a tile and loads them
 // straight into registers (lane: row l % 32, half h = l / 32 of its words, 16-byte loads;
 // the next tile in flight while this one computes), widens one 32-bit word per k-step into
-// the A fragment and runs 8 MFMAs against the 8 resident query blocks.  K mapping: k-step s
+// the A fragment and runs NB MFMAs against the resident query blocks.  K mapping: k-step s
 // takes word h·W/2 + s of the half, widened by the same bit-to-slot assignment on both sides
 // (widen_row, widen_query).  No workgroup barrier after the query load.  Filter epilogue as in
 // i8_resq_kernel: a pass is d <= tau, tested in the form 512 + a.b - |x|/2 >= 512 + (|q| -
 // tau)/2 with the accumulators started from 512 - |x|/2, a per-lane maximum first; passes go to
 // a per-wave LDS list flushed when full.
+// A batch takes the smallest of 32, 64, 128 and 256 resident queries that holds it.  One query is
+// already cheaper here than by xor + popcount (two VALU ops per word and pair; here ~5 per word of
+// a row and MFMAs that a batch shares).  Whole searches, 10M x 768 bits, top-10, popcount scan ->
+// here: Q = 1 245 -> 217 us (the codes alone are 170 us at the card's read rate), 32 479 -> 226, 64
+// 862 -> 270, 100 1,296 -> 441, 192 2,385 -> 695; 10M x 128 bits, Q = 32 845 -> 141.
 namespace hmf {
-constexpr int TQ = 256, NW = 8, WR = 32, TN = NW * WR, LCAP = 80;
-constexpr int STAGE = NW * LCAP * 12;
+constexpr int NW = 8, WR = 32, TN = NW * WR;
 constexpr int PA = NW * WR * 4;  // per-wave row popcounts
-constexpr int PB = TQ * 4;       // query popcounts
-// resident queries, chunk-major: 16-byte chunk c (of W) of query r at c * 4096 + r * 16, so the
-// fragments of all 8 query blocks of one k-step lie within a 16-bit DS offset of one address
-constexpr int qbytes(int W) { return TQ * 16 * W; }
+// staged passes per wave: fewer where a smaller tile then fits two workgroups per CU
+constexpr int lcap(int NB) { return NB == 8 ? 80 : 48; }
+constexpr int stage(int NB) { return NW * lcap(NB) * 12; }
+// resident queries, chunk-major: 16-byte chunk c (of W) of query r of 32 NB at c * 512 NB + r * 16, so
+// the fragments of all query blocks of one k-step lie within a 16-bit DS offset of one address
+constexpr int qbytes(int W, int NB) { return 32 * NB * 16 * W; }
 constexpr int rows_bytes(int W) { return NW * WR * (W + 1) * 4; }  // per-wave row words, rows W + 1 apart
-constexpr size_t lds_bytes(int W) { return size_t(qbytes(W)) + STAGE + PA + PB + rows_bytes(W); }
+constexpr size_t lds_bytes(int W, int NB) {
+    return size_t(qbytes(W, NB)) + stage(NB) + PA + 32 * NB * 4 + rows_bytes(W);
+}
 }  // namespace hmf
 
 // 32 bits -> 32 fp4 (e2m1) nibbles in four dwords: nibble i of dword j holds bit 4i + j of the
@@ -208,11 +216,12 @@ __device__ __forceinline__ i32x8h fp4_operand(const i32x4h& v) { return i32x8h{v
 typedef float f32x16h __attribute__((ext_vector_type(16)));
 typedef float f32x4h __attribute__((ext_vector_type(4)));
 
-template <int W>
-__global__ __launch_bounds__(512, 2) void hamming_mfma_kernel(HamArgs a, uint32_t R) {
+template <int W, int NB>
+__global__ __launch_bounds__(512, NB == 8 ? 2 : 4) void hamming_mfma_kernel(HamArgs a, uint32_t R) {
     using namespace hmf;
     constexpr int HW = W / 2;  // words per lane half = k-steps per tile
-    constexpr int QB = qbytes(W);
+    constexpr int TQ = 32 * NB, QB = qbytes(W, NB), STAGE = stage(NB), PB = TQ * 4, LCAP = lcap(NB);
+    constexpr int CS = TQ * 16;  // bytes per chunk of all resident queries
     extern __shared__ __attribute__((aligned(16))) char lds8[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -240,7 +249,7 @@ __global__ __launch_bounds__(512, 2) void hamming_mfma_kernel(HamArgs a, uint32_
         const int r = e / W, w = e % W;
         const uint32_t v = uint32_t(r) < qn ? a.q[uint64_t(q0 + r) * W + w] : 0u;
         const int c = 2 * (w % HW) + w / HW;
-        *reinterpret_cast<uint4*>(lds8 + c * 4096 + r * 16) = widen_query(v);
+        *reinterpret_cast<uint4*>(lds8 + c * CS + r * 16) = widen_query(v);
     }
     for (int r = tid; r < TQ; r += 512) {
         uint32_t pb = 0;
@@ -252,11 +261,11 @@ __global__ __launch_bounds__(512, 2) void hamming_mfma_kernel(HamArgs a, uint32_
     // pass iff 2 a.b - |x| >= |q| - tau, i.e. 512 + a.b - |x|/2 >= 512 + (|q| - tau)/2 (halves of
     // integers below 2^24: exact).  The accumulators start from 512 - |x|/2, so the left side is
     // what they hold, and every value on either side is a positive float (|x|, |q|, tau <= 32 W
-    // <= 768), whose bit patterns order like the values: the quick test is an unsigned maximum.
+    // <= 1024), whose bit patterns order like the values: the quick test is an unsigned maximum.
     // tau >= 32 W passes everything (0); padding never passes (+inf)
-    float cq[8];
+    float cq[NB];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < NB; ++u) {
         const uint32_t ql = uint32_t(u * 32 + l32);
         const uint32_t t = a.thr[q0 + (ql < qn ? ql : 0u)];
         cq[u] = ql >= qn ? __builtin_inff() : (t >= uint32_t(32 * W) ? 0.0f : 512.0f + 0.5f * (s_pb[ql] - float(t)));
@@ -270,21 +279,30 @@ __global__ __launch_bounds__(512, 2) void hamming_mfma_kernel(HamArgs a, uint32_
         const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<uint32_t*>(a.x + r0 * W), 0, int(rows * uint32_t(W) * 4u), 0x00020000);
         const uint32_t off = (uint32_t(l32) * W + uint32_t(hh) * HW) * 4u;
+        if constexpr (HW % 4 == 0) {
 #pragma unroll
-        for (int i = 0; i < HW / 4; ++i) {
-            const auto v = __builtin_amdgcn_raw_buffer_load_b128(xr, off + 16u * i, 0, 0);
-            xw[4 * i] = uint32_t(v[0]);
-            xw[4 * i + 1] = uint32_t(v[1]);
-            xw[4 * i + 2] = uint32_t(v[2]);
-            xw[4 * i + 3] = uint32_t(v[3]);
+            for (int i = 0; i < HW / 4; ++i) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b128(xr, off + 16u * i, 0, 0);
+                xw[4 * i] = uint32_t(v[0]);
+                xw[4 * i + 1] = uint32_t(v[1]);
+                xw[4 * i + 2] = uint32_t(v[2]);
+                xw[4 * i + 3] = uint32_t(v[3]);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < HW / 2; ++i) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b64(xr, off + 8u * i, 0, 0);
+                xw[2 * i] = uint32_t(v[0]);
+                xw[2 * i + 1] = uint32_t(v[1]);
+            }
         }
     };
-    const char* qrd = lds8 + hh * 4096 + l32 * 16;
+    const char* qrd = lds8 + hh * CS + l32 * 16;
     // The query fragments are the same for every tile; an opaque per-tile zero in their
     // address keeps the compiler from hoisting all 8 x W/2 of them out of the tile loop into
     // registers (it would spill them).
     uint32_t qz = 0;
-    auto rd_q = [&](int st, int u) { return *reinterpret_cast<const i32x4h*>(qrd + qz + st * 8192 + u * 512); };
+    auto rd_q = [&](int st, int u) { return *reinterpret_cast<const i32x4h*>(qrd + qz + st * (2 * CS) + u * 512); };
 
     // ---- filter epilogue ------------------------------------------------------------------
     uint32_t* s_qi = reinterpret_cast<uint32_t*>(lds8 + QB) + wave * 3 * LCAP;
@@ -305,14 +323,14 @@ __global__ __launch_bounds__(512, 2) void hamming_mfma_kernel(HamArgs a, uint32_
         }
         lc = 0;
     };
-    f32x16h acc[8];
+    f32x16h acc[NB];
     // Lane value v of a block is row 8 (v >> 2) + 4 hh + (v & 3) of the wave's 32; it holds
     // 512 + a.b - |x|/2 at the end of a tile.  The passes of block u of a tile whose first row id is
     // r0 and whose rows past N start at lim (this lane half's view) go to the staging list.
     auto block_passes = [&](int u, uint32_t r0, int32_t lim) {
         const float c = cq[u];
         // an opaque zero: without it the compiler precomputes this rare path's per-block query
-        // values for all 8 blocks ahead of the loop and spills them
+        // values for all blocks ahead of the loop and spills them
         uint32_t oz;
         asm volatile("v_mov_b32 %0, 0" : "=v"(oz));
         const uint32_t ql = uint32_t(u * 32 + l32) + oz;
@@ -352,9 +370,9 @@ __global__ __launch_bounds__(512, 2) void hamming_mfma_kernel(HamArgs a, uint32_
     // staging code.
     uint32_t xw[HW], xn[HW];
     load_tile(0, xw);
-    i32x4h bq[8];
+    i32x4h bq[NB];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) bq[u] = rd_q(0, u);
+    for (int u = 0; u < NB; ++u) bq[u] = rd_q(0, u);
     uint32_t* myrow = s_rw + l32 * (W + 1) + hh * HW;
     auto widen_operand = [&](uint32_t w) {
         const uint4 d = widen_row(w);
@@ -381,14 +399,14 @@ __global__ __launch_bounds__(512, 2) void hamming_mfma_kernel(HamArgs a, uint32_
         }
         asm volatile("v_mov_b32 %0, 0" : "=v"(qz));
         // One k-step: block u's MFMA, then the read of its fragment for the next step, a full
-        // step (8 MFMAs) ahead of its use; the row word of the step after next is read at the
+        // step (NB MFMAs) ahead of its use; the row word of the step after next is read at the
         // start.  Scheduling barriers keep this program order: left alone, the scheduler moves
         // every read behind the step's last MFMA and the next step waits for all of them.
         uint32_t word = 0;
         auto k_step = [&](const i32x8h& af, const f32x16h* init, int nq, int nw) {
             if (nw >= 0) word = myrow[nw];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
+            for (int u = 0; u < NB; ++u) {
                 acc[u] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af, fp4_operand(bq[u]), init ? *init : acc[u],
                                                                          4, 4, 0, 127, 0, 127);
                 bq[u] = rd_q(nq, u);
@@ -408,7 +426,7 @@ __global__ __launch_bounds__(512, 2) void hamming_mfma_kernel(HamArgs a, uint32_
         if (lt + 1 < tcount) row_counts();
         uint32_t hit = 0;  // blocks with a lane whose best value passes (wave-uniform)
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < NB; ++u) {
             uint32_t m = __float_as_uint(acc[u][0]);
 #pragma unroll
             for (int v = 1; v < 16; ++v) m = max(m, __float_as_uint(acc[u][v]));
@@ -418,46 +436,60 @@ __global__ __launch_bounds__(512, 2) void hamming_mfma_kernel(HamArgs a, uint32_
             const uint64_t r64 = uint64_t(t0 + lt) * TN + uint32_t(wave) * WR;
             const int32_t lim = int32_t(r64 < N ? min(uint64_t(N) - r64, uint64_t(WR)) : 0) - 4 * hh;
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
+            for (int u = 0; u < NB; ++u)
                 if (hit & (1u << u)) block_passes(u, uint32_t(r64), lim);  // ids below N fit 32 bits
         }
     }
     flush();
 }
 
-// The fp4 MFMA filter scan needs whole 16-byte loads of each half row (W % 8 == 0), rows
-// whose widened queries fit the LDS with the row buffers (W <= 24), enough queries to fill a
-// 256-query block reasonably and dense rows.
+// The fp4 MFMA filter scan needs row halves of whole word pairs (W % 4 == 0), rows whose widened
+// queries fit the LDS with the row buffers, and dense, aligned rows.
 bool hmf_ok(const HamArgs& a) {
-#ifndef VA_HAM_MFMA
-#define VA_HAM_MFMA 1
-#endif
-    return VA_HAM_MFMA && !a.qrow && a.q0 == 0 && a.c0 == 0 && a.stride == 1 && a.nq > 192 &&
-           (a.W == 8 || a.W == 16 || a.W == 24) && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0 &&
+    return !a.qrow && a.q0 == 0 && a.c0 == 0 && a.stride == 1 && a.W >= 4 && a.W <= 32 &&
+           a.W % 4 == 0 && a.W != 20 && a.W != 28 && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0 &&
            uint64_t(a.cols) * a.W * 4 <= 0xFFFFFFFFFFFFull;
 }
 
-template <int W>
-va_status launch_hmf_w(va_context* ctx, const HamArgs& a) {
+template <int W, int NB>
+va_status launch_hmf_nb(va_context* ctx, const HamArgs& a) {
     using namespace hmf;
+    constexpr uint32_t TQ = 32 * NB;
+    // workgroups per CU by LDS and by the waves per SIMD the kernel is compiled for: two (one of 256
+    // queries), so that one's row loads are in flight while the other computes
+    constexpr uint32_t kPerCu = NB == 8 || 2 * lds_bytes(W, NB) > 160 * 1024 ? 1 : 2;
     const uint32_t nqb = (a.nq + TQ - 1) / TQ;
-    const uint32_t per = (uint32_t(std::max(ctx->num_cus, 8)) + nqb - 1) / nqb;
+    const uint32_t per = (kPerCu * uint32_t(std::max(ctx->num_cus, 8)) + nqb - 1) / nqb;
     const uint32_t R = std::max<uint32_t>(kXcds, (per + kXcds - 1) / kXcds * kXcds);
     const uint64_t grid = uint64_t(nqb) * R;
     if (grid > 0x7FFFFFFFull) return fail(ctx, VA_ERR_INVALID_ARG, "Hamming scan grid too large");
-    auto kern = &hamming_mfma_kernel<W>;
+    auto kern = &hamming_mfma_kernel<W, NB>;
     VA_CHECK_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, int(lds_bytes(W))));
-    kern<<<dim3(uint32_t(grid)), dim3(512), lds_bytes(W), ctx->stream>>>(a, R);
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, int(lds_bytes(W, NB))));
+    kern<<<dim3(uint32_t(grid)), dim3(512), lds_bytes(W, NB), ctx->stream>>>(a, R);
     VA_CHECK_LAUNCH(ctx);
     return VA_OK;
 }
 
+// 32, 64, 128 or 256 resident queries: the smallest that holds the batch (256 of 32-word queries do
+// not fit the LDS).
+template <int W>
+va_status launch_hmf_w(va_context* ctx, const HamArgs& a) {
+    if (a.nq <= 32) return launch_hmf_nb<W, 1>(ctx, a);
+    if (a.nq <= 64) return launch_hmf_nb<W, 2>(ctx, a);
+    if constexpr (W <= 24)
+        if (a.nq > 128) return launch_hmf_nb<W, 8>(ctx, a);
+    return launch_hmf_nb<W, 4>(ctx, a);
+}
+
 va_status launch_hmf(va_context* ctx, const HamArgs& a) {
     switch (a.W) {
+        case 4: return launch_hmf_w<4>(ctx, a);
         case 8: return launch_hmf_w<8>(ctx, a);
+        case 12: return launch_hmf_w<12>(ctx, a);
         case 16: return launch_hmf_w<16>(ctx, a);
-        default: return launch_hmf_w<24>(ctx, a);
+        case 24: return launch_hmf_w<24>(ctx, a);
+        default: return launch_hmf_w<32>(ctx, a);
     }
 }
 
@@ -467,23 +499,18 @@ va_status launch_ham(va_context* ctx, const HamArgs& a, bool filter) {
     const dim3 grid((a.cols + 255) / 256);
     const bool aligned = (a.W & 3) == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0;
     if (a.W <= kMaxWords && (aligned || (a.W & 3) != 0)) {
-#define VA_HAM_CASE(WC)                                                                       \
-    if (filter)                                                                               \
-        hamming_scan_kernel<WC, true><<<grid, dim3(256), 0, ctx->stream>>>(a);               \
-    else                                                                                      \
-        hamming_scan_kernel<WC, false><<<grid, dim3(256), 0, ctx->stream>>>(a);
-        if (a.W == 8 && aligned) {
-            VA_HAM_CASE(8)
-        } else if (a.W == 16 && aligned) {
-            VA_HAM_CASE(16)
-        } else if (a.W == 24 && aligned) {
-            VA_HAM_CASE(24)
-        } else if (a.W == 32 && aligned) {
-            VA_HAM_CASE(32)
-        } else {
-            VA_HAM_CASE(0)
-        }
-#undef VA_HAM_CASE
+        if (filter)  // (rows of other widths: the MFMA scan takes every aligned width below)
+            hamming_scan_kernel<0, true><<<grid, dim3(256), 0, ctx->stream>>>(a);
+        else if (a.W == 8 && aligned)
+            hamming_scan_kernel<8, false><<<grid, dim3(256), 0, ctx->stream>>>(a);
+        else if (a.W == 16 && aligned)
+            hamming_scan_kernel<16, false><<<grid, dim3(256), 0, ctx->stream>>>(a);
+        else if (a.W == 24 && aligned)
+            hamming_scan_kernel<24, false><<<grid, dim3(256), 0, ctx->stream>>>(a);
+        else if (a.W == 32 && aligned)
+            hamming_scan_kernel<32, false><<<grid, dim3(256), 0, ctx->stream>>>(a);
+        else
+            hamming_scan_kernel<0, false><<<grid, dim3(256), 0, ctx->stream>>>(a);
     } else {
         if (filter)
             hamming_scan_wide_kernel<true><<<grid, dim3(256), 0, ctx->stream>>>(a);

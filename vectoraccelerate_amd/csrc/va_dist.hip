@@ -623,8 +623,8 @@ __global__ __launch_bounds__(256, 2) void dist_stream_kernel(DistArgs a) {
 
 // The launches dist_stream_kernel takes: keys or a filter over dense query rows, at most 32 queries
 // or so few GEMM tiles that the chip would be mostly idle (past that the GEMM's tiles read the rows
-// once for up to 128 queries: 500,000 x 768, Q = 40 595 us on them, 810 streamed), every offset
-// within a tile below 2^31.
+// once for up to 128 queries: 500,000 x 768, Q = 40 595 us on them, 810 streamed; 4,096 x 768 centroids,
+// Q = 1,024 86 and 110), every offset within a tile below 2^31.
 bool stream_ok(const va_context* ctx, const DistArgs& a, int wq, int wn) {
     if (a.wq || a.wn || a.plan.pre || a.gather || a.qrow || a.ids || (a.out != OUT_KEYS && a.out != OUT_FILTER)) return false;
     if (a.op != OP_L2SQ && a.op != OP_L2 && a.op != OP_COS_DIST && a.op != OP_NEG_DOT) return false;
@@ -632,7 +632,10 @@ bool stream_ok(const va_context* ctx, const DistArgs& a, int wq, int wn) {
     if (uint64_t(31) * uint64_t(a.ldq) * 4 + uint64_t(a.D) * 4 > kDmaMaxBytes ||
         uint64_t(31) * uint64_t(a.ldx) * 4 + uint64_t(a.D) * 4 > kDmaMaxBytes)
         return false;
-    return a.Q <= 32 || uint64_t(ceil_div(a.Q, 32 * wq)) * ceil_div(a.N, 128 * wn) < 2ull * uint64_t(ctx->num_cus);
+    if (a.Q <= 32) return true;
+    const uint64_t waves = uint64_t(ceil_div(a.N, 32)) * ceil_div(a.Q, 32);
+    return (a.Q <= 64 || waves <= 8ull * uint64_t(ctx->num_cus)) &&
+           uint64_t(ceil_div(a.Q, 32 * wq)) * ceil_div(a.N, 128 * wn) < 2ull * uint64_t(ctx->num_cus);
 }
 
 template <int OUT, int OP>
