@@ -15,6 +15,7 @@
 #include <algorithm>
 
 #include "va_fallback.hpp"
+#include "va_int8.hpp"
 #include "va_internal.hpp"
 
 namespace va {
@@ -195,22 +196,6 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const int8_t* __restric
 #endif
 constexpr int KB = VA_I8_KB;           // bytes of each row per LDS stage (32-byte k-steps)
 constexpr int ROWB = KB + 16;          // +16 B pad: conflict-free ds_read_b128 across 16 rows
-
-struct I8Args {
-    const int8_t* q = nullptr;
-    const uint32_t* qrow = nullptr;
-    int64_t ldq = 0;
-    const int8_t* x = nullptr;
-    int64_t ldx = 0;
-    uint32_t Q = 0, N = 0, D = 0;
-    uint32_t* out_k = nullptr;
-    int64_t ldo = 0;
-    const uint32_t* thr = nullptr;
-    uint32_t* cnt = nullptr;
-    uint32_t* cand_key = nullptr;
-    uint32_t* cand_id = nullptr;
-    uint32_t cap = 0;
-};
 
 // Tile shapes: QBW query blocks of 32 per wave, WQ x WN waves; wave tile = 32*QBW queries x
 // 128 rows; workgroup tile = 32*QBW*WQ queries x 128*WN rows.  The 8-wave 256 x 256 shape is
@@ -1170,7 +1155,7 @@ bool resq_ok(const I8Args& a, bool vec) {
 #ifndef VA_I8_RESQ
 #define VA_I8_RESQ 1
 #endif
-    return VA_I8_RESQ && vec && !a.qrow && a.Q > 192 && a.D <= 512 && a.N <= 0xFFFFFF00u &&
+    return VA_I8_RESQ && vec && !a.qrow && a.Q > kI8SmallQueries && a.D <= 512 && a.N <= 0xFFFFFF00u &&
            uint64_t(resq::TQ - 1) * uint64_t(a.ldq) + a.D <= kDmaMaxBytes &&
            uint64_t(resq::WR - 1) * uint64_t(a.ldx) + a.D <= kDmaMaxBytes;
 }
@@ -1182,7 +1167,7 @@ bool resq16_ok(const I8Args& a, bool vec) {
 #ifndef VA_I8_RESQ16
 #define VA_I8_RESQ16 1
 #endif
-    return VA_I8_RESQ16 && vec && !a.qrow && a.Q > 192 && a.D % 256 == 0 && a.D <= 1024 &&
+    return VA_I8_RESQ16 && vec && !a.qrow && a.Q > kI8SmallQueries && a.D % 256 == 0 && a.D <= 1024 &&
            a.N <= 0xFFFFFE00u && uint64_t(resq16::TQMAX - 1) * uint64_t(a.ldq) + a.D <= kDmaMaxBytes &&
            uint64_t(resq16::WR - 1) * uint64_t(a.ldx) + a.D <= kDmaMaxBytes;
 }
@@ -1255,6 +1240,8 @@ bool i8_vec(const I8Args& a) {
 
 va_status launch_i8(va_context* ctx, const I8Args& a, bool filter) {
     if (a.Q == 0 || a.N == 0) return VA_OK;
+    const bool small = i8_small_ok(a);
+    if (small && a.Q <= kI8SmallQueries) return launch_i8_small(ctx, a, filter);
     const bool vec = i8_vec(a);
     if (filter && resq16_ok(a, vec)) return launch_i8_resq16(ctx, a);
     if (filter && resq_ok(a, vec)) return launch_i8_resq(ctx, a);
@@ -1263,10 +1250,11 @@ va_status launch_i8(va_context* ctx, const I8Args& a, bool filter) {
 #endif
     // The DMA pipeline needs whole 16-byte chunks, dense query rows (no indirection) and
     // descriptor offsets below 2^31.
-    const bool dma_ok = VA_I8_DMA && vec && !a.qrow && a.Q > 192 && a.D <= 131071 &&
+    const bool dma_ok = VA_I8_DMA && vec && !a.qrow && a.Q > kI8SmallQueries && a.D <= 131071 &&
                         uint64_t(a.Q - 1) * uint64_t(a.ldq) + a.D <= kDmaMaxBytes &&
                         uint64_t(dmai8::TN - 1) * uint64_t(a.ldx) + a.D <= kDmaMaxBytes;
     if (dma_ok) return filter ? launch_i8_dma<true>(ctx, a) : launch_i8_dma<false>(ctx, a);
+    if (small) return launch_i8_small(ctx, a, filter);  // (rows that are not whole 16-byte chunks)
     if (a.Q <= 32) return launch_i8_shape<1, 1, 4>(ctx, a, vec, filter);
     if (a.Q <= 64) return launch_i8_shape<1, 2, 2>(ctx, a, vec, filter);
 // Large-Q shape: 0 = 128 x 128 (4 waves), 1 = 128 x 256 (4 waves), 2 = 256 x 256 (8 waves).
