@@ -159,7 +159,7 @@ struct F32Producer final : KeyProducer {
 // fixed scratch block too small for the device fallback.
 va_status flat_topk(va_context* ctx, DistOp op, const float* q, const float* x, uint32_t Q, uint32_t N, uint32_t D,
                     uint32_t k, uint32_t* out_idx, float* out_dist, const _Float16* shadow, const float* norms,
-                    const uint8_t* skip, const float* errs) {
+                    const uint8_t* skip, const float* errs, const uint32_t* map) {
     F32Producer p;
     p.ctx = ctx;
     p.q = q;
@@ -173,6 +173,7 @@ va_status flat_topk(va_context* ctx, DistOp op, const float* q, const float* x, 
     o.f = out_dist;
     o.key_kind = 0;
     o.skip = skip;
+    o.map = map;
     ScreenInput si;
     si.q = q;
     si.x = x;
@@ -183,6 +184,7 @@ va_status flat_topk(va_context* ctx, DistOp op, const float* q, const float* x, 
     si.xh = shadow;
     si.xn = norms;
     si.xe = shadow ? errs : nullptr;
+    si.masked = skip != nullptr;
     if (screen_applies(ctx, si, k)) return screened_topk_scan(ctx, si, p, k, o);
     return exact_topk_scan(ctx, p, Q, N, k, o);
 }

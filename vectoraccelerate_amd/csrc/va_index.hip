@@ -65,14 +65,6 @@ __global__ void fill_byte_kernel(uint8_t* dst, uint64_t n, uint8_t v) {
     for (uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += uint64_t(gridDim.x) * 256) dst[i] = v;
 }
 
-// results: slot ids -> stable ids (sentinels stay)
-__global__ void slots_to_handles_kernel(uint32_t* idx, uint64_t n, const uint32_t* __restrict__ slot_stable) {
-    for (uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += uint64_t(gridDim.x) * 256) {
-        const uint32_t s = idx[i];
-        if (s != kSentinel) idx[i] = slot_stable[s];
-    }
-}
-
 // compaction: row keep[j] -> slot j of the new arrays (one workgroup per kept row)
 __global__ void gather_rows_kernel(const float* __restrict__ rows, const _Float16* __restrict__ shadow,
                                    const float* __restrict__ norms, const float* __restrict__ errs,
@@ -484,16 +476,13 @@ va_status va_index_search(va_context* ctx, const va_index* index, va_metric metr
         // nearest lists, deleted slots excluded inside the scan (no over-fetch)
         VA_REQUIRE(ctx, metric == VA_METRIC_L2SQ, "an IVF index searches by L2^2 only (metric %d)", int(metric));
         VA_CHECK_STATUS(va::ivf_search_masked(ctx, index->ivf, queries, num_queries, index->nprobe, k, out_handles,
-                                              out_dist, index->deleted ? index->skip : nullptr));
+                                              out_dist, index->deleted ? index->skip : nullptr, index->slot_stable));
     } else {
         VA_CHECK_STATUS(va::flat_topk(ctx, va::metric_op(metric), queries, index->rows, num_queries, index->slots,
                                       index->dim, k, out_handles, out_dist, index->pitch ? index->shadow : nullptr,
                                       index->pitch ? index->norms : nullptr, index->deleted ? index->skip : nullptr,
-                                      index->pitch ? index->errs : nullptr));
+                                      index->pitch ? index->errs : nullptr, index->slot_stable));
     }
-    va::slots_to_handles_kernel<<<dim3(va::grid_for(total)), dim3(256), 0, ctx->stream>>>(out_handles, total,
-                                                                                         index->slot_stable);
-    VA_CHECK_LAUNCH(ctx);
     return VA_OK;
 }
 

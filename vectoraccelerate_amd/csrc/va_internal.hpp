@@ -11,6 +11,7 @@
 #include "../../include/va_hip.h"
 #include "va_keys.hpp"
 #include "va_plan.hpp"
+#include "va_screen_bound.hpp"
 
 // ---------------------------------------------------------------------------
 // context
@@ -465,9 +466,15 @@ struct SelectArgs {
     uint32_t k = 0;
     uint32_t id_offset = 0;        // added to output ids
     const uint32_t* row_map = nullptr;  // output row for each input row (nullptr: identity)
+    // threshold mode: also the pre-test constants of the fp16 screen, ptc[row] = {A, B, C, 2^-scale}
+    // of the row's query (qinfo) and threshold (nullptr: not written)
+    float4* ptc = nullptr;
+    const float4* qinfo = nullptr;
+    ScreenBound bound{};
     // outputs (row stride out_ld, default k)
     int64_t out_ld = 0;
     uint32_t* out_idx = nullptr;   // [rows x k]
+    const uint32_t* out_map = nullptr;  // ids are written as out_map[id] (nullptr: the id)
     uint32_t* out_key = nullptr;   // [rows x k] keys (optional)
     float* out_f = nullptr;        // [rows x k] float values (optional)
     int32_t* out_i32 = nullptr;    // [rows x k] int32 values (optional)
@@ -549,6 +556,8 @@ struct ScanOutputs {
     // rows excluded from the search (skip[row] != 0; the deleted rows of an index), or nullptr:
     // their keys become kAbsentKey before every selection
     const uint8_t* skip = nullptr;
+    // ids are written as map[id] (an index's handles), or nullptr
+    const uint32_t* map = nullptr;
 };
 
 // keys[r * ld + j] = kAbsentKey for the rows + j * stride (j < cols) that skip excludes
@@ -569,9 +578,10 @@ va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t
 // va_ivf_search.
 va_status ivf_scan_masked(va_context* ctx, const va_ivf* ivf, const float* queries, uint32_t num_queries,
                           const uint32_t* probes, uint32_t nprobe, uint32_t k, uint32_t* out_idx, float* out_dist,
-                          const uint8_t* skip);
+                          const uint8_t* skip, const uint32_t* map = nullptr);
 va_status ivf_search_masked(va_context* ctx, const va_ivf* ivf, const float* queries, uint32_t num_queries,
-                            uint32_t nprobe, uint32_t k, uint32_t* out_idx, float* out_dist, const uint8_t* skip);
+                            uint32_t nprobe, uint32_t k, uint32_t* out_idx, float* out_dist, const uint8_t* skip,
+                            const uint32_t* map = nullptr);
 uint32_t ivf_num_lists(const va_ivf* ivf);
 
 // Plan of the sampled scan: S sample rows (every stride-th row), candidate capacity per query,
@@ -653,12 +663,15 @@ struct ScreenInput {
     // optional with the shadow: xe[j] >= |fp16(x_j) - x_j| (build_shadow's errs); the candidates'
     // intervals then use the measured rounding errors (narrower than the worst case)
     const float* xe = nullptr;
+    bool masked = false;  // rows are excluded: the sample's threshold is its k-th bound
 };
 // Exact top-k of device queries against a device database (va_fused_topk's body).  shadow /
-// norms: an fp16 shadow of x (see build_shadow) or nullptr; skip: rows excluded, or nullptr.
+// norms: an fp16 shadow of x (see build_shadow) or nullptr; skip: rows excluded, or nullptr; map: the
+// ids written for the rows, or nullptr.
 va_status flat_topk(va_context* ctx, DistOp op, const float* q, const float* x, uint32_t Q, uint32_t N, uint32_t D,
                     uint32_t k, uint32_t* out_idx, float* out_dist, const _Float16* shadow = nullptr,
-                    const float* norms = nullptr, const uint8_t* skip = nullptr, const float* errs = nullptr);
+                    const float* norms = nullptr, const uint8_t* skip = nullptr, const float* errs = nullptr,
+                    const uint32_t* map = nullptr);
 // Halves per row of an fp16 shadow (D rounded up to a multiple of 64).
 uint32_t shadow_pitch(uint32_t D);
 // shadow[r * shadow_pitch(D) + d] = fp16(x[r * D + d]) (RNE, zeros past D), norms[r] = |x_r|^2
@@ -668,8 +681,7 @@ uint32_t shadow_pitch(uint32_t D);
 va_status build_shadow(va_context* ctx, const float* x, uint32_t N, uint32_t D, _Float16* shadow, float* norms,
                        float2* norm_err = nullptr, float* errs = nullptr);
 // Pieces of the screened scan shared with the IVF list scan (va_screen.hip).  The bound itself
-// is va_screen_bound.hpp's.
-struct ScreenBound;
+// is va_screen_bound.hpp's, the rerank lists va_band.hpp's.
 // qh[q * shadow_pitch(D) + d] = fp16(q[q * D + d] * 2^sc_q) (the query's scale puts its largest
 // entry in [2^14, 2^15)), qinfo[q] = {|q|^2, |q|, 2^-sc_q, c0 * 2^-25 * 2^-sc_q}; qerr (may be
 // nullptr): an upper bound of the norm of the (unscaled) rounding error of each query's fp16 image.
@@ -677,16 +689,6 @@ struct ScreenBound;
 va_status screen_prepare_queries(va_context* ctx, const float* q, uint32_t Q, uint32_t D, _Float16* qh,
                                  float4* qinfo, float c0, float* qerr = nullptr, uint32_t* zero0 = nullptr,
                                  uint32_t n0 = 0, uint32_t* zero1 = nullptr, uint32_t n1 = 0);
-// Candidate lists of screened pairs, in place: (unscaled fp16 dot, |x|^2) -> (key of the upper
-// bound, key of the lower bound) of the pair's fp32 key, for i < min(cnt[q], cap).
-va_status screen_list_bounds(va_context* ctx, const ScreenBound& b, const float4* qinfo, float* dot, float* xx,
-                             const uint32_t* cnt, uint32_t cap, uint32_t Q);
-// Rerank lists: rr[q * rcap ..] = the cand_id of the candidates with lower bound <= bound[q];
-// queries whose candidates overflowed (cnt > cap) or whose list outgrows rcap get rcount 0 and
-// are appended to ovf_rows (ovf_cnt[0] counts them; ovf_cnt[1] receives the longest list).
-va_status screen_compact(va_context* ctx, const uint32_t* cnt, const uint32_t* cand_lo, const uint32_t* cand_id,
-                         const uint32_t* bound, uint32_t cap, uint32_t Q, uint32_t* rr, uint32_t* rcount, uint32_t rcap,
-                         uint32_t* ovf_cnt, uint32_t* ovf_rows);
 // Whether the screened path applies (metric, alignment, sizes, VA_OPT_SCREEN).
 bool screen_applies(const va_context* ctx, const ScreenInput& in, uint32_t k);
 va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer& exact, uint32_t k,

@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "va_band.hpp"
 #include "va_fallback.hpp"
 #include "va_internal.hpp"
 #include "va_screen_bound.hpp"
@@ -355,7 +356,7 @@ __global__ __launch_bounds__(256) void ivf_small_kernel(DistArgs a) {
 // loads: a narrow lane loads 32 and a wide lane 64 contiguous bytes of its row or query, and
 // the two lanes that meet in an MFMA hold the same k indices.  The pre-test's constants come
 // from the query's threshold; the appended (dot, |x|^2, position) triples become intervals in
-// screen_list_bounds.
+// ivf_band_kernel.
 namespace iv16 {
 constexpr uint32_t TN = 128, WAVES = 4;
 constexpr int kGroupsUsed = 3;  // narrow, wide<1>, wide<2>
@@ -551,30 +552,26 @@ __device__ __forceinline__ void wide_tile(const Ivf16Args& a, float2* xs, uint32
     }
 }
 
-// Candidate lists of the screened scan, in place: (unscaled fp16 dot, position) -> the key of the
-// pair's upper bound (over the dot) and of its lower bound (into lo), for i < min(cnt[q], cap).
-// Pairs that cannot be bounded get [0, the NaN key].
-__global__ __launch_bounds__(256) void ivf_bound_kernel(BoundV b, const float4* __restrict__ qinfo,
-                                                        const float* __restrict__ qerr, const float2* __restrict__ xn,
-                                                        float* __restrict__ dot, const uint32_t* __restrict__ pos,
-                                                        uint32_t* __restrict__ lo, const uint32_t* __restrict__ cnt,
-                                                        uint32_t cap) {
-    const uint32_t q = blockIdx.y;
+// Candidate lists of the screened scan, (unscaled fp16 dot, position): the pairs' intervals ([0, the
+// NaN key] for pairs that cannot be bounded), then the threshold of the sample or the rerank lists
+// (va_band.hpp).
+template <int NT>
+__global__ __launch_bounds__(NT) void ivf_band_kernel(BoundV bv, const float4* __restrict__ qinfo,
+                                                      const float* __restrict__ qerr, const float2* __restrict__ xn,
+                                                      BandArgs b) {
+    extern __shared__ uint32_t s_band[];
+    __shared__ BandLds lds;
+    const uint32_t q = blockIdx.x;
     const float4 inf = qinfo[q];
     const float eq = qerr[q];
-    const uint32_t m = min(cnt[q], cap);
-    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < m; i += gridDim.x * 256) {
-        const int64_t o = int64_t(q) * cap + i;
-        const float2 n = xn[pos[o]];
+    const float* dot = reinterpret_cast<const float*>(b.hi);
+    band_row<NT>(b, q, lds, s_band, [&](int64_t o, uint32_t& klo, uint32_t& khi) {
+        const float2 n = xn[b.id[o]];
         float l, h;
-        uint32_t klo = 0u, khi = 0xFFFFFFFEu;
-        if (screen_bounds_v(b, dot[o], inf.x, inf.y, eq, n.x, sqrtf(n.x), n.y, l, h)) {
-            klo = key_of_float(l);
-            khi = key_of_float(h);
-        }
-        reinterpret_cast<uint32_t*>(dot)[o] = khi;
-        lo[o] = klo;
-    }
+        const bool ok = screen_bounds_v(bv, dot[o], inf.x, inf.y, eq, n.x, sqrtf(n.x), n.y, l, h);
+        klo = ok ? key_of_float(l) : 0u;
+        khi = ok ? key_of_float(h) : 0xFFFFFFFEu;  // the NaN key
+    });
 }
 
 // The 16-query tiles, one independent tile per wave, software-pipelined across the wave's tiles:
@@ -1921,7 +1918,7 @@ bool ivf_screen_applies(const va_context* ctx, const va_ivf* ivf, const float* q
 //   select  : exact (key, id) top-k.  Overflowed queries take the device fallback.
 va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* queries, uint32_t Q,
                             const uint32_t* probes, uint32_t np, uint32_t k, uint32_t* out_idx, float* out_dist,
-                            const uint8_t* skip) {
+                            const uint8_t* skip, const uint32_t* map) {
     const uint32_t C = ivf->C, D = ivf->D, Dp = shadow_pitch(D);
     const uint32_t npc = std::min(np, C);
     const uint64_t cap_s = std::max<uint64_t>(1, ivf->top_sample[npc]);
@@ -1951,7 +1948,6 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     // list counts: [0, Q) the sample pass's, [Q, 2Q) the full pass's (both cleared by the prep)
     uint32_t* const cnt2 = s.carve<uint32_t>(uint64_t(Q) * 2);
     uint32_t* cnt = cnt2;
-    uint32_t* ubound = s.carve<uint32_t>(Q);
     uint32_t* rcount = s.carve<uint32_t>(Q);
     uint32_t* ovf_rows = s.carve<uint32_t>(Q);
     uint32_t* ovf_cnt = s.carve<uint32_t>(va::kZeroWords);
@@ -1996,14 +1992,31 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     float4* gpt = dp.big_tq ? s.carve<float4>(pairs) : nullptr;
     float2* gqv = dp.big_tq ? s.carve<float2>(pairs) : nullptr;
     VA_CHECK_STATUS(s.verify(need));
-    uint32_t* chi = reinterpret_cast<uint32_t*>(cdot);
-    auto bounds = [&](uint64_t cp) -> va_status {
-        const uint32_t bx = uint32_t(std::min<uint64_t>(4, (cp + 255) / 256));
-        ivf_bound_kernel<<<dim3(bx, Q), dim3(256), 0, ctx->stream>>>(make_bound_v(D), qinfo, qerr, ivf->norms, cdot,
-                                                                     cpos, clo, cnt, uint32_t(cp));
+    // intervals, k-th upper bound and rerank lists (excluded rows, an index's deletions, never count)
+    BandArgs band;
+    band.hi = reinterpret_cast<uint32_t*>(cdot);
+    band.lo = clo;
+    band.id = cpos;
+    band.k = k;
+    band.skip = skip;
+    band.skip_id = ivf->ids;
+    auto launch_band = [&](uint64_t cp) -> va_status {
+        band.cnt = cnt;
+        band.cap = uint32_t(cp);
+        const bool tall = band_tall(ctx, Q);
+        band.list = band_list(tall, band.cap);
+        const size_t lds = size_t(band.list) * 8;
+        if (tall) {
+            VA_CHECK_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(&ivf_band_kernel<1024>),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+            ivf_band_kernel<1024><<<dim3(Q), dim3(1024), lds, ctx->stream>>>(make_bound_v(D), qinfo, qerr, ivf->norms,
+                                                                            band);
+        } else {
+            ivf_band_kernel<512><<<dim3(Q), dim3(512), lds, ctx->stream>>>(make_bound_v(D), qinfo, qerr, ivf->norms,
+                                                                          band);
+        }
         VA_CHECK_LAUNCH(ctx);
-        // excluded rows (an index's deletions) become absent keys before every selection
-        return mask_list_keys(ctx, chi, clo, cpos, cnt, Q, uint32_t(cp), int64_t(cp), skip, ivf->ids);
+        return VA_OK;
     };
 
     ScanPhaseMarks pm(ctx);
@@ -2029,20 +2042,10 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     VA_CHECK_STATUS(fill_u32(ctx, thr, Q, 0xFFFFFFFFu));
     a.cap = uint32_t(cap_s);
     VA_CHECK_STATUS(run_screen_pass(ctx, dp, 0, a));
-    VA_CHECK_STATUS(bounds(cap_s));
-    {
-        SelectArgs sel;
-        sel.keys = chi;
-        sel.ids = cpos;
-        sel.counts = cnt;
-        sel.ld = int64_t(cap_s);
-        sel.n = uint32_t(cap_s);
-        sel.rows = Q;
-        sel.k = k;
-        sel.out_kth = thr;
-        VA_CHECK_STATUS(launch_select(ctx, sel));
-    }
-    // ---- 2. screen, 3. U_q (overflowed queries are listed) ---------------------------------------
+    band.out_kth = thr;
+    VA_CHECK_STATUS(launch_band(cap_s));
+    band.out_kth = nullptr;
+    // ---- 2. screen, 3. U_q and the rerank lists (overflowed queries are listed) ---------------------------------------
     cnt = cnt2 + Q;
     a.cnt = cnt;
     a.cap = uint32_t(cap);
@@ -2058,24 +2061,13 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     VA_CHECK_STATUS(pm.mark(1));
     VA_CHECK_STATUS(run_screen_pass(ctx, dp, 1, a));
     VA_CHECK_STATUS(pm.mark(2));
-    VA_CHECK_STATUS(bounds(cap));
-    {
-        SelectArgs sel;
-        sel.keys = chi;
-        sel.ids = cpos;
-        sel.counts = cnt;
-        sel.ld = int64_t(cap);
-        sel.n = uint32_t(cap);
-        sel.rows = Q;
-        sel.k = k;
-        sel.out_kth = ubound;
-        sel.overflow_count = ovf_cnt;
-        sel.overflow_rows = ovf_rows;
-        VA_CHECK_STATUS(launch_select(ctx, sel));
-    }
-    // ---- 4. rerank lists, 5. exact keys ----------------------------------------------------------
-    VA_CHECK_STATUS(screen_compact(ctx, cnt, clo, cpos, ubound, uint32_t(cap), Q, rr, rcount, uint32_t(rcap), ovf_cnt,
-                                   ovf_rows));
+    band.rr = rr;
+    band.rcount = rcount;
+    band.rcap = uint32_t(rcap);
+    band.ovf_cnt = ovf_cnt;
+    band.ovf_rows = ovf_rows;
+    VA_CHECK_STATUS(launch_band(cap));
+    // ---- 4. exact keys ---------------------------------------------------------------------------
     {
         const uint64_t items = uint64_t(Q) * ((rcap + 63) / 64);
         const uint32_t blocks = uint32_t(std::min<uint64_t>(2048, (items + 3) / 4));
@@ -2083,12 +2075,12 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
                                                                        ivf->offsets, C, dp.qcnt, D, rr, rcount,
                                                                        uint32_t(rcap), Q, rkey, rid);
         VA_CHECK_LAUNCH(ctx);
-        VA_CHECK_STATUS(mask_list_keys(ctx, rkey, nullptr, rid, rcount, Q, uint32_t(rcap), int64_t(rcap), skip));
     }
-    // ---- 6. exact (key, id) top-k, 7. overflowed queries -----------------------------------------
+    // ---- 5. exact (key, id) top-k, 6. overflowed queries -----------------------------------------
     SelectArgs base;
     base.k = k;
     base.out_idx = out_idx;
+    base.out_map = map;
     base.out_f = out_dist;
     {
         SelectArgs sel = base;
@@ -2106,8 +2098,7 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     VA_CHECK_STATUS(pm.count_sum(rcount, Q));
     VA_CHECK_STATUS(pm.count_overflow(ovf_cnt));
     VA_CHECK_STATUS(pm.mark(3));
-    // ---- 7. exact top-k of the overflowed queries (listed by the U_q selection and the
-    // compaction), over the rows the selection wrote
+    // ---- 6. exact top-k of the overflowed queries (listed with U_q), over the rows the selection wrote
     VA_CHECK_STATUS(ivf_fallback(ctx, ivf, queries, dp, np, fb, base));
     return pm.finish(true, true);
 }
@@ -2304,7 +2295,7 @@ namespace va {
 // a place in a result or hold a threshold down (nullptr: none excluded).
 va_status ivf_scan_masked(va_context* ctx, const va_ivf* ivf, const float* queries, uint32_t num_queries,
                           const uint32_t* probes, uint32_t nprobe, uint32_t k, uint32_t* out_idx, float* out_dist,
-                          const uint8_t* skip) {
+                          const uint8_t* skip, const uint32_t* map) {
     using va::Scratch;
     if (!ctx) return VA_ERR_INVALID_ARG;
     VA_REQUIRE(ctx, ivf && queries && probes && out_idx, "va_ivf_scan: NULL pointer");
@@ -2313,7 +2304,8 @@ va_status ivf_scan_masked(va_context* ctx, const va_ivf* ivf, const float* queri
     VA_REQUIRE(ctx, nprobe >= 1, "nprobe must be at least 1, got %u", nprobe);
     va::DeviceGuard g(ctx->device);
     if (va::ivf_screen_applies(ctx, ivf, queries))
-        return va::ivf_scan_screened(ctx, ivf, queries, num_queries, probes, nprobe, k, out_idx, out_dist, skip);
+        return va::ivf_scan_screened(ctx, ivf, queries, num_queries, probes, nprobe, k, out_idx, out_dist, skip,
+                                     map);
     const uint32_t Q = num_queries, C = ivf->C, np = nprobe;
 
     // ---- sizes from the list lengths alone (nothing is read back) --------------------------------
@@ -2394,6 +2386,7 @@ va_status ivf_scan_masked(va_context* ctx, const va_ivf* ivf, const float* queri
     va::SelectArgs base;
     base.k = k;
     base.out_idx = out_idx;
+    base.out_map = map;
     base.out_f = out_dist;
     {
         va::SelectArgs a = base;
@@ -2418,7 +2411,8 @@ va_status ivf_scan_masked(va_context* ctx, const va_ivf* ivf, const float* queri
 
 // va_ivf_search with an exclusion mask (see ivf_scan_masked)
 va_status ivf_search_masked(va_context* ctx, const va_ivf* ivf, const float* queries, uint32_t num_queries,
-                            uint32_t nprobe, uint32_t k, uint32_t* out_idx, float* out_dist, const uint8_t* skip) {
+                            uint32_t nprobe, uint32_t k, uint32_t* out_idx, float* out_dist, const uint8_t* skip,
+                            const uint32_t* map) {
     if (!ctx) return VA_ERR_INVALID_ARG;
     VA_REQUIRE(ctx, ivf && queries && out_idx, "va_ivf_search: NULL pointer");
     VA_REQUIRE(ctx, num_queries > 0, "Queries cannot be empty");
@@ -2438,7 +2432,7 @@ va_status ivf_search_masked(va_context* ctx, const va_ivf* ivf, const float* que
         m->probe_cap = need;
     }
     VA_CHECK_STATUS(va_ivf_probe(ctx, ivf, queries, num_queries, nprobe, m->probe_buf));
-    return ivf_scan_masked(ctx, ivf, queries, num_queries, m->probe_buf, nprobe, k, out_idx, out_dist, skip);
+    return ivf_scan_masked(ctx, ivf, queries, num_queries, m->probe_buf, nprobe, k, out_idx, out_dist, skip, map);
 }
 
 uint32_t ivf_num_lists(const va_ivf* ivf) { return ivf->C; }

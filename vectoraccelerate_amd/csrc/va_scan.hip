@@ -190,6 +190,7 @@ va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t
     SelectArgs base;
     base.k = k;
     base.out_idx = out.idx;
+    base.out_map = out.map;
     base.out_f = out.f;
     base.out_i32 = out.i32;
     base.out_key = out.key;

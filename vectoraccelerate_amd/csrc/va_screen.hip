@@ -40,6 +40,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "va_band.hpp"
 #include "va_fallback.hpp"
 #include "va_internal.hpp"
 #include "va_screen_bound.hpp"
@@ -66,8 +67,8 @@ constexpr int PF_AHEAD = 3;               // stages between a row prefetch and t
 constexpr int DP_ALIGN = KC;              // fp16 query rows are padded to a multiple of KC
 }  // namespace scr
 
-// SCREEN_GMIN: per query, the smallest approximate upper bound of each 32-row group (the sample of
-// a search whose threshold is checked afterwards, where any threshold is safe)
+// SCREEN_GMIN: per query, the smallest (approximate) upper bound of each group of rows (the sample
+// of a search whose threshold is checked afterwards, where any threshold is safe)
 enum ScreenMode : int { SCREEN_KEYS = 0, SCREEN_FILTER = 1, SCREEN_GMIN = 2 };
 // below this many queries a search over the fp16 shadow takes screen16_small_kernel (a 256-query
 // tile of screen16_kernel would be mostly padding)
@@ -87,7 +88,8 @@ struct ScreenArgs {
     float c1 = 0, cn = 0, c0x = 0, kabs = 0;  // bound coefficients (see screen_bounds)
     // SCREEN_KEYS: out_dot[q * ldo + j] = fp16 dot of query q and row j; out_xx[j] = |x_j|^2
     // SCREEN_GMIN: out_dot[q * ldo + g] (as keys) = smallest approximate upper bound of the rows
-    // 32g .. 32g + 31 (ldo = 8 x the row tiles; groups past N hold the key of +inf)
+    // 32g .. 32g + 31 (ldo = 8 x the row tiles; groups past N hold the key of +inf).
+    // screen16_small_kernel: groups of 4 MB rows, four per wave tile, exact upper bounds
     float* out_dot = nullptr;
     float* out_xx = nullptr;
     int64_t ldo = 0;
@@ -104,7 +106,9 @@ struct ScreenArgs {
     const float* xn = nullptr;
     // screen16_small_kernel: row j of the scan is shadow row j * xstride (the threshold sample)
     uint32_t xstride = 1;
-    // screen16_kernel: the pre-test constants of each query, {A, B, C, 2^-scale} (pretest_kernel)
+    // screen16_kernel: the pre-test constants of each query, {A, B, C, 2^-scale},
+    // written once per search with its threshold (per tile they cost each wave a division and the
+    // op's branch per query block)
     const float4* ptc = nullptr;
     // the candidates' intervals with measured rounding errors (screen_bounds_m) when both are
     // set: qerr[q] >= |fp16 image of q - q| (unscaled), xe[id] >= |fp16(x_id) - x_id|
@@ -124,17 +128,6 @@ __device__ __forceinline__ void screen_keys(const ScreenArgs& a, float dot, floa
 }
 __device__ __forceinline__ PreTest pretest_consts(const ScreenArgs& a, float4 info, uint32_t thr_key) {
     return pretest_consts(bound_of(a), info.x, info.y, info.z, info.w, thr_key);
-}
-
-// The pre-test constants of every query, once per search (they depend on the query and its
-// threshold only; computing them per tile cost each wave a division and the op's branch per
-// query block): ptc[q] = {A, B, C, 2^-scale}.
-__global__ __launch_bounds__(256) void pretest_kernel(ScreenArgs a, uint32_t Q, float4* __restrict__ ptc) {
-    const uint32_t q = blockIdx.x * 256 + threadIdx.x;
-    if (q >= Q) return;
-    const float4 inf = a.qinfo[q];
-    const PreTest p = pretest_consts(a, inf, a.thr[q]);
-    ptc[q] = float4{p.A, p.B, p.C, inf.z};
 }
 
 // ---- query preparation: one wave per query ------------------------------------------------
@@ -1130,6 +1123,13 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void screen16_kernel(Screen
 // screen16_kernel on each value (flagged rows always pass) and appends from registers.
 template <int MODE, int NQB, int MB, int L, int R>
 __global__ __launch_bounds__(256, 2) void screen16_small_kernel(ScreenArgs a) {
+    if constexpr (MODE == SCREEN_GMIN) {  // blocks of 16 NQB queries along the grid
+        const uint32_t q0 = blockIdx.y * uint32_t(16 * NQB);
+        a.qh += int64_t(q0) * a.Dp;
+        a.qinfo += q0;
+        a.out_dot += int64_t(q0) * a.ldo;
+        a.Q = min(uint32_t(16 * NQB), a.Q - q0);
+    }
     constexpr int TNW = 16 * MB;       // rows per wave tile
     constexpr uint32_t CH = 64u * L;   // bytes per chunk of a row
     const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
@@ -1220,6 +1220,29 @@ __global__ __launch_bounds__(256, 2) void screen16_small_kernel(ScreenArgs a) {
             }
             continue;
         }
+        if constexpr (MODE == SCREEN_GMIN) {
+            // the smallest upper bound of the lane's 4 MB rows per query (absent past the end)
+#pragma unroll
+            for (int n = 0; n < NQB; ++n) {
+                const uint32_t qt = uint32_t(16 * n + r16);
+                if (qt >= a.Q) continue;
+                const float4 inf = a.qinfo[qt];
+                uint32_t best = kAbsentKey;
+#pragma unroll
+                for (int m = 0; m < MB; ++m)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const uint32_t row = uint32_t(16 * m + 4 * g + v);
+                        if (row >= rc) continue;
+                        const float xx = a.xn[uint64_t(rs + row) * a.xstride];
+                        uint32_t klo, khi;
+                        screen_keys(a, acc[m][n][v] * inf.z, inf.x, inf.y, xx, sqrtf(xx), inf.w, klo, khi);
+                        best = min(best, khi);
+                    }
+                reinterpret_cast<uint32_t*>(a.out_dot)[int64_t(qt) * a.ldo + 4u * tile + uint32_t(g)] = best;
+            }
+            continue;
+        }
         // ---- filter epilogue: the row norms one block at a time, a pass mask per query block;
         // the appends re-read the norms of passing rows
         uint32_t mk[NQB];
@@ -1250,8 +1273,15 @@ __global__ __launch_bounds__(256, 2) void screen16_small_kernel(ScreenArgs a) {
             const uint32_t qt = uint32_t(16 * n + r16);
             const uint32_t mq = qt < a.Q ? mk[n] : 0u;
             if (!__ballot(mq != 0u)) continue;
+            // one atomic for the four lanes of a query: their places in lane order
+            const uint32_t c = uint32_t(__popc(mq));
+            const uint32_t c16 = uint32_t(__shfl_xor(int(c), 16)), pair = c + c16;
+            const uint32_t other = uint32_t(__shfl_xor(int(pair), 32));
+            uint32_t base = 0;
+            if (g == 0 && pair + other) base = atomicAdd(a.cnt + qt, pair + other);
+            base = uint32_t(__shfl(int(base), r16));
             if (!mq) continue;
-            uint32_t pos = atomicAdd(a.cnt + qt, uint32_t(__popc(mq)));
+            uint32_t pos = base + (g & 1 ? c16 : 0u) + (g & 2 ? other : 0u);
 #pragma unroll
             for (int m = 0; m < MB; ++m)
 #pragma unroll
@@ -1316,102 +1346,47 @@ __global__ __launch_bounds__(256) void shadow_kernel(const float* __restrict__ x
 }
 
 // ---- exact intervals of the screened pairs -----------------------------------------------------
-// Dense (the sample): keys[q * ld + j] = key(hi) from dot[q * ld + j] and xx[j], in place.
-// Lists (the scan's candidates): (dot, xx) -> (key(hi), key(lo)), in place, for i < min(cnt, cap).
-__global__ __launch_bounds__(256) void screen_bound_kernel(ScreenArgs a, float* dot, const float* xx_dense, float* xx_list,
-                                                           const uint32_t* cnt, uint32_t n, int64_t ld) {
+// Dense (a sample whose threshold is not checked): keys[q * ld + j] = key(hi) from dot[q * ld + j]
+// and xx[j], in place.
+__global__ __launch_bounds__(256) void screen_bound_kernel(ScreenArgs a, float* dot, const float* xx, uint32_t n,
+                                                           int64_t ld) {
     const uint32_t q = blockIdx.y;
     const float4 info = a.qinfo[q];
-    const uint32_t m = cnt ? min(cnt[q], n) : n;
-    // lists with the measured rounding errors: narrower intervals than the worst case the scan's
-    // pre-test used (the list holds a superset of what they would admit)
-    const bool measured = cnt && a.xe && a.qerr;
-    const BoundV bv{a.vcn, a.vgd, a.vg2d};
-    const float eq = measured ? a.qerr[q] : 0.0f;
-    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < m; i += gridDim.x * 256) {
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
         const int64_t o = int64_t(q) * ld + i;
-        const float xx = cnt ? xx_list[o] : xx_dense[i];
         uint32_t klo, khi;
-        if (measured) {
-            float lo, hi;
-            if (screen_bounds_m(bv, a.op, dot[o], info.x, info.y, eq, xx, sqrtf(xx), a.xe[a.cand_id[o]], lo, hi)) {
-                klo = key_of_float(lo);
-                khi = key_of_float(hi);
-            } else {
-                klo = 0u;
-                khi = 0xFFFFFFFEu;  // the NaN key
-            }
-        } else {
-            screen_keys(a, dot[o], info.x, info.y, xx, sqrtf(xx), info.w, klo, khi);
-        }
+        screen_keys(a, dot[o], info.x, info.y, xx[i], sqrtf(xx[i]), info.w, klo, khi);
         reinterpret_cast<uint32_t*>(dot)[o] = khi;
-        if (cnt) reinterpret_cast<uint32_t*>(xx_list)[o] = klo;
     }
 }
-
-// ---- rerank list: the candidates whose lower bound is within the k-th upper bound -------------
-// One workgroup per query.  Lists that overflowed (count > cap), fell short of min_count (both
-// listed by the candidate select), whose k-th upper bound exceeds the threshold they were
-// filtered with (thr non-null: a threshold below the sample's k-th bound, which holds only when k
-// candidates lie within it) or whose rerank list outgrows rcap take the fallback and are left
-// empty here; the last two are listed here.
-__global__ __launch_bounds__(256) void screen_compact_kernel(const uint32_t* __restrict__ cnt,
-                                                             const uint32_t* __restrict__ cand_lo,
-                                                             const uint32_t* __restrict__ cand_id,
-                                                             const uint32_t* __restrict__ bound, uint32_t cap,
-                                                             uint32_t min_count, const uint32_t* __restrict__ thr,
-                                                             uint32_t* __restrict__ rr, uint32_t* __restrict__ rcount,
-                                                             uint32_t rcap, uint32_t* __restrict__ ovf_cnt,
-                                                             uint32_t* __restrict__ ovf_rows,
-                                                             uint32_t* __restrict__ max_count) {
-    __shared__ uint32_t s_n;
+// The candidates: intervals, k-th upper bound, rerank list (va_band.hpp).  With the measured
+// rounding errors the intervals are narrower than the worst case the scan's pre-test used (the list
+// holds a superset of what they would admit).  With the threshold and its pre-test constants in one
+// launch, and an index's handles written by the selections: 13 launches a search -> 8, 1M x 768, Q = 1
+// 339 -> 328 us; with the smaller sample, 256-row tiles and 8-row rerank chunks 100,000 x 768, Q = 100
+// 159 -> 130.
+template <int NT>
+__global__ __launch_bounds__(NT) void screen_band_kernel(ScreenArgs a, BandArgs b) {
+    extern __shared__ uint32_t s_band[];
+    __shared__ BandLds lds;
     const uint32_t q = blockIdx.x;
-    const int tid = threadIdx.x;
-    const uint32_t n = cnt[q];
-    if (n > cap || n < min_count) {
-        // the candidate select has already listed this query for the fallback
-        if (tid == 0) rcount[q] = 0;
-        return;
-    }
-    if (thr && bound[q] > thr[q]) {
-        // fewer than k candidates have an upper bound within the threshold: the list may miss
-        // a row of the top-k
-        if (tid == 0) {
-            rcount[q] = 0;
-            ovf_rows[atomicAdd(ovf_cnt, 1u)] = q;
-        }
-        return;
-    }
-    if (tid == 0) s_n = 0;
-    __syncthreads();
-    const uint32_t u = bound[q];
-    const uint32_t* lo = cand_lo + int64_t(q) * cap;
-    const uint32_t* id = cand_id + int64_t(q) * cap;
-    uint32_t* out = rr + int64_t(q) * rcap;
-    for (uint32_t i0 = 0; i0 < n; i0 += 256) {
-        const uint32_t i = i0 + uint32_t(tid);
-        const bool p = i < n && lo[i] <= u;
-        const uint64_t b = __ballot(p);
-        const int lane = tid & 63;
-        uint32_t base = 0;
-        if (lane == 0 && b) base = atomicAdd(&s_n, uint32_t(__popcll(b)));
-        base = __shfl(base, 0);
-        if (p) {
-            const uint32_t pos = base + uint32_t(__popcll(b & ((1ull << lane) - 1)));
-            if (pos < rcap) out[pos] = id[i];
-        }
-    }
-    __syncthreads();
-    if (tid == 0) {
-        const uint32_t m = s_n;
-        if (m > rcap) {
-            rcount[q] = 0;
-            const uint32_t p = atomicAdd(ovf_cnt, 1u);
-            ovf_rows[p] = q;
-        } else {
-            rcount[q] = m;
-            atomicMax(max_count, m);
-        }
+    const float4 info = a.qinfo[q];
+    if (a.xe && a.qerr) {
+        const BoundV bv{a.vcn, a.vgd, a.vg2d};
+        const float eq = a.qerr[q];
+        band_row<NT>(b, q, lds, s_band, [&](int64_t o, uint32_t& klo, uint32_t& khi) {
+            const float xx = a.cand_xx[o];
+            float lo, hi;
+            const bool ok = screen_bounds_m(bv, a.op, a.cand_dot[o], info.x, info.y, eq, xx, sqrtf(xx),
+                                            a.xe[a.cand_id[o]], lo, hi);
+            klo = ok ? key_of_float(lo) : 0u;
+            khi = ok ? key_of_float(hi) : 0xFFFFFFFEu;  // the NaN key
+        });
+    } else {
+        band_row<NT>(b, q, lds, s_band, [&](int64_t o, uint32_t& klo, uint32_t& khi) {
+            const float xx = a.cand_xx[o];
+            screen_keys(a, a.cand_dot[o], info.x, info.y, xx, sqrtf(xx), info.w, klo, khi);
+        });
     }
 }
 
@@ -1526,8 +1501,16 @@ va_status launch_screen16_gmin(va_context* ctx, const ScreenArgs& a) {
 }
 va_status launch_screen16(va_context* ctx, const ScreenArgs& a) {
     using namespace s16;
-    if (a.Q <= kHalfTileQueries)
+    if (a.Q <= kHalfTileQueries) {
+        // 384-row tiles of twelve waves, or 256-row tiles of eight (a tenth slower a row) where
+        // those need fewer rows' worth of rounds over the CUs (100,000 rows: 261 tiles of 384 on 256
+        // CUs are two rounds, and so are 391 of 256)
+        const uint64_t cus = std::max<uint64_t>(uint64_t(ctx->num_cus), kXcds) / kXcds * kXcds;
+        auto rounds = [&](uint64_t tn) { return ((a.N + tn - 1) / tn + cus - 1) / cus; };
+        if (rounds(256) * 282 < rounds(384) * 384)
+            return launch_screen16_shape<kWaves / 2, kQueryBlocks, kRowBlocks, int(kHalfTileQueries)>(ctx, a);
         return launch_screen16_shape<3 * kWaves / 4, kQueryBlocks, kRowBlocks, int(kHalfTileQueries)>(ctx, a);
+    }
     return launch_screen16_shape<kWaves, kQueryBlocks, kRowBlocks, TQ>(ctx, a);
 }
 
@@ -1569,12 +1552,37 @@ va_status launch_screen16_small(va_context* ctx, const ScreenArgs& a) {
     return fail(ctx, VA_ERR_INVALID_ARG, "launch_screen16_small: %u queries (at most %u)", a.Q, kSmallBatchMax);
 }
 
-va_status launch_bounds(va_context* ctx, const ScreenArgs& a, float* dot, const float* xx_dense, float* xx_list,
-                        const uint32_t* cnt, uint32_t n, int64_t ld, uint32_t rows) {
+// The threshold sample of a small or middling batch: group minima (groups of 4 MB rows) by
+// screen16_small_kernel, blocks of 16 or 32 queries along the grid.
+#define VA_GM_A 1, 1, 2, 8
+#define VA_GM_B 2, 2, 2, 4
+using GminA = Launch<VA_GM_A>;
+using GminB = Launch<VA_GM_B>;
+// It re-reads its queries for every wave tile, so past kSmallGminPairs pairs screen16_kernel's tiles
+// win (1M x 768: 128 queries against 15,625 rows 424 / 455 us a search, 256 queries 630 / 612).
+constexpr uint32_t kSmallGminMax = 256;
+constexpr uint64_t kSmallGminPairs = 2ull << 20;
+// (narrow: the 16-query tile, for searches of at most that many queries)
+uint32_t small_gmin_groups(bool narrow, uint64_t S) {
+    const uint32_t tn = narrow ? GminA::TNW : GminB::TNW;
+    return uint32_t((S + tn - 1) / tn) * 4u;
+}
+va_status launch_small_gmin(va_context* ctx, const ScreenArgs& a, bool narrow) {
+    if (a.Q == 0 || a.N == 0) return VA_OK;
+    const uint32_t tn = narrow ? GminA::TNW : GminB::TNW, tq = narrow ? GminA::queries : GminB::queries;
+    const uint32_t tiles = (a.N + tn - 1) / tn, nqb = (a.Q + tq - 1) / tq;
+    const dim3 grid(std::min<uint32_t>((tiles + 3) / 4, 2u * uint32_t(ctx->num_cus)), nqb);
+    if (narrow) screen16_small_kernel<SCREEN_GMIN, VA_GM_A><<<grid, dim3(256), 0, ctx->stream>>>(a);
+    else screen16_small_kernel<SCREEN_GMIN, VA_GM_B><<<grid, dim3(256), 0, ctx->stream>>>(a);
+    VA_CHECK_LAUNCH(ctx);
+    return VA_OK;
+}
+
+va_status launch_bounds(va_context* ctx, const ScreenArgs& a, float* dot, const float* xx, uint32_t n, int64_t ld,
+                        uint32_t rows) {
     if (rows == 0 || n == 0) return VA_OK;
-    // lists are short (a few thousand): one block per query row; the dense sample: up to 16
-    const uint32_t bx = cnt ? std::min<uint32_t>(4, (n + 255) / 256) : std::min<uint32_t>(16, (n + 255) / 256);
-    screen_bound_kernel<<<dim3(bx, rows), dim3(256), 0, ctx->stream>>>(a, dot, xx_dense, xx_list, cnt, n, ld);
+    screen_bound_kernel<<<dim3(std::min<uint32_t>(16, (n + 255) / 256), rows), dim3(256), 0, ctx->stream>>>(a, dot, xx, n,
+                                                                                                           ld);
     VA_CHECK_LAUNCH(ctx);
     return VA_OK;
 }
@@ -1613,35 +1621,19 @@ va_status screen_prepare_queries(va_context* ctx, const float* q, uint32_t Q, ui
     return VA_OK;
 }
 
-va_status screen_list_bounds(va_context* ctx, const ScreenBound& b, const float4* qinfo, float* dot, float* xx,
-                             const uint32_t* cnt, uint32_t cap, uint32_t Q) {
-    ScreenArgs a;
-    a.op = b.op;
-    a.c1 = b.c1;
-    a.cn = b.cn;
-    a.c0x = b.c0x;
-    a.kabs = b.kabs;
-    a.qinfo = qinfo;
-    return launch_bounds(ctx, a, dot, nullptr, xx, cnt, cap, int64_t(cap), Q);
-}
-
-va_status screen_compact(va_context* ctx, const uint32_t* cnt, const uint32_t* cand_lo, const uint32_t* cand_id,
-                         const uint32_t* bound, uint32_t cap, uint32_t Q, uint32_t* rr, uint32_t* rcount, uint32_t rcap,
-                         uint32_t* ovf_cnt, uint32_t* ovf_rows) {
-    screen_compact_kernel<<<dim3(Q), dim3(256), 0, ctx->stream>>>(cnt, cand_lo, cand_id, bound, cap, 0u, nullptr, rr,
-                                                                 rcount, rcap, ovf_cnt, ovf_rows, ovf_cnt + 1);
-    VA_CHECK_LAUNCH(ctx);
-    return VA_OK;
-}
-
-// The plan of a screened search: plan_scan's, except that small batches over the fp16 shadow
-// sample N/256 rows (at least 4096): for them the sample and its per-row selection are a visible
-// share of a search that streams the shadow once, while the screen's band, not the sample's
-// threshold, sets the rerank.
+// The plan of a screened search: plan_scan's, except that over the fp16 shadow small batches sample
+// N/256 rows and middling ones N/64 (both at least 4096): for them the sample and its per-row
+// selection are a visible share of the search, while the screen's band, not the sample's
+// threshold, sets the rerank.  (64 to 128 queries of 1M rows: N/256 lets through so many more
+// candidates that it is 2% slower than N/64; for 100,000 rows and 100 queries 4,096 rows instead
+// of 16,384 take the sample from 27 to 20 us.)  With excluded rows the threshold is the sample's k-th
+// bound itself, which lets through k N / S rows: long lists for N/256 (1M x 384, k = 10,
+// 1,000 deleted, Q = 32: 418 -> 310 us).
 ScanPlan screen_plan(const va_context* ctx, const ScreenInput& in, uint32_t k) {
-    if (in.xh && in.Q <= kSmallBatchMax && !ctx->opt_sample_rows)
-        return plan_scan_for(dense_budget(ctx), std::max<uint64_t>(4096, in.N / 256), ctx->opt_candidate_cap, in.Q,
-                             in.N, k);
+    const bool small = in.Q <= kSmallBatchMax, middling = in.Q <= kSmallGminMax && in.N > kMinSample;
+    if (in.xh && (small || middling) && !ctx->opt_sample_rows)
+        return plan_scan_for(dense_budget(ctx), std::max<uint64_t>(4096, in.N / (small && !in.masked ? 256 : 64)),
+                             ctx->opt_candidate_cap, in.Q, in.N, k);
     return plan_scan(ctx, in.Q, in.N, k);
 }
 
@@ -1666,6 +1658,7 @@ bool screen_applies(const va_context* ctx, const ScreenInput& in, uint32_t k) {
     return in.xh ? true : in.Q >= kSmallBatch;
 }
 
+constexpr uint32_t kRerankSmall = 128;
 va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer& exact, uint32_t k,
                              const ScanOutputs& out) {
     const uint32_t Q = in.Q, N = in.N, D = in.D;
@@ -1684,6 +1677,7 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
     SelectArgs base;
     base.k = k;
     base.out_idx = out.idx;
+    base.out_map = out.map;
     base.out_f = out.f;
     base.key_kind = 0;
 
@@ -1699,7 +1693,6 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
     VA_CHECK_STATUS(s.reserve(need));
     uint32_t* thr = s.carve<uint32_t>(Q);
     uint32_t* cnt = s.carve<uint32_t>(Q);
-    uint32_t* ubound = s.carve<uint32_t>(Q);
     uint32_t* rcount = s.carve<uint32_t>(Q);
     uint32_t* ovf_rows = s.carve<uint32_t>(Q);
     uint32_t* ovf_cnt = s.carve<uint32_t>(kZeroWords);
@@ -1746,8 +1739,19 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
     // approximate bound per 32-row group (the scan's epilogue takes the group minimum: no dense
     // keys, no bound pass) and selects among those: the rank-th smallest group minimum is close
     // to the rank-th smallest bound when the rank is far below the group count.
-    const bool group_min = rank < k && !(in.xh && Q <= kSmallBatchMax) && S >= 128ull * rank;
-    const uint32_t groups = uint32_t((S + scr::TN - 1) / scr::TN * (scr::TN / 32));
+    // Small batches over the shadow take groups of 4 or 8 rows.
+    const bool narrow = Q <= GminA::queries;
+    const bool small_min = rank < k && in.xh && Q <= kSmallGminMax && uint64_t(Q) * S <= kSmallGminPairs &&
+                           S >= 32ull * rank;
+    const bool group_min = small_min || (rank < k && !(in.xh && Q <= kSmallBatchMax) && S >= 128ull * rank);
+    const uint32_t groups = small_min ? small_gmin_groups(narrow, S)
+                                      : uint32_t((S + scr::TN - 1) / scr::TN * (scr::TN / 32));
+    auto with_pretest = [&](SelectArgs& sel, uint32_t q0) {
+        if (!in.xh) return;
+        sel.ptc = ptc + q0;
+        sel.qinfo = qinfo + q0;
+        sel.bound = ScreenBound{sa.op, sa.c1, sa.cn, sa.c0x, sa.kabs};
+    };
     for (uint32_t q0 = 0; q0 < Q; q0 += plan.qs) {
         const uint32_t nq = std::min(plan.qs, Q - q0);
         ScreenArgs a = sa;
@@ -1768,7 +1772,8 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
                 a.xn = in.xn;
                 a.xstride = plan.stride;
             }
-            if (in.xh && screen16_gmin_fits(a)) VA_CHECK_STATUS(launch_screen16_gmin(ctx, a));
+            if (small_min) VA_CHECK_STATUS(launch_small_gmin(ctx, a, narrow));
+            else if (in.xh && screen16_gmin_fits(a)) VA_CHECK_STATUS(launch_screen16_gmin(ctx, a));
             else VA_CHECK_STATUS(launch_screen<SCREEN_GMIN>(ctx, a));
             SelectArgs sel;
             sel.keys = skeys;
@@ -1777,6 +1782,7 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
             sel.rows = nq;
             sel.k = rank;
             sel.out_kth = thr + q0;
+            with_pretest(sel, q0);
             VA_CHECK_STATUS(launch_select(ctx, sel));
             continue;
         }
@@ -1789,8 +1795,7 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
         } else {
             VA_CHECK_STATUS(launch_screen<SCREEN_KEYS>(ctx, a));
         }
-        VA_CHECK_STATUS(launch_bounds(ctx, a, reinterpret_cast<float*>(skeys), sxx, nullptr, nullptr, uint32_t(S),
-                                      int64_t(S), nq));
+        VA_CHECK_STATUS(launch_bounds(ctx, a, reinterpret_cast<float*>(skeys), sxx, uint32_t(S), int64_t(S), nq));
         VA_CHECK_STATUS(mask_dense_keys(ctx, skeys, nq, uint32_t(S), int64_t(S), 0, plan.stride, out.skip));
         SelectArgs sel;
         sel.keys = skeys;
@@ -1799,6 +1804,7 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
         sel.rows = nq;
         sel.k = rank;
         sel.out_kth = thr + q0;
+        with_pretest(sel, q0);
         VA_CHECK_STATUS(launch_select(ctx, sel));
     }
     // ---- 3. screening scan -------------------------------------------------------------------
@@ -1829,8 +1835,6 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
             a.xh = in.xh;
             a.xn = in.xn;
             a.ptc = ptc;
-            pretest_kernel<<<dim3((Q + 255) / 256), dim3(256), 0, ctx->stream>>>(a, Q, ptc);
-            VA_CHECK_LAUNCH(ctx);
             if (Q <= kSmallBatchMax)
                 VA_CHECK_STATUS(launch_screen16_small<SCREEN_FILTER>(ctx, a));
             else
@@ -1839,37 +1843,38 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
             VA_CHECK_STATUS(launch_screen<SCREEN_FILTER>(ctx, a));
         }
         VA_CHECK_STATUS(pm.mark(2));
-        // (dot, |x|^2) -> (key of hi, key of lo), in place
-        VA_CHECK_STATUS(launch_bounds(ctx, a, reinterpret_cast<float*>(chi), nullptr, reinterpret_cast<float*>(clo), cnt,
-                                      uint32_t(cap), int64_t(cap), Q));
-        VA_CHECK_STATUS(mask_list_keys(ctx, chi, clo, cid, cnt, Q, uint32_t(cap), int64_t(cap), out.skip));
+        // ---- 4. k-th smallest upper bound among the candidates and the rerank lists ------------
+        BandArgs b;
+        b.cnt = cnt;
+        b.hi = chi;
+        b.lo = clo;
+        b.id = cid;
+        b.cap = uint32_t(cap);
+        b.k = k;
+        b.min_count = rank < k ? k : 0u;
+        b.thr = rank < k ? thr : nullptr;
+        b.skip = out.skip;
+        b.rr = rr;
+        b.rcount = rcount;
+        b.rcap = uint32_t(rcap);
+        b.ovf_cnt = ovf_cnt;
+        b.ovf_rows = ovf_rows;
+        const bool tall = band_tall(ctx, Q);
+        b.list = band_list(tall, b.cap);
+        const size_t lds = size_t(b.list) * 8;
+        if (tall) {
+            VA_CHECK_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(&screen_band_kernel<1024>),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+            screen_band_kernel<1024><<<dim3(Q), dim3(1024), lds, ctx->stream>>>(a, b);
+        } else {
+            screen_band_kernel<512><<<dim3(Q), dim3(512), lds, ctx->stream>>>(a, b);
+        }
+        VA_CHECK_LAUNCH(ctx);
     }
     ctx->last_scan.scan_launches = 1;
     ctx->last_scan.sample_rows = uint32_t(S);
     ctx->last_scan.candidate_cap = uint32_t(cap);
     ctx->last_scan.screened = in.xh ? 2u : 1u;  // 2: screen16_kernel over the fp16 shadow
-    // ---- 4. k-th smallest upper bound among the candidates (overflowed lists are listed) ------
-    {
-        SelectArgs a;
-        a.keys = chi;
-        a.ids = cid;
-        a.counts = cnt;
-        a.ld = int64_t(cap);
-        a.n = uint32_t(cap);
-        a.rows = Q;
-        a.k = k;
-        a.out_kth = ubound;
-        a.overflow_count = ovf_cnt;
-        a.overflow_rows = ovf_rows;
-        a.min_count = rank < k ? k : 0;
-        VA_CHECK_STATUS(launch_select(ctx, a));
-    }
-    // ---- 5. rerank lists ------------------------------------------------------------------------
-    screen_compact_kernel<<<dim3(Q), dim3(256), 0, ctx->stream>>>(cnt, clo, cid, ubound, uint32_t(cap),
-                                                                 rank < k ? k : 0u, rank < k ? thr : nullptr, rr,
-                                                                 rcount, uint32_t(rcap), ovf_cnt, ovf_rows,
-                                                                 ovf_cnt + 1);
-    VA_CHECK_LAUNCH(ctx);
     // Without the device fallback the overflow count is read back (one synchronisation).
     uint32_t n_ovf = 0;
     if (!device_fb) {
@@ -1877,15 +1882,16 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
         VA_CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
         n_ovf = ctx->host_word[0];
     }
-    // ---- 6. exact fp32 keys of the rerank rows ---------------------------------------------------
+    // ---- 5. exact fp32 keys of the rerank rows ---------------------------------------------------
     {
         const uint64_t items = uint64_t(Q) * ((rcap + 63) / 64);
         const uint32_t blocks = uint32_t(std::min<uint64_t>(2048, (items + 3) / 4));
         // small batches keep few waves busy, each on its own: 8-row chunks (eight times the waves,
         // each streaming an eighth of the rows), the query staged in LDS and eight row groups in
-        // flight per wave
+        // flight per wave (100,000 x 768, Q = 100: 27.6 -> 16.3 us; the lanes past the eighth idle,
+        // so a full chip takes the 64-row chunks: 1M x 768, Q = 1024 178 us against 446)
         const size_t qlds = size_t(4) * ((D + 3) & ~3u) * 4;
-        if (Q <= kSmallBatchMax && qlds <= 64 * 1024) {
+        if (Q <= kRerankSmall && qlds <= 64 * 1024) {
             const uint64_t items8 = uint64_t(Q) * ((rcap + 7) / 8);
             rerank_kernel<8, true, 1><<<dim3(uint32_t(std::min<uint64_t>(4096, (items8 + 3) / 4))), dim3(256), qlds,
                                         ctx->stream>>>(in.q, in.x, D, int(in.op), rr, rcount, uint32_t(rcap), Q, rkey);
@@ -1893,9 +1899,8 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
             rerank_kernel<2, false><<<dim3(blocks), dim3(256), 0, ctx->stream>>>(in.q, in.x, D, int(in.op), rr,
                                                                                 rcount, uint32_t(rcap), Q, rkey);
         VA_CHECK_LAUNCH(ctx);
-        VA_CHECK_STATUS(mask_list_keys(ctx, rkey, nullptr, rr, rcount, Q, uint32_t(rcap), int64_t(rcap), out.skip));
     }
-    // ---- 7. exact (key, id) top-k ----------------------------------------------------------------
+    // ---- 6. exact (key, id) top-k ----------------------------------------------------------------
     {
         SelectArgs a = base;
         a.keys = rkey;
@@ -1911,8 +1916,7 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
     if (device_fb) VA_CHECK_STATUS(pm.count_overflow(ovf_cnt));
     VA_CHECK_STATUS(pm.mark(3));
     if (device_fb) {
-        // ---- 8. exact top-k of the overflowed queries (listed by steps 4 and 5), over the rows
-        // step 7 wrote
+        // ---- 7. exact top-k of the overflowed queries (listed by step 4), over the rows step 6 wrote
         VA_CHECK_STATUS(exact.fallback(fb, fb_select_args(fb, base, exact.key_bits())));
         return pm.finish(true, true);
     }

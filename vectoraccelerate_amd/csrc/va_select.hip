@@ -31,6 +31,12 @@ __global__ __launch_bounds__(NT) void select_kernel(SelectArgs a) {
         select_row<NT, true, KTH>(a, row, lds, s_row);
     else
         select_row<NT, false, KTH>(a, row, lds, s_row);
+    if constexpr (KTH)
+        if (a.ptc && threadIdx.x == 0) {  // (the thread that wrote the threshold)
+            const float4 inf = a.qinfo[row];
+            const PreTest p = pretest_consts(a.bound, inf.x, inf.y, inf.z, inf.w, a.out_kth[row]);
+            a.ptc[row] = float4{p.A, p.B, p.C, inf.z};
+        }
 }
 
 // float values -> ordering keys (dense matrices given to va_topk_select)

@@ -25,12 +25,15 @@ struct RowView {
     __device__ uint32_t id(uint32_t i) const { return ids ? ids[i] : i; }
 };
 
-// The LDS of a row's selection (KTH: threshold mode, without the winners).
-template <bool KTH>
-struct SelectLds {
+// The LDS of a search for the k-th smallest value.
+struct RadixLds {
     uint32_t digit, before, bin, cnt, lo, hi;
     uint32_t wsum[16];
     uint32_t whist[SEL_BINS];
+};
+// ... and of a row's selection (KTH: threshold mode, without the winners).
+template <bool KTH>
+struct SelectLds : RadixLds {
     uint32_t okey[KTH ? 1 : SEL_BUF];
     uint32_t oid[KTH ? 1 : SEL_BUF];
 };
@@ -94,15 +97,103 @@ __device__ __forceinline__ void hist_add(uint32_t* hist, bool m, uint32_t d) {
     if ((rest >> lane) & 1ull) atomicAdd(&hist[d], 1u);
 }
 
+// The need-th smallest value of the items for_vals(f) runs f(value, taken) over, all within
+// [base, base + 2^bits): histograms of up to 11 bits at a time, from the top, until the bin that
+// holds it has at most SEL_FEW items (the tail of a spread of distances: usually after the
+// first), which are ranked directly.  need becomes its rank among the items equal to it, eq
+// their number.  Every thread of an NT-thread workgroup calls it.
+template <int NT, class ForVals>
+__device__ inline uint32_t radix_kth(RadixLds& lds, ForVals&& for_vals, uint32_t base, uint32_t bits, uint32_t& need,
+                                     uint32_t& eq) {
+    const int tid = threadIdx.x;
+    uint32_t prefix = 0;
+    uint32_t left = bits;
+    while (left) {
+        const uint32_t w = left < SEL_BITS ? left : SEL_BITS, sh = left - w, nb = 1u << w;
+        for (uint32_t b = tid; b < nb; b += NT) lds.whist[b] = 0;
+        __syncthreads();
+        for_vals([&](uint32_t v, bool taken) {
+            const uint32_t d = v - base;
+            const bool m = taken && (left == bits || (d >> left) == prefix);
+            // (a value past the range, a sentinel above every real one, lands in the top bin)
+            const uint32_t bin = d >> sh;
+            hist_add(lds.whist, m, left == bits ? min(bin, nb - 1u) : (bin & (nb - 1u)));
+        });
+        __syncthreads();
+        find_bin_wide<NT>(lds.whist, nb, need, lds.wsum, &lds.digit, &lds.before, &lds.bin);
+        __syncthreads();
+        prefix = (prefix << w) | lds.digit;
+        need -= lds.before;
+        eq = lds.bin;
+        left = sh;
+        __syncthreads();
+        if (left && eq <= SEL_FEW) {
+            if (tid == 0) lds.cnt = 0;
+            __syncthreads();
+            for_vals([&](uint32_t v, bool taken) {
+                if (taken && ((v - base) >> left) == prefix) lds.whist[atomicAdd(&lds.cnt, 1u)] = v;
+            });
+            __syncthreads();
+            const uint32_t few = eq, want = need;
+            if (uint32_t(tid) < few) {
+                const uint32_t v = lds.whist[tid];
+                uint32_t below = 0, same = 0;
+                for (uint32_t j = 0; j < few; ++j) {
+                    const uint32_t o = lds.whist[j];
+                    below += o < v;
+                    same += o == v;
+                }
+                if (below < want && want <= below + same) {  // (every item equal to the answer writes the same)
+                    lds.lo = v;
+                    lds.before = below;
+                    lds.bin = same;
+                }
+            }
+            __syncthreads();
+            const uint32_t t = lds.lo;
+            need = want - lds.before;
+            eq = lds.bin;
+            __syncthreads();
+            return t;
+        }
+    }
+    return base + prefix;
+}
+
+// The need-th smallest key of for_keys(f): mn and mx are the smallest and largest of this thread's
+// keys.  The histograms start below the leading bits that all keys share: nearby distances have
+// equal top bits, and bins of those bits alone would count everything in one bin.
+template <int NT, class ForKeys>
+__device__ inline uint32_t kth_key(RadixLds& lds, ForKeys&& for_keys, uint32_t mn, uint32_t mx, uint32_t& need,
+                                   uint32_t& eq) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        mn = min(mn, uint32_t(__shfl_xor(int(mn), off)));
+        mx = max(mx, uint32_t(__shfl_xor(int(mx), off)));
+    }
+    if (threadIdx.x == 0) {
+        lds.lo = 0xFFFFFFFFu;
+        lds.hi = 0;
+    }
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) {
+        atomicMin(&lds.lo, mn);
+        atomicMax(&lds.hi, mx);
+    }
+    __syncthreads();
+    const uint32_t lo = lds.lo, hi = lds.hi;
+    return radix_kth<NT>(lds, [&](auto&& f) { for_keys([&](uint32_t k) { f(k, true); }); }, lo,
+                         hi == lo ? 0u : 32u - uint32_t(__builtin_clz(hi - lo)), need, eq);
+}
+
 // Exact top-k of one row (every thread of an NT-thread workgroup calls it; a caller that selects
 // several rows in turn puts a barrier between them).  KTH: threshold mode only (a.out_kth
 // set): no winners buffer, so a cached row of up to 16K keys leaves room for two workgroups per CU.
 // CACHED: the row's keys are copied to s_row (LDS) first.
 template <int NT, bool CACHED, bool KTH>
 __device__ void select_row(const SelectArgs& a, uint32_t row, SelectLds<KTH>& lds, uint32_t* s_row) {
-    uint32_t &s_digit = lds.digit, &s_before = lds.before, &s_bin = lds.bin, &s_cnt = lds.cnt;
-    uint32_t &s_lo = lds.lo, &s_hi = lds.hi;
-    uint32_t *const okey = lds.okey, *const oid = lds.oid, *const whist = lds.whist;
+    uint32_t& s_cnt = lds.cnt;
+    uint32_t *const okey = lds.okey, *const oid = lds.oid;
     const int tid = threadIdx.x;
     const uint32_t orow = a.row_map ? a.row_map[row] : row;
 
@@ -173,105 +264,29 @@ __device__ void select_row(const SelectArgs& a, uint32_t row, SelectLds<KTH>& ld
         for (; i < n; i += NT) f(rv.key(i));
     };
 
-    // The need-th smallest value of the items for_vals(f) runs f(value, taken) over, all within
-    // [base, base + 2^bits): histograms of up to 11 bits at a time, from the top, until the bin that
-    // holds it has at most SEL_FEW items (the tail of a spread of distances: usually after the
-    // first), which are ranked directly.  need becomes its rank among the items equal to it, eq
-    // their number.
-    auto radix = [&](auto&& for_vals, uint32_t base, uint32_t bits, uint32_t& need, uint32_t& eq) {
-        uint32_t prefix = 0;
-        uint32_t left = bits;
-        while (left) {
-            const uint32_t w = left < SEL_BITS ? left : SEL_BITS, sh = left - w, nb = 1u << w;
-            for (uint32_t b = tid; b < nb; b += NT) whist[b] = 0;
-            __syncthreads();
-            for_vals([&](uint32_t v, bool taken) {
-                const uint32_t d = v - base;
-                const bool m = taken && (left == bits || (d >> left) == prefix);
-                // (a value past the range, a sentinel above every real one, lands in the top bin)
-                const uint32_t bin = d >> sh;
-                hist_add(whist, m, left == bits ? min(bin, nb - 1u) : (bin & (nb - 1u)));
-            });
-            __syncthreads();
-            find_bin_wide<NT>(whist, nb, need, lds.wsum, &s_digit, &s_before, &s_bin);
-            __syncthreads();
-            prefix = (prefix << w) | s_digit;
-            need -= s_before;
-            eq = s_bin;
-            left = sh;
-            __syncthreads();
-            if (left && eq <= SEL_FEW) {
-                if (tid == 0) s_cnt = 0;
-                __syncthreads();
-                for_vals([&](uint32_t v, bool taken) {
-                    if (taken && ((v - base) >> left) == prefix) whist[atomicAdd(&s_cnt, 1u)] = v;
-                });
-                __syncthreads();
-                const uint32_t few = eq, want = need;
-                if (uint32_t(tid) < few) {
-                    const uint32_t v = whist[tid];
-                    uint32_t below = 0, same = 0;
-                    for (uint32_t j = 0; j < few; ++j) {
-                        const uint32_t o = whist[j];
-                        below += o < v;
-                        same += o == v;
-                    }
-                    if (below < want && want <= below + same) {  // (every item equal to the answer writes the same)
-                        s_lo = v;
-                        s_before = below;
-                        s_bin = same;
-                    }
-                }
-                __syncthreads();
-                const uint32_t t = s_lo;
-                need = want - s_before;
-                eq = s_bin;
-                __syncthreads();
-                return t;
-            }
-        }
-        return base + prefix;
-    };
-
     uint32_t T = 0xFFFFFFFFu, Tid = 0xFFFFFFFFu;
     bool take_all = (n <= a.k);
     if (!take_all) {
         // ---- phase 1: k-th smallest key ---------------------------------------------
-        // The histograms start below the leading bits that all keys share: nearby distances have
-        // equal top bits, and bins of those bits alone would count everything in one bin.
-        uint32_t need = K, eq = n, lo = 0, bits = a.key_bits;
-        if (a.key_bits > SEL_BITS) {
+        uint32_t need = K, eq = n;
+        if (a.key_bits <= SEL_BITS) {
+            T = radix_kth<NT>(lds, [&](auto&& f) { for_keys([&](uint32_t k) { f(k, true); }); }, 0u, a.key_bits, need, eq);
+        } else {
             if (!CACHED)
                 for_keys([&](uint32_t k) {
                     mn = min(mn, k);
                     mx = max(mx, k);
                 });
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                mn = min(mn, uint32_t(__shfl_xor(int(mn), off)));
-                mx = max(mx, uint32_t(__shfl_xor(int(mx), off)));
-            }
-            if (tid == 0) {
-                s_lo = 0xFFFFFFFFu;
-                s_hi = 0;
-            }
-            __syncthreads();
-            if ((tid & 63) == 0) {
-                atomicMin(&s_lo, mn);
-                atomicMax(&s_hi, mx);
-            }
-            __syncthreads();
-            lo = s_lo;
-            bits = s_hi == lo ? 0u : 32u - uint32_t(__builtin_clz(s_hi - lo));
+            T = kth_key<NT>(lds, for_keys, mn, mx, need, eq);
         }
-        T = radix([&](auto&& f) { for_keys([&](uint32_t k) { f(k, true); }); }, lo, bits, need, eq);
         if (KTH || a.out_kth) {
             if (tid == 0) a.out_kth[orow] = T;
             return;
         }
         // ---- phase 2: among key == T take the `need` lowest ids ----------------------
         if (need < eq)
-            Tid = radix(
+            Tid = radix_kth<NT>(
+                lds,
                 [&](auto&& f) {
                     for (uint32_t i = tid; i < n; i += NT) {
                         const bool t = rv.key(i) == T;
@@ -309,7 +324,7 @@ __device__ void select_row(const SelectArgs& a, uint32_t row, SelectLds<KTH>& ld
         const int64_t o = int64_t(orow) * (a.out_ld ? a.out_ld : int64_t(a.k)) + r;
         have = have && wk != kAbsentKey;
         const uint32_t k = have ? wk : 0xFFFFFFFFu;
-        if (a.out_idx) a.out_idx[o] = have ? wid + id_offset : kSentinel;
+        if (a.out_idx) a.out_idx[o] = !have ? kSentinel : a.out_map ? a.out_map[wid + id_offset] : wid + id_offset;
         if (a.out_key) a.out_key[o] = k;
         if (a.out_f) {
             float v;
