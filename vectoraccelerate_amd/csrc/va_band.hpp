@@ -61,6 +61,7 @@ __device__ inline void band_row(const BandArgs& a, uint32_t q, BandLds& lds, uin
             a.rcount[q] = 0;
             a.ovf_rows[atomicAdd(a.ovf_cnt, 1u)] = q;
         }
+        if (tid == 0 && a.out_kth) a.out_kth[q] = 0xFFFFFFFFu;
     };
     if (n > a.cap || n < a.min_count) return give_up();
     const int64_t o = int64_t(q) * a.cap;

@@ -498,8 +498,10 @@ va_status launch_shape(va_context* ctx, const DistArgs& a, bool vec) {
 // Measured against one-wave GEMM tiles, whole searches, top-10: 20,000 x 768, Q = 1 104 -> 38 us;
 // 200,000 x 768, Q = 8 189 -> 186; 500,000 x 768, Q = 1 390 -> 353 (1.5 GB: 4.4 TB/s).
 // TAIL: D % 4 != 0 (a lane's four values may run into the next row: cleared past D).
+// A launch of at most one wave per SIMD is bound by its waves' own chains: R = 8 there, one wave per
+// workgroup so that they spread over the CUs (1,024 x 768, Q = 16: 24.6 -> 21.2 us; a search of 5,000 x 128, Q = 1: 18.4 -> 17.0).
 template <int R, bool TAIL, int OUT, int OP>
-__global__ __launch_bounds__(256, 2) void dist_stream_kernel(DistArgs a) {
+__global__ __launch_bounds__(256, R > 4 ? 1 : 2) void dist_stream_kernel(DistArgs a) {
     const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t D = a.D, nch = (D + 31) / 32, nqb = (a.Q + 31) / 32;
@@ -507,7 +509,8 @@ __global__ __launch_bounds__(256, 2) void dist_stream_kernel(DistArgs a) {
     struct Slot {
         f32x4v x[4], q[4];
     };
-    for (uint32_t tile = blockIdx.x * 4 + wave; tile < ntiles; tile += gridDim.x * 4) {
+    const uint32_t nw = blockDim.x >> 6;
+    for (uint32_t tile = blockIdx.x * nw + wave; tile < ntiles; tile += gridDim.x * nw) {
         const uint32_t rt = nqb == 1 ? tile : tile / nqb;
         const uint32_t q0 = (tile - rt * nqb) * 32, qn = min(32u, a.Q - q0);
         const __amdgpu_buffer_rsrc_t qres =
@@ -642,7 +645,10 @@ template <int OUT, int OP>
 void launch_stream_op(va_context* ctx, const DistArgs& a) {
     const uint32_t tiles = ceil_div(a.N, 32) * ceil_div(a.Q, 32);
     const uint32_t grid = std::min((tiles + 3) / 4, 8 * uint32_t(ctx->num_cus));
-    if (a.D % 4)
+    if (tiles <= 4 * uint32_t(ctx->num_cus)) {
+        if (a.D % 4) dist_stream_kernel<8, true, OUT, OP><<<dim3(tiles), dim3(64), 0, ctx->stream>>>(a);
+        else dist_stream_kernel<8, false, OUT, OP><<<dim3(tiles), dim3(64), 0, ctx->stream>>>(a);
+    } else if (a.D % 4)
         dist_stream_kernel<4, true, OUT, OP><<<dim3(grid), dim3(256), 0, ctx->stream>>>(a);
     else
         dist_stream_kernel<4, false, OUT, OP><<<dim3(grid), dim3(256), 0, ctx->stream>>>(a);

@@ -689,6 +689,8 @@ va_status build_shadow(va_context* ctx, const float* x, uint32_t N, uint32_t D, 
 va_status screen_prepare_queries(va_context* ctx, const float* q, uint32_t Q, uint32_t D, _Float16* qh,
                                  float4* qinfo, float c0, float* qerr = nullptr, uint32_t* zero0 = nullptr,
                                  uint32_t n0 = 0, uint32_t* zero1 = nullptr, uint32_t n1 = 0);
+// Reranks of at most this many queries take 8-row chunks (rerank_kernel, ivf_rerank_kernel).
+constexpr uint32_t kRerankSmall = 128;
 // Whether the screened path applies (metric, alignment, sizes, VA_OPT_SCREEN).
 bool screen_applies(const va_context* ctx, const ScreenInput& in, uint32_t k);
 va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer& exact, uint32_t k,

@@ -360,6 +360,8 @@ __global__ __launch_bounds__(256) void ivf_small_kernel(DistArgs a) {
 namespace iv16 {
 constexpr uint32_t TN = 128, WAVES = 4;
 constexpr int kGroupsUsed = 3;  // narrow, wide<1>, wide<2>
+// groups that the lists of a search of Q queries can fall into (no list is probed by more)
+inline int groups_for(uint32_t Q) { return Q <= 16 ? 1 : (Q <= 32 ? 2 : kGroupsUsed); }
 __host__ __device__ inline int group_of(uint32_t nq) { return nq <= 16 ? 0 : (nq <= 32 ? 1 : 2); }
 __host__ __device__ inline uint32_t group_tq(int g) { return g == 0 ? 16u : 32u * uint32_t(g); }
 }  // namespace iv16
@@ -378,7 +380,7 @@ struct Ivf16Args {
     const float2* xn = nullptr;      // [N] {|x|^2, bound of |fp16(x) - x|}
     uint32_t Dp = 0;
     BoundV bnd{};
-    const uint32_t* thr = nullptr;   // tau_q as keys (~0: every pair passes)
+    const uint32_t* thr = nullptr;   // tau_q as keys (nullptr or ~0: every pair passes)
     uint32_t* cnt = nullptr;
     float* cand_dot = nullptr;       // unscaled fp16 dots
     uint32_t* cand_pos = nullptr;    // CSR positions
@@ -519,7 +521,7 @@ __device__ __forceinline__ void wide_tile(const Ivf16Args& a, float2* xs, uint32
 #pragma unroll
     for (int n = 0; n < W; ++n) {
         const float4 inf = a.qinfo[qi[n]];
-        pt[n] = pretest_v(a.bnd, inf.x, inf.y, a.qerr[qi[n]], inf.z, a.thr[qi[n]]);
+        pt[n] = pretest_v(a.bnd, inf.x, inf.y, a.qerr[qi[n]], inf.z, a.thr ? a.thr[qi[n]] : 0xFFFFFFFFu);
         inv[n] = inf.z;
     }
 #pragma unroll
@@ -663,7 +665,7 @@ __global__ __launch_bounds__(256, 2) void ivf16_narrow_kernel(Ivf16Args a) {
         const float2 xn1 = uint32_t(64 + lane) < cur.rc ? a.xn[cur.rs + 64u + uint32_t(lane)] : make_float2(0.0f, 0.0f);
         const float4 inf = a.qinfo[cur.qi];
         const float eq = a.qerr[cur.qi];
-        const uint32_t th = a.thr[cur.qi];
+        const uint32_t th = a.thr ? a.thr[cur.qi] : 0xFFFFFFFFu;
 #pragma unroll
         for (int b = 0; b < 8; ++b) acc[b] = f32x4s{0.f, 0.f, 0.f, 0.f};
         // an even number of chunks (one of zeros when nch is odd), so the next tile's chunk 0
@@ -1432,7 +1434,6 @@ struct DevPlan {
     uint32_t* qoff = nullptr;   // [C + 1]
     uint32_t* qfill = nullptr;  // [C] fill cursors
     uint32_t* qlist = nullptr;  // [Q x np] (the first qoff[C] are used)
-    uint32_t* counts = nullptr; // [2][kGroups][C] tiles per list
     uint32_t* pre = nullptr;    // [2][kGroups][C + 1]
 };
 
@@ -1448,34 +1449,6 @@ __global__ __launch_bounds__(256) void plan_probes_kernel(DevPlan p) {
     }
 }
 
-// Exclusive prefix of in[0..n) into out[0..n] (out[n] = total), one workgroup of 1024 threads;
-// copy (may be null) receives out[0..n) as well.  Workgroup b scans array b of a batch.
-__global__ __launch_bounds__(1024) void plan_scan_kernel(const uint32_t* in, uint32_t n, uint32_t* out, uint32_t* copy,
-                                                        int64_t in_stride, int64_t out_stride) {
-    __shared__ uint32_t part[1024];
-    in += int64_t(blockIdx.x) * in_stride;
-    out += int64_t(blockIdx.x) * out_stride;
-    const uint32_t t = threadIdx.x, per = (n + 1023) / 1024;
-    const uint32_t b0 = min(n, t * per), b1 = min(n, b0 + per);
-    uint32_t s = 0;
-    for (uint32_t i = b0; i < b1; ++i) s += in[i];
-    part[t] = s;
-    __syncthreads();
-    for (uint32_t w = 1; w < 1024; w <<= 1) {  // inclusive Hillis-Steele scan of the partial sums
-        const uint32_t v = t >= w ? part[t - w] : 0u;
-        __syncthreads();
-        part[t] += v;
-        __syncthreads();
-    }
-    uint32_t run = part[t] - s;
-    for (uint32_t i = b0; i < b1; ++i) {
-        out[i] = run;
-        if (copy) copy[i] = run;
-        run += in[i];
-    }
-    if (t == 1023) out[n] = part[1023];
-}
-
 __global__ __launch_bounds__(256) void plan_fill_kernel(DevPlan p) {
     const uint64_t total = uint64_t(p.Q) * p.np;
     for (uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x; i < total; i += uint64_t(gridDim.x) * 256) {
@@ -1486,50 +1459,140 @@ __global__ __launch_bounds__(256) void plan_fill_kernel(DevPlan p) {
     }
 }
 
-__global__ __launch_bounds__(256) void plan_counts_kernel(DevPlan p) {
-    for (uint32_t l = blockIdx.x * 256 + threadIdx.x; l < p.C; l += gridDim.x * 256) {
-        const uint32_t nq = p.qcnt[l], n = p.roff[l + 1] - p.roff[l];
-        int g;
-        uint32_t TQ, TN;
-        if (p.screen) {
-            g = iv16::group_of(nq);
-            TQ = iv16::group_tq(g);
-            TN = iv16::TN;
-        } else {
-            g = (p.small_ok && nq <= kSmallListQueries) ? kSmallGroup : shape_for(nq, n);
-            group_tile(g, TQ, TN);
+// A list's tiles in a pass and the group that scans them.
+__device__ inline void plan_tiles(const DevPlan& p, int pass, uint32_t nq, uint32_t n, int& g, uint32_t& tiles) {
+    uint32_t TQ, TN;
+    if (p.screen) {
+        g = iv16::group_of(nq);
+        TQ = iv16::group_tq(g);
+        TN = iv16::TN;
+        if (pass == 1 && p.big_tq && nq > ivb::kMinQueries) {
+            g = 3;
+            TN = p.big_tn;
+            TQ = p.big_tq;
+        } else if (g == 2 && pass == 1 && p.wide_tn) {
+            TN = p.wide_tn;
+            TQ = p.wide_tq;
         }
-        for (int pass = 0; pass < 2; ++pass) {
-            if (p.screen && pass == 1 && p.big_tq && nq > ivb::kMinQueries) {
-                g = 3;
-                TN = p.big_tn;
-                TQ = p.big_tq;
-            } else if (p.screen && g == 2 && pass == 1 && p.wide_tn) {
-                TN = p.wide_tn;
-                TQ = p.wide_tq;
-            }
-            const uint32_t rows = pass == 0 ? ivf_sample_rows(n) : n;
-            const uint32_t tiles = (nq == 0 || rows == 0) ? 0u : ((nq + TQ - 1) / TQ) * ((rows + TN - 1) / TN);
-            for (int gi = 0; gi < kGroups; ++gi)
-                p.counts[(int64_t(pass) * kGroups + gi) * p.C + l] = gi == g ? tiles : 0u;
+    } else {
+        g = (p.small_ok && nq <= kSmallListQueries) ? kSmallGroup : shape_for(nq, n);
+        group_tile(g, TQ, TN);
+    }
+    const uint32_t rows = pass == 0 ? ivf_sample_rows(n) : n;
+    tiles = (nq == 0 || rows == 0) ? 0u : ((nq + TQ - 1) / TQ) * ((rows + TN - 1) / TN);
+}
+
+// The lists' query offsets and every group's tile prefixes, one workgroup: each thread sums its run
+// of lists, one scan of all sums at once (wave shuffles, then the waves' totals), and each thread
+// walks its run again.  ONE (few probes over few lists): the probes are counted before and the query
+// lists filled after, with the counters in LDS, so the whole plan is one launch (six of them took 38 us
+// of a search of 16 queries).
+constexpr uint32_t kPlanOneLists = 8192, kPlanOnePairs = 4096, kPlanOneProbes = 64;
+template <bool ONE>
+__global__ __launch_bounds__(1024) void plan_lists_kernel(DevPlan p) {
+    constexpr int A = 2 * kGroups + 1;
+    __shared__ uint32_t s_tot[16][A];
+    __shared__ uint32_t s_cnt[ONE ? kPlanOneLists : 1];
+    const uint32_t t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const uint32_t pairs = p.Q * p.np;  // (ONE: at most kPlanOnePairs)
+    if constexpr (ONE) {
+        for (uint32_t l = t; l < p.C; l += 1024) s_cnt[l] = 0;
+        __syncthreads();
+        for (uint32_t i = t; i < pairs; i += 1024) {
+            const uint32_t q0 = i / p.np * p.np, l = p.probes[i];
+            bool ok = l < p.C;
+            for (uint32_t j = q0; ok && j < i; ++j) ok = p.probes[j] != l;
+            p.P[i] = ok ? l : 0xFFFFFFFFu;
+            if (ok) atomicAdd(s_cnt + l, 1u);
+        }
+        __syncthreads();
+    }
+    const uint32_t per = (p.C + 1023) / 1024;
+    const uint32_t b0 = min(p.C, t * per), b1 = min(p.C, b0 + per);
+    // f(list, queries, per pass: group, tiles)
+    auto walk = [&](auto&& f) {
+        for (uint32_t l = b0; l < b1; ++l) {
+            const uint32_t nq = ONE ? s_cnt[l] : p.qcnt[l], n = p.roff[l + 1] - p.roff[l];
+            int g0, g1;
+            uint32_t t0, t1;
+            plan_tiles(p, 0, nq, n, g0, t0);
+            plan_tiles(p, 1, nq, n, g1, t1);
+            f(l, nq, g0, t0, g1, t1);
+        }
+    };
+    uint32_t run[A];
+#pragma unroll
+    for (int i = 0; i < A; ++i) run[i] = 0;
+    auto add = [&](uint32_t nq, int g0, uint32_t t0, int g1, uint32_t t1) {
+        run[0] += nq;
+#pragma unroll
+        for (int g = 0; g < kGroups; ++g) {
+            run[1 + g] += g == g0 ? t0 : 0u;
+            run[1 + kGroups + g] += g == g1 ? t1 : 0u;
+        }
+    };
+    walk([&](uint32_t, uint32_t nq, int g0, uint32_t t0, int g1, uint32_t t1) { add(nq, g0, t0, g1, t1); });
+#pragma unroll
+    for (int i = 0; i < A; ++i) {
+        const uint32_t own = run[i];
+        uint32_t v = own;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t o = uint32_t(__shfl_up(int(v), off));
+            if (lane >= uint32_t(off)) v += o;
+        }
+        if (lane == 63) s_tot[w][i] = v;
+        run[i] = v - own;
+    }
+    __syncthreads();
+    for (uint32_t i = 0; i < w; ++i)
+#pragma unroll
+        for (int j = 0; j < A; ++j) run[j] += s_tot[i][j];
+    uint32_t* const pre = p.pre;
+    const int64_t ld = int64_t(p.C) + 1;
+    auto put = [&](uint32_t l) {
+        p.qoff[l] = run[0];
+#pragma unroll
+        for (int i = 0; i < 2 * kGroups; ++i) pre[i * ld + l] = run[1 + i];
+    };
+    walk([&](uint32_t l, uint32_t nq, int g0, uint32_t t0, int g1, uint32_t t1) {
+        put(l);
+        if constexpr (ONE) {
+            p.qcnt[l] = nq;
+            s_cnt[l] = run[0];  // (this thread's list: read above)
+        } else {
+            p.qfill[l] = run[0];
+        }
+        add(nq, g0, t0, g1, t1);
+    });
+    if (t == 1023) put(p.C);  // (the last thread's sums end at the totals)
+    if constexpr (ONE) {
+        __syncthreads();
+        for (uint32_t i = t; i < pairs; i += 1024) {
+            const uint32_t l = p.P[i];  // (written by this thread)
+            if (l != 0xFFFFFFFFu) p.qlist[atomicAdd(s_cnt + l, 1u)] = i / p.np;
         }
     }
 }
 
-// Enqueues the device plan (probes -> lists -> tile prefixes).
-va_status plan_on_device(va_context* ctx, const DevPlan& p) {
-    VA_CHECK_STATUS(fill_u32(ctx, p.qcnt, p.C, 0));
+// Whether the whole plan is one launch (which also clears the list counters).
+bool plan_is_one(const DevPlan& p) {
+    return p.C <= kPlanOneLists && p.np <= kPlanOneProbes && uint64_t(p.Q) * p.np <= kPlanOnePairs;
+}
+// Enqueues the device plan (probes -> lists -> tile prefixes); cleared: p.qcnt holds zeros.
+va_status plan_on_device(va_context* ctx, const DevPlan& p, bool cleared) {
+    if (plan_is_one(p)) {
+        plan_lists_kernel<true><<<dim3(1), dim3(1024), 0, ctx->stream>>>(p);
+        VA_CHECK_LAUNCH(ctx);
+        return VA_OK;
+    }
+    if (!cleared) VA_CHECK_STATUS(fill_u32(ctx, p.qcnt, p.C, 0));
     plan_probes_kernel<<<dim3(p.Q), dim3(256), 0, ctx->stream>>>(p);
     VA_CHECK_LAUNCH(ctx);
-    plan_scan_kernel<<<dim3(1), dim3(1024), 0, ctx->stream>>>(p.qcnt, p.C, p.qoff, p.qfill, 0, 0);
+    plan_lists_kernel<false><<<dim3(1), dim3(1024), 0, ctx->stream>>>(p);
     VA_CHECK_LAUNCH(ctx);
     const uint64_t pairs = uint64_t(p.Q) * p.np;
     plan_fill_kernel<<<dim3(uint32_t(std::min<uint64_t>(4096, (pairs + 255) / 256))), dim3(256), 0, ctx->stream>>>(p);
-    VA_CHECK_LAUNCH(ctx);
-    plan_counts_kernel<<<dim3(std::min<uint32_t>(1024, (p.C + 255) / 256)), dim3(256), 0, ctx->stream>>>(p);
-    VA_CHECK_LAUNCH(ctx);
-    plan_scan_kernel<<<dim3(2 * kGroups), dim3(1024), 0, ctx->stream>>>(p.counts, p.C, p.pre, nullptr, p.C,
-                                                                          int64_t(p.C) + 1);
     VA_CHECK_LAUNCH(ctx);
     return VA_OK;
 }
@@ -1599,11 +1662,11 @@ va_status run_screen_pass(va_context* ctx, const DevPlan& dp, int pass, Ivf16Arg
     a.plan.C = dp.C;
     a.plan.sample = pass == 0 ? 1u : 0u;
     va_status st = VA_OK;
-    // the groups after the first run on aux streams 0 .. kGroupsUsed - 2 (each fork and join is a
-    // barrier packet on the context's stream: only the streams used)
-    constexpr int kAuxUsed = iv16::kGroupsUsed - 1;
-    static_assert(kAuxUsed <= va_context::kAux, "one aux stream per group after the first");
-    VA_CHECK_STATUS(aux_fork(ctx, kAuxUsed));
+    // the groups after the first run on auxiliary streams (each fork and join is a barrier packet on
+    // the context's stream, about 8 us a pair: only the streams used, none for up to 16 queries)
+    static_assert(iv16::kGroupsUsed - 1 <= va_context::kAux, "one aux stream per group after the first");
+    const int groups = iv16::groups_for(dp.Q), aux = groups - 1;
+    if (aux) VA_CHECK_STATUS(aux_fork(ctx, aux));
     if (pass == 1 && dp.big_tq) {
         // on the context's stream, ahead of the narrow tiles, while the wide groups start on the
         // auxiliary streams
@@ -1620,7 +1683,7 @@ va_status run_screen_pass(va_context* ctx, const DevPlan& dp, int pass, Ivf16Arg
                ctx->stream>>>(b);
         if (hipGetLastError() != hipSuccess) st = fail(ctx, VA_ERR_HIP, "ivf16_big_kernel launch failed");
     }
-    for (int g = 0; g < iv16::kGroupsUsed && st == VA_OK; ++g) {
+    for (int g = 0; g < groups && st == VA_OK; ++g) {
         a.plan.pre = dp.pre + (int64_t(pass) * kGroups + g) * (int64_t(dp.C) + 1);
         const hipStream_t s = g == 0 ? ctx->stream : ctx->aux[g - 1];
         if (g == 0) {
@@ -1657,7 +1720,7 @@ va_status run_screen_pass(va_context* ctx, const DevPlan& dp, int pass, Ivf16Arg
         }
         if (hipGetLastError() != hipSuccess) st = fail(ctx, VA_ERR_HIP, "screened list scan launch failed");
     }
-    const va_status j = aux_join(ctx, kAuxUsed);
+    const va_status j = aux ? aux_join(ctx, aux) : VA_OK;
     return st != VA_OK ? st : j;
 }
 
@@ -1790,6 +1853,9 @@ __global__ __launch_bounds__(256) void fb_ivf_kernel(FbIvf v, FbArgs a, SelectAr
 // probed by at most 16 queries; GemmChain: the distance GEMM's, otherwise), so every key equals
 // the fp32 list scan's, and the row's id replaces its position.  The rows pass through the wave's
 // LDS slot in coalesced 128-byte lines (rows_through_lds).
+// R, QLDS, NRG: as rerank_kernel's (few queries: 8-row chunks, the query in LDS; 1M x 768, Q = 16: 35.6 ->
+// 25.8 us).
+template <int R, bool QLDS, int NRG>
 __global__ __launch_bounds__(256) void ivf_rerank_kernel(const float* __restrict__ q, const float* __restrict__ x,
                                                          const uint32_t* __restrict__ ids,
                                                          const uint32_t* __restrict__ roff, uint32_t C,
@@ -1797,22 +1863,24 @@ __global__ __launch_bounds__(256) void ivf_rerank_kernel(const float* __restrict
                                                          const uint32_t* __restrict__ rr,
                                                          const uint32_t* __restrict__ rcount, uint32_t rcap, uint32_t Q,
                                                          uint32_t* __restrict__ rkey, uint32_t* __restrict__ rid) {
+    constexpr uint32_t CH = 8 * NRG;  // rows per chunk (one wave's)
     __shared__ fb_f32x4 slots[4][64 * 8];
+    extern __shared__ __attribute__((aligned(16))) float qstage[];  // QLDS: 4 x D floats
     const int lane = threadIdx.x & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t nch = (rcap + 63) / 64;
+    const uint32_t nch = (rcap + CH - 1) / CH;
     const uint64_t items = uint64_t(Q) * nch;
     const uint32_t nw = gridDim.x * 4;
     for (uint64_t it = uint64_t(blockIdx.x) * 4 + wave; it < items; it += nw) {
         const uint32_t c = uint32_t(it / Q), qi = uint32_t(it % Q);
         const uint32_t n = min(rcount[qi], rcap);
-        if (c * 64 >= n) continue;  // (uniform)
-        const uint32_t* rl = rr + int64_t(qi) * rcap + c * 64;
-        const uint32_t m = min(64u, n - c * 64);
-        uint32_t pos8[8];
-        bool rv[8];
+        if (c * CH >= n) continue;  // (uniform)
+        const uint32_t* rl = rr + int64_t(qi) * rcap + c * CH;
+        const uint32_t m = min(CH, n - c * CH);
+        uint32_t pos8[NRG];
+        bool rv[NRG];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < NRG; ++i) {
             const uint32_t r = uint32_t(8 * i + (lane >> 3));
             rv[i] = r < m;
             pos8[i] = rv[i] ? rl[r] : 0u;
@@ -1830,16 +1898,24 @@ __global__ __launch_bounds__(256) void ivf_rerank_kernel(const float* __restrict
             }
             small = qcnt[lo] <= kSmallListQueries;
         }
+        const float* qp = q + int64_t(qi) * D;
+        if constexpr (QLDS) {
+            // (the wave writes and then reads only its own region: in order, no barrier)
+            float* qw = qstage + wave * D;
+            for (uint32_t d = uint32_t(lane) * 4; d < D; d += 256)
+                *reinterpret_cast<fb_f32x4*>(qw + d) = *reinterpret_cast<const fb_f32x4*>(qp + d);
+            qp = qw;
+        }
         GemmChain gc;
         SmallChain sc;
-        rows_through_lds(q + int64_t(qi) * D, x, pos8, rv, D, slots[wave],
+        rows_through_lds<R, NRG>(qp, x, pos8, rv, D, slots[wave],
                          [&](uint32_t j, const fb_f32x4(&xv)[8], const fb_f32x4(&qv)[8]) {
                              if (small) sc.group(xv, qv);
                              else gc.group(xv, qv, j, D);
                          });
         if (mine) {
-            rkey[int64_t(qi) * rcap + c * 64 + lane] = small ? sc.key() : gc.key(int(OP_L2SQ));
-            rid[int64_t(qi) * rcap + c * 64 + lane] = ids[pos];
+            rkey[int64_t(qi) * rcap + c * CH + lane] = small ? sc.key() : gc.key(int(OP_L2SQ));
+            rid[int64_t(qi) * rcap + c * CH + lane] = ids[pos];
         }
     }
 }
@@ -1938,18 +2014,17 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     const size_t need = q4 * 5 + Scratch::round(uint64_t(Q) * 8) + Scratch::round(256) + Scratch::round(uint64_t(Q) * 16) +
                         Scratch::round(uint64_t(Q) * Dp * 2) + Scratch::round(pairs * 4) * 2 +
                         Scratch::round(uint64_t(C) * 4) * 2 + Scratch::round((uint64_t(C) + 1) * 4) +
-                        Scratch::round(uint64_t(2 * kGroups) * C * 4) +
                         Scratch::round(uint64_t(2 * kGroups) * (uint64_t(C) + 1) * 4) +
                         Scratch::round(uint64_t(Q) * cand * 4) * 3 + Scratch::round(uint64_t(Q) * rcap * 4) * 3 +
                         fb_bytes(Q, id_span, k, ivf->N) +
                         (ivf_big_applies(ctx, Q, Dp) ? Scratch::round(pairs * 16) + Scratch::round(pairs * 8) : 0);
     VA_CHECK_STATUS(s.reserve(need));
     uint32_t* thr = s.carve<uint32_t>(Q);
+    uint32_t* rcount = s.carve<uint32_t>(Q);
+    uint32_t* ovf_rows = s.carve<uint32_t>(Q);
     // list counts: [0, Q) the sample pass's, [Q, 2Q) the full pass's (both cleared by the prep)
     uint32_t* const cnt2 = s.carve<uint32_t>(uint64_t(Q) * 2);
     uint32_t* cnt = cnt2;
-    uint32_t* rcount = s.carve<uint32_t>(Q);
-    uint32_t* ovf_rows = s.carve<uint32_t>(Q);
     uint32_t* ovf_cnt = s.carve<uint32_t>(va::kZeroWords);
     float4* qinfo = s.carve<float4>(Q);
     float* qerr = s.carve<float>(Q);
@@ -1976,7 +2051,6 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     dp.qcnt = s.carve<uint32_t>(C);
     dp.qfill = s.carve<uint32_t>(C);
     dp.qoff = s.carve<uint32_t>(uint64_t(C) + 1);
-    dp.counts = s.carve<uint32_t>(uint64_t(2 * kGroups) * C);
     dp.pre = s.carve<uint32_t>(uint64_t(2 * kGroups) * (uint64_t(C) + 1));
     float* cdot = s.carve<float>(uint64_t(Q) * cand);  // becomes the keys of the upper bounds
     uint32_t* clo = s.carve<uint32_t>(uint64_t(Q) * cand);
@@ -2023,8 +2097,11 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     ctx->last_scan = va_scan_timings{};
     VA_CHECK_STATUS(pm.mark(0));
     // ---- 0. plan and queries --------------------------------------------------------------------
-    VA_CHECK_STATUS(plan_on_device(ctx, dp));
-    VA_CHECK_STATUS(screen_prepare_queries(ctx, queries, Q, D, qh, qinfo, bnd.c0, qerr, cnt2, 2 * Q, ovf_cnt, kZeroWords));
+    // (the preparation clears the counters: the list counts and, next to them, the overflow words; the
+    // plan's)
+    VA_CHECK_STATUS(screen_prepare_queries(ctx, queries, Q, D, qh, qinfo, bnd.c0, qerr, cnt2,
+                                           uint32_t(ovf_cnt + kZeroWords - cnt2), dp.qcnt, plan_is_one(dp) ? 0u : C));
+    VA_CHECK_STATUS(plan_on_device(ctx, dp, true));
     Ivf16Args a;
     a.qh = qh;
     a.nq = Q;
@@ -2034,12 +2111,10 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     a.xn = ivf->norms;
     a.Dp = Dp;
     a.bnd = make_bound_v(D);
-    a.thr = thr;
     a.cnt = cnt;
     a.cand_dot = cdot;
     a.cand_pos = cpos;
     // ---- 1. sample: tau_q = k-th smallest upper bound of the sampled pairs ----------------------
-    VA_CHECK_STATUS(fill_u32(ctx, thr, Q, 0xFFFFFFFFu));
     a.cap = uint32_t(cap_s);
     VA_CHECK_STATUS(run_screen_pass(ctx, dp, 0, a));
     band.out_kth = thr;
@@ -2048,6 +2123,7 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     // ---- 2. screen, 3. U_q and the rerank lists (overflowed queries are listed) ---------------------------------------
     cnt = cnt2 + Q;
     a.cnt = cnt;
+    a.thr = thr;
     a.cap = uint32_t(cap);
     if (dp.big_tq) {
         // the pre-test constants of every plan slot, for the tiles of ivf16_big_kernel
@@ -2069,11 +2145,15 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     VA_CHECK_STATUS(launch_band(cap));
     // ---- 4. exact keys ---------------------------------------------------------------------------
     {
-        const uint64_t items = uint64_t(Q) * ((rcap + 63) / 64);
-        const uint32_t blocks = uint32_t(std::min<uint64_t>(2048, (items + 3) / 4));
-        ivf_rerank_kernel<<<dim3(blocks), dim3(256), 0, ctx->stream>>>(queries, ivf->list_vectors, ivf->ids,
-                                                                       ivf->offsets, C, dp.qcnt, D, rr, rcount,
-                                                                       uint32_t(rcap), Q, rkey, rid);
+        auto go = [&](auto kern, uint32_t rows, uint32_t most, size_t lds) {
+            const uint64_t items = uint64_t(Q) * ((rcap + rows - 1) / rows);
+            kern<<<dim3(uint32_t(std::min<uint64_t>(most, (items + 3) / 4))), dim3(256), lds, ctx->stream>>>(
+                queries, ivf->list_vectors, ivf->ids, ivf->offsets, C, dp.qcnt, D, rr, rcount, uint32_t(rcap), Q, rkey,
+                rid);
+        };
+        const size_t qlds = size_t(4) * D * 4;
+        if (Q <= kRerankSmall && qlds <= 64 * 1024) go(&ivf_rerank_kernel<8, true, 1>, 8, 4096, qlds);
+        else go(&ivf_rerank_kernel<2, false, 8>, 64, 2048, 0);
         VA_CHECK_LAUNCH(ctx);
     }
     // ---- 5. exact (key, id) top-k, 6. overflowed queries -----------------------------------------
@@ -2092,7 +2172,7 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
         sel.rows = Q;
         VA_CHECK_STATUS(launch_select(ctx, sel));
     }
-    ctx->last_scan.scan_launches = iv16::kGroupsUsed + (dp.big_tq ? 1 : 0);
+    ctx->last_scan.scan_launches = uint32_t(iv16::groups_for(Q)) + (dp.big_tq ? 1 : 0);
     ctx->last_scan.candidate_cap = uint32_t(cap);
     ctx->last_scan.screened = 1;
     VA_CHECK_STATUS(pm.count_sum(rcount, Q));
@@ -2323,7 +2403,6 @@ va_status ivf_scan_masked(va_context* ctx, const va_ivf* ivf, const float* queri
     Scratch s(ctx);
     const size_t need = Scratch::round(uint64_t(Q) * 4) * 3 + Scratch::round(256) + Scratch::round(pairs * 4) * 2 +
                         Scratch::round(uint64_t(C) * 4) * 2 + Scratch::round((uint64_t(C) + 1) * 4) +
-                        Scratch::round(uint64_t(2 * va::kGroups) * C * 4) +
                         Scratch::round(uint64_t(2 * va::kGroups) * (uint64_t(C) + 1) * 4) +
                         Scratch::round(uint64_t(Q) * cand * 4) * 2 + va::fb_bytes(Q, id_span, k, ivf->N);
     VA_CHECK_STATUS(s.reserve(need));
@@ -2343,7 +2422,6 @@ va_status ivf_scan_masked(va_context* ctx, const va_ivf* ivf, const float* queri
     dp.qcnt = s.carve<uint32_t>(C);
     dp.qfill = s.carve<uint32_t>(C);
     dp.qoff = s.carve<uint32_t>(uint64_t(C) + 1);
-    dp.counts = s.carve<uint32_t>(uint64_t(2 * va::kGroups) * C);
     dp.pre = s.carve<uint32_t>(uint64_t(2 * va::kGroups) * (uint64_t(C) + 1));
     uint32_t* ckey = s.carve<uint32_t>(uint64_t(Q) * cand);
     uint32_t* cid = s.carve<uint32_t>(uint64_t(Q) * cand);
@@ -2358,7 +2436,7 @@ va_status ivf_scan_masked(va_context* ctx, const va_ivf* ivf, const float* queri
     ctx->last_scan = va_scan_timings{};
     VA_CHECK_STATUS(pm.mark(0));
     // ---- 0. plan: the queries of every probed list, tile prefixes per group and pass ------------
-    VA_CHECK_STATUS(va::plan_on_device(ctx, dp));
+    VA_CHECK_STATUS(va::plan_on_device(ctx, dp, false));
     // ---- 1. sample pass: every sampled candidate, then tau = k-th smallest ----------------------
     VA_CHECK_STATUS(va::fill_u32(ctx, thr, Q, 0xFFFFFFFFu));
     VA_CHECK_STATUS(va::fill_u32(ctx, cnt, Q, 0));

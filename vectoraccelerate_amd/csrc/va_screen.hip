@@ -1658,7 +1658,6 @@ bool screen_applies(const va_context* ctx, const ScreenInput& in, uint32_t k) {
     return in.xh ? true : in.Q >= kSmallBatch;
 }
 
-constexpr uint32_t kRerankSmall = 128;
 va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer& exact, uint32_t k,
                              const ScanOutputs& out) {
     const uint32_t Q = in.Q, N = in.N, D = in.D;
