@@ -349,7 +349,7 @@ __global__ __launch_bounds__(256) void ivf_small_kernel(DistArgs a) {
 // list scan, so the result is the fp32 list scan's, bit for bit.
 //
 // One wave per tile (no LDS staging, no barrier), persistent over the device plan:
-//   narrow : 16 queries x 128 rows, v_mfma_f32_16x16x32_f16 (lists probed by <= 16 queries);
+//   narrow : 16 queries x 32 rows, v_mfma_f32_16x16x32_f16 (lists probed by <= 16 queries);
 //   wide<W>: 32W queries x 128 rows, v_mfma_f32_32x32x16_f16 (W = 1: 17-32 queries, 2: more).
 // Both operands load straight into registers.  A dot is the same sum whatever the order of its
 // terms (the bound does not depend on it), so the k order inside a 64-value chunk follows the
@@ -359,6 +359,7 @@ __global__ __launch_bounds__(256) void ivf_small_kernel(DistArgs a) {
 // ivf_band_kernel.
 namespace iv16 {
 constexpr uint32_t TN = 128, WAVES = 4;
+constexpr uint32_t NTN = 32;  // rows of a narrow tile
 constexpr int kGroupsUsed = 3;  // narrow, wide<1>, wide<2>
 // groups that the lists of a search of Q queries can fall into (no list is probed by more)
 inline int groups_for(uint32_t Q) { return Q <= 16 ? 1 : (Q <= 32 ? 2 : kGroupsUsed); }
@@ -434,15 +435,6 @@ __device__ __forceinline__ void append_pairs(const Ivf16Args& a, uint32_t qi, ui
     }
 }
 
-// narrow tiles: lane (j, g) = (lane % 16, lane / 16) loads 16 halves at 64c + 16g of row j of
-// each 16-row block and of query j; MFMA u of chunk c takes halves 8u .. 8u + 7 of them.  The
-// result: lane (j, g) holds query j against rows 16b + 4g + v in acc[b][v].
-struct NarrowTile {
-    uint32_t qs = 0, qc = 0, rs = 0, rc = 0;
-    uint32_t qi = 0;                 // the lane's query (query j of the tile; query 0 of it past qc)
-    __amdgpu_buffer_rsrc_t xr;       // the tile's rows (loads past rc read zeros)
-    bool valid = false;              // false: every load of the tile reads zeros
-};
 // wide tile: lane (l32, hh) loads 32 halves at 64c + 32hh of row l32 of each 32-row block and of
 // query l32 of each 32-query block; MFMA u of chunk c takes halves 8u .. 8u + 7.  The result:
 // lane (l32, hh) holds query 32n + l32 against rows 32m + 8i + 4hh + e in acc[n][m][4i + e].
@@ -576,144 +568,149 @@ __global__ __launch_bounds__(NT) void ivf_band_kernel(BoundV bv, const float4* _
     });
 }
 
-// The 16-query tiles, one independent tile per wave, software-pipelined across the wave's tiles:
-// the next tile is located, and its first 64-value chunk requested, while the current one is
-// scanned, so the chunk's HBM latency overlaps the current tile's last chunk and epilogue; the
-// epilogue's inputs (the rows' {|x|^2, error bound}, the query's pre-test constants) are loaded
-// at the tile's start and used after its main loop.  Every wait for a load also waits for the
-// loads issued before it, so each wait is placed where those are due anyway.
+// The lists probed by at most 16 queries: one independent wave per share of their rows.  Reading the
+// rows is the cost (2 bytes a value, each once), so every wave takes an equal run of consecutive
+// 32-row tiles of the plan and streams the part of the run that lies in one list through a ring of
+// R chunks (64 values of 32 rows and of the 16 queries), R - 1 in flight, across the tiles: no drain
+// between them, and no last round in which few waves still have a tile.  Lane (j, g) = (lane % 16,
+// lane / 16) loads 16 halves at 64c + 16g of row j of each 16-row block and of query j; MFMA u of a
+// chunk takes halves 8u .. 8u + 7 of them, and lane (j, g) gets query j against rows 16b + 4g + v in
+// acc[b][v].
+// Passes are staged per query in the wave's LDS and appended at the stretch's end or when a query's
+// stage could overflow: the threshold lets through a few rows of most tiles, and one atomic per tile
+// and lane on the few counters of a small batch was the bound (36,000 pairs of a tile and a query, 4
+// passes each).  A tile's norms are requested a tile ahead, before the loads in flight.
+// 1M x 768, 16 queries, 16 of 1,024 lists (687 MB of rows): tiles of 128 rows dealt out in turn, one
+// chunk in flight and an atomic per lane and tile, 238 us and 41 for the sample; now 139 (4.9 TB/s) and
+// 13.  (The ring without the stages: 271 and 25.)
 __global__ __launch_bounds__(256, 2) void ivf16_narrow_kernel(Ivf16Args a) {
-    __shared__ __attribute__((aligned(16))) float2 xs_all[iv16::WAVES][iv16::TN];
-    // a tile's 32 values per lane, kept for its appends ([b][lane]: conflict-free 16-byte accesses)
-    __shared__ __attribute__((aligned(16))) f32x4s dump_all[iv16::WAVES][8 * 64];
+    constexpr int R = 6;
+    __shared__ __attribute__((aligned(16))) float2 xs_all[iv16::WAVES][iv16::NTN];
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
     float2* xs = xs_all[wave];
-    f32x4s* dump = dump_all[wave];
     const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
     const uint32_t total = a.plan.pre[a.plan.C];
-    const uint32_t stride = gridDim.x * iv16::WAVES;
-    uint32_t t = blockIdx.x * iv16::WAVES + uint32_t(wave);
-    if (t >= total) return;
-    const uint32_t rowb = a.Dp * 2u;
-    const uint32_t nch = a.Dp / 64, nce = (nch + 1) & ~1u;
-    const uint32_t lo = uint32_t(j) * rowb + 32u * uint32_t(g);
+    const uint64_t nw = uint64_t(gridDim.x) * iv16::WAVES, w = uint64_t(blockIdx.x) * iv16::WAVES + uint32_t(wave);
+    uint32_t t = uint32_t(total * w / nw);
+    const uint32_t tend = uint32_t(total * (w + 1) / nw);
+    const uint32_t rowb = a.Dp * 2u, nch = a.Dp / 64;
+    // tiles of a stretch: every byte offset within it stays below 2^30
+    const uint32_t most = max(1u, 0x40000000u / (rowb * iv16::NTN));
+    struct Slot {
+        h8v q[2], r[2][2];
+    };
+    Slot ring[R];
+    f32x4s acc[2];
+    // the staged passes of query j: stage[j][0 .. n), n in its four lanes
+    constexpr uint32_t CAP = 2 * iv16::NTN;  // (a tile adds at most NTN)
+    __shared__ float2 stage_all[iv16::WAVES][16][CAP];  // {unscaled dot, position}
+    float2(*stage)[CAP] = stage_all[wave];
+    uint32_t n = 0;
+    auto flush = [&](uint32_t qi) {
+        uint32_t base = 0;
+        if (g == 0 && n) base = atomicAdd(a.cnt + qi, n);
+        base = uint32_t(__shfl(int(base), j));
+        const int64_t ob = int64_t(qi) * a.cap;
+        __builtin_amdgcn_wave_barrier();  // (one wave's LDS accesses are in order)
+        for (uint32_t i = uint32_t(g); i < n; i += 4)
+            if (base + i < a.cap) {
+                const float2 e = stage[j][i];
+                a.cand_dot[ob + base + i] = e.x;
+                a.cand_pos[ob + base + i] = __float_as_uint(e.y);
+            }
+        __builtin_amdgcn_wave_barrier();
+        n = 0;
+    };
     uint32_t h = 0;  // the list of the wave's last located tile
-    auto setup = [&](uint32_t tt, NarrowTile& T) {
-        T.valid = tt < total;
-        if (!T.valid) {
-            // no tile: a zero-length descriptor (every row load out of range); the query loads
-            // (of query 0) are zeroed by the mask
-            T.qs = T.qc = T.rs = T.rc = T.qi = 0;
-            T.xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(a.xh), 0, 0, 0x00020000);
-            return;
-        }
-        h = plan_tile_wave(a.plan, tt, h, 16, iv16::TN, T.qs, T.qc, T.rs, T.rc);
-        T.qi = a.qrow[T.qs + (uint32_t(j) < T.qc ? uint32_t(j) : 0u)];
-        T.xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(a.xh + int64_t(T.rs) * a.Dp), 0,
-                                                 int(T.rc * rowb), 0x00020000);
-    };
-    // chunk c of tile T (c past the last chunk, or an invalid tile: zeros, no memory traffic)
-    auto load = [&](const NarrowTile& T, uint32_t c, h8v(&q2)[2], h8v(&r2)[8][2]) {
-        const bool in = T.valid && c < nch;
-        const bool qv = uint32_t(j) < T.qc && in;
-        const uint32_t k = in ? 64u * c : 0u;
-        const _Float16* qp = a.qh + int64_t(T.qi) * a.Dp + 16 * g + k;
-        q2[0] = masked_h8(qp, qv);
-        q2[1] = masked_h8(qp + 8, qv);
-        const uint32_t vo = in ? lo + 2u * k : 0x80000000u;
+    while (t < tend) {
+        uint32_t qs, qc, rs, rc;
+        h = plan_tile_wave(a.plan, t, h, 16, iv16::NTN, qs, qc, rs, rc);
+        // the stretch: the wave's tiles of this list from t on (one query block: consecutive rows)
+        const uint32_t ntile = min(min(tend, a.plan.pre[h + 1]) - t, most);
+        const uint32_t l0 = a.plan.roff[h], len = a.plan.roff[h + 1] - l0;
+        const uint32_t rows = min(ntile * iv16::NTN, l0 + (a.plan.sample ? ivf_sample_rows(len) : len) - rs);
+        t += ntile;
+        const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<_Float16*>(a.xh + int64_t(rs) * a.Dp), 0, int(rows * rowb), 0x00020000);
+        // (lanes past qc compute the stretch's first query again; their values are not looked at)
+        const uint32_t qi = a.qrow[qs + (uint32_t(j) < qc ? uint32_t(j) : 0u)];
+        const _Float16* const qp = a.qh + int64_t(qi) * a.Dp + 16 * g;
+        const float4 inf = a.qinfo[qi];
+        const PreTestV pt = pretest_v(a.bnd, inf.x, inf.y, a.qerr[qi], inf.z, a.thr ? a.thr[qi] : 0xFFFFFFFFu);
+        // the next chunk of the stretch (past its end: zeros, no memory traffic but the queries')
+        uint32_t lt = 0, lk = 0, lo = uint32_t(j) * rowb + 32u * uint32_t(g);
+        auto load = [&](Slot& s) {
+            const uint32_t vo = lt < ntile ? lo + 128u * lk : 0x80000000u;
 #pragma unroll
-        for (int b = 0; b < 8; ++b)
+            for (int u = 0; u < 2; ++u) s.q[u] = *reinterpret_cast<const h8v*>(qp + 64u * lk + 8 * u);
 #pragma unroll
-            for (int u = 0; u < 2; ++u)
-                r2[b][u] = __builtin_bit_cast(
-                    h8v, __builtin_amdgcn_raw_buffer_load_b128(T.xr, vo + uint32_t(b) * 16u * rowb + 16u * uint32_t(u), 0, 0));
-    };
-    f32x4s acc[8];
-    auto compute = [&](const h8v(&q2)[2], const h8v(&r2)[8][2]) {
+            for (int b = 0; b < 2; ++b)
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int b = 0; b < 8; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(r2[b][u], q2[u], acc[b], 0, 0, 0);
-    };
-    // The appends of a tile wait for their atomic's result, and the wait for a returning atomic
-    // also waits for every load issued before it (the next tile's chunk 0, in flight during the
-    // epilogue), so they run one tile late: the epilogue keeps the tile's values in LDS and issues
-    // the atomic; the stores follow at the next tile's first chunk step, where chunk 0 is due.
-    uint32_t p_mask = 0, p_qi = 0, p_rs = 0, p_pos = 0;
-    float p_inv = 0.0f;
-    const float* dumpf = reinterpret_cast<const float*>(dump);
-    auto flush = [&]() {
-        if (!__ballot(p_mask != 0u)) return;
-        uint32_t pos = p_pos, m = p_mask;
-        const int64_t ob = int64_t(p_qi) * a.cap;
-        while (m && pos < a.cap) {
-            const uint32_t tt = uint32_t(__builtin_ctz(m));  // value tt = 4 b + v: row 16 b + 4 g + v
-            m &= m - 1;
-            a.cand_dot[ob + pos] = dumpf[((tt >> 2) * 64 + uint32_t(lane)) * 4 + (tt & 3)] * p_inv;
-            a.cand_pos[ob + pos] = p_rs + 16 * (tt >> 2) + 4 * uint32_t(g) + (tt & 3);
-            ++pos;
-        }
-        p_mask = 0;
-    };
-    NarrowTile cur, nxt;
-    setup(t, cur);
-    h8v qa[2], qb[2], ra[8][2], rb[8][2];
-    load(cur, 0, qa, ra);
-    while (true) {
-        // this tile's epilogue inputs, used after its main loop
-        const float2 xn0 = uint32_t(lane) < cur.rc ? a.xn[cur.rs + uint32_t(lane)] : make_float2(0.0f, 0.0f);
-        const float2 xn1 = uint32_t(64 + lane) < cur.rc ? a.xn[cur.rs + 64u + uint32_t(lane)] : make_float2(0.0f, 0.0f);
-        const float4 inf = a.qinfo[cur.qi];
-        const float eq = a.qerr[cur.qi];
-        const uint32_t th = a.thr ? a.thr[cur.qi] : 0xFFFFFFFFu;
-#pragma unroll
-        for (int b = 0; b < 8; ++b) acc[b] = f32x4s{0.f, 0.f, 0.f, 0.f};
-        // an even number of chunks (one of zeros when nch is odd), so the next tile's chunk 0
-        // always lands in the first register set
-        for (uint32_t c = 0; c < nce; c += 2) {
-            if (c == 0) flush();  // the previous tile's appends (chunk 0, older than their atomic, is due now)
-            load(cur, c + 1, qb, rb);
-            compute(qa, ra);
-            __builtin_amdgcn_sched_barrier(0);
-            // the next tile (its chunk 0 is requested during this tile's last step), located while
-            // chunk 1 is in flight: the lookup's waits also wait for chunk 1, which is due next
-            if (c == 0) setup(t + stride, nxt);
-            if (c + 2 < nce) load(cur, c + 2, qa, ra);
-            else load(nxt, 0, qa, ra);
-            compute(qb, rb);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        // ---- epilogue of this tile (the next tile's chunk 0 in flight)
-        xs[lane] = xn0;
-        xs[64 + lane] = xn1;  // (read back by this wave only: in order, no barrier)
-        if (uint32_t(j) < cur.qc) {
-            const PreTestV pt = pretest_v(a.bnd, inf.x, inf.y, eq, inf.z, th);
+                for (int u = 0; u < 2; ++u)
+                    s.r[b][u] = __builtin_bit_cast(
+                        h8v, __builtin_amdgcn_raw_buffer_load_b128(xr, vo + uint32_t(b) * 16u * rowb + 16u * uint32_t(u), 0, 0));
+            if (++lk == nch) {
+                lk = 0;
+                ++lt;
+                lo += iv16::NTN * rowb;
+            }
+        };
+        uint32_t tile = 0, k = 0;
+        float2 xn = uint32_t(lane & 31) < rows ? a.xn[rs + uint32_t(lane & 31)] : make_float2(0.0f, 0.0f);
+        auto epilogue = [&]() {
+            const uint32_t r0 = tile * iv16::NTN;
+            if (lane < 32) xs[lane] = xn;  // (read back by this wave only: in order, no barrier)
             uint32_t mask = 0;
 #pragma unroll
-            for (int b = 0; b < 8; ++b) {
+            for (int b = 0; b < 2; ++b)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const uint32_t row = uint32_t(16 * b + 4 * g + v);
                     float xxp, nxp, exp;
                     screen_norms(xs[row], xxp, nxp, exp);
-                    mask |= uint32_t((row < cur.rc) & !(acc[b][v] < pretest_rhs(pt, xxp, nxp, exp))) << (4 * b + v);
+                    mask |= uint32_t((r0 + row < rows) & !(acc[b][v] < pretest_rhs(pt, xxp, nxp, exp))) << (4 * b + v);
                 }
-            }
-            if (mask) {
+            if (uint32_t(j) >= qc) mask = 0;
+            if (__ballot(mask != 0u)) {
+                // places within the query's stage: its four lanes in order
+                const uint32_t c = uint32_t(__popc(mask));
+                const uint32_t c16 = uint32_t(__shfl_xor(int(c), 16)), pair = c + c16;
+                const uint32_t other = uint32_t(__shfl_xor(int(pair), 32));
+                uint32_t pos = n + (g & 1 ? c16 : 0u) + (g & 2 ? other : 0u);
+                n += pair + other;
 #pragma unroll
-                for (int b = 0; b < 8; ++b) dump[b * 64 + lane] = acc[b];
-                p_pos = atomicAdd(a.cnt + cur.qi, uint32_t(__popc(mask)));  // (awaited in flush)
-                p_mask = mask;
-                p_qi = cur.qi;
-                p_rs = cur.rs;
-                p_inv = inf.z;
+                for (int i = 0; i < 8; ++i)  // value i = 4 b + v: row 16 b + 4 g + v
+                    if ((mask >> i) & 1u)
+                        stage[j][pos++] = make_float2(acc[i >> 2][i & 3] * inf.z,
+                                                      __uint_as_float(rs + r0 + 16u * (i >> 2) + 4u * uint32_t(g) + (i & 3)));
+                if (__ballot(n > CAP - iv16::NTN)) flush(qi);
+            }
+            const uint32_t rn = r0 + iv16::NTN + uint32_t(lane & 31);
+            xn = rn < rows ? a.xn[rs + rn] : make_float2(0.0f, 0.0f);
+        };
+        acc[0] = acc[1] = f32x4s{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int r = 0; r < R - 1; ++r) load(ring[r]);
+        while (tile < ntile) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                load(ring[(r + R - 1) % R]);
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int b = 0; b < 2; ++b)
+                        acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ring[r].r[b][u], ring[r].q[u], acc[b], 0, 0, 0);
+                if (++k == nch) {
+                    if (tile < ntile) epilogue();  // (past the end: steps of zeros up to a whole ring)
+                    ++tile;
+                    k = 0;
+                    acc[0] = acc[1] = f32x4s{0.f, 0.f, 0.f, 0.f};
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (!nxt.valid) break;
-        t += stride;
-        cur = nxt;
+        if (__ballot(n != 0u)) flush(qi);
     }
-    flush();  // the last tile's appends
 }
 
 template <int W>
@@ -1465,7 +1462,7 @@ __device__ inline void plan_tiles(const DevPlan& p, int pass, uint32_t nq, uint3
     if (p.screen) {
         g = iv16::group_of(nq);
         TQ = iv16::group_tq(g);
-        TN = iv16::TN;
+        TN = g == 0 ? iv16::NTN : iv16::TN;
         if (pass == 1 && p.big_tq && nq > ivb::kMinQueries) {
             g = 3;
             TN = p.big_tn;
@@ -2120,7 +2117,7 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     band.out_kth = thr;
     VA_CHECK_STATUS(launch_band(cap_s));
     band.out_kth = nullptr;
-    // ---- 2. screen, 3. U_q and the rerank lists (overflowed queries are listed) ---------------------------------------
+    // ---- 2. screen, 3. U_q and the rerank lists (overflowed queries are listed) ------------------
     cnt = cnt2 + Q;
     a.cnt = cnt;
     a.thr = thr;
