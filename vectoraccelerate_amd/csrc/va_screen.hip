@@ -10,12 +10,13 @@
 //               interval [lo, hi] that provably contains the fp32 scan's key s for that pair;
 //               tau_q = k-th smallest hi, so the true k-th key s_k <= tau_q.  With a checked
 //               rank r < k (step 5 verifies the threshold, so any tau_q is safe) the sample
-//               keeps only the smallest approximate hi of each 32-row group and tau_q is the
-//               r-th smallest of those;
-//   3. screen:  the full pass appends (hi, lo, id) for every pair with lo <= tau_q (every row
+//               keeps only the smallest (approximate) hi of each group of 4 to 32 rows and tau_q
+//               is the r-th smallest of those;
+//   3. screen:  the full pass appends (dot, |x|^2, id) for every pair with lo <= tau_q (every row
 //               with s <= s_k is among them);
-//   4. bound:   U_q = k-th smallest hi among the candidates (>= s_k again);
-//   5. compact: the rows with lo <= U_q (a superset of the fp32 top-k, ~k + a thin band);
+//   4. band:    U_q = k-th smallest hi among the candidates (>= s_k again);
+//   5.          the rows with lo <= U_q (a superset of the fp32 top-k, ~k + a thin band), in the
+//               same kernel (va_band.hpp);
 //   6. rerank:  the fp32 distance kernel (the same kernel, k order and epilogue as the fp32
 //               scan, so the same bits) computes the exact keys of those rows;
 //   7. select:  exact (key, id) top-k.  Lists that overflow take the exact chunked path.
@@ -1665,7 +1666,7 @@ va_status screened_topk_scan(va_context* ctx, const ScreenInput& in, KeyProducer
     const ScanPlan plan = screen_plan(ctx, in, k);
     const uint64_t S = plan.S;
     const uint64_t cap = plan.cap;
-    // the threshold: the sample's rank-th smallest upper bound (checked in the compaction when
+    // the threshold: the sample's rank-th smallest upper bound (checked in the band kernel when
     // rank < k)
     const uint32_t rank = sample_rank(ctx, k, S, N, out.skip != nullptr);
     // rerank capacity: k plus the band of rows whose interval straddles the k-th bound (the
