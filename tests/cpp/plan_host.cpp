@@ -115,6 +115,32 @@ int main() {
         }
     }
 
+    // the segments of a dense row: they cover it without a gap, and none begins at or past its end
+    // (the floor of n over the least length, kept as the count, leaves such segments past 4096^2 keys)
+    {
+        std::vector<uint32_t> lens = {1, 8192, 8193, 12288, 12289, 100003, 16777216, 16777217, 16789504, 16789505,
+                                      20480001, 30000000, 50000000, 100000000, 0xFFFFFFFEu, 0xFFFFFFFFu};
+        uint64_t r = 12345;
+        for (int i = 0; i < 20000; ++i) {
+            r = r * 6364136223846793005ull + 1442695040888963407ull;
+            lens.push_back(uint32_t(std::exp(9.0 + 13.18 * double(r >> 40) / double(1 << 24))));
+        }
+        for (uint32_t n : lens)
+            for (uint32_t k : ks) {
+                const SegmentPlan s = select_segments(n, k);
+                CHECK(u128(select_scratch(n, k)) == u128(s.n) * k, "select_scratch n=%u k=%u", n, k);
+                if (n <= kSegRow) CHECK(s.n == 0, "short row cut n=%u", n);
+                if (s.n <= 1) {
+                    CHECK(s.n == 0 && n / std::max(kSegKeys, 16u * k) <= 1 + (n <= kSegRow), "uncut row n=%u k=%u", n, k);
+                    continue;
+                }
+                CHECK(u128(s.n - 1) * s.len < n, "a segment past the row: n=%u k=%u nseg=%u len=%u", n, k, s.n, s.len);
+                CHECK(u128(s.n) * s.len >= n, "row not covered: n=%u k=%u", n, k);
+                CHECK(s.len >= std::max(kSegKeys, 16u * k) && u128(s.n) * k * 16 <= n, "segment length n=%u k=%u", n, k);
+                CHECK(u128(s.n) * k <= 0xFFFFFFFFu, "winners of a row n=%u k=%u", n, k);
+            }
+    }
+
     // device fallback buffers
     for (uint32_t N : Ns)
         for (uint32_t k : ks)

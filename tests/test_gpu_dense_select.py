@@ -50,6 +50,23 @@ def test_select_rows(ctx, oracle, rows, n, k, kind, mode):
     np.testing.assert_array_equal(np.where(gv[:, :kk] == 0, 0, gv[:, :kk]), np.where(ov[:, :kk] == 0, 0, ov[:, :kk]))
 
 
+@pytest.mark.parametrize("rows,n,k", [(1, 16_789_505, 10), (2, 20_480_001, 10), (1, 20_480_001, 1024)])
+def test_select_rows_of_many_segments(ctx, oracle, rows, n, k):
+    """Rows past 4096^2 values, where the segments' length rounds up enough that one fewer covers the
+    row.  The winners lie at both ends, and the rows differ there: values read from beyond a row, or
+    winners counted twice, would be among the results."""
+    g = np.random.default_rng(n)
+    v = np.tile(g.random((1, 1 << 20), dtype=np.float32), (rows, n // (1 << 20) + 1))[:, :n].copy()
+    half = min(k, 40) // 2
+    for r in range(rows):
+        v[r, :half] = -1.0 - 3.0 * r - np.arange(half, dtype=np.float32) / 64
+        v[r, n - half:] = -2.0 - 3.0 * r - np.arange(half, dtype=np.float32) / 64
+    gi, gv = _select(ctx, v, k, 0)
+    oi, ov = oracle.topk_rows(v, k)
+    np.testing.assert_array_equal(gi, oi)
+    np.testing.assert_array_equal(gv, ov)
+
+
 @pytest.mark.parametrize("metric", [L2SQ, COSINE, DOT, L2])
 @pytest.mark.parametrize("Q,N,D", [(1, 1, 1), (1, 31, 3), (2, 32, 15), (31, 33, 16), (32, 95, 17), (33, 127, 32), (5, 129, 36),
                                    (40, 200, 48), (3, 97, 100), (65, 64, 127), (1, 300, 128), (17, 161, 130), (100, 250, 260)])

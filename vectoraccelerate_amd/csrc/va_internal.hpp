@@ -489,7 +489,8 @@ struct SelectArgs {
     // every key is below 2^key_bits (Hamming distances: a few bits)
     uint32_t key_bits = 32;
     // segmented rows (dense keys only): selection row r takes keys [seg (r % nseg), + seg) of dense
-    // row r / nseg; `rows` counts segments, ids are columns of the dense row
+    // row r / nseg; `rows` counts segments, ids are columns of the dense row; every segment begins
+    // within the row (select_segments)
     uint32_t seg = 0, nseg = 0;
     // cleared on the side, so that the scan behind a threshold selection needs no fill launch:
     // zero_cnt[row] and the kZeroWords words at zero_words (by row 0)
@@ -501,10 +502,6 @@ struct SelectArgs {
 constexpr uint32_t kZeroWords = 64;
 constexpr uint32_t kFbSync = 8;
 va_status launch_select(va_context* ctx, const SelectArgs& a);
-// Segments of each row in launch_select_dense, and the (key, id) pairs of scratch it needs per row
-// (0 and 0: one workgroup selects the row).
-uint32_t select_segments(uint32_t n, uint32_t k);
-inline uint64_t select_scratch(uint32_t n, uint32_t k) { return uint64_t(select_segments(n, k)) * k; }
 // Top-k of dense rows whose winners per segment go through wkey / wid (select_scratch(n, k) words
 // per row each; unused with one segment).
 va_status launch_select_dense(va_context* ctx, const SelectArgs& a, uint32_t* wkey, uint32_t* wid);

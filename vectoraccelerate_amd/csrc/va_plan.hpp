@@ -72,6 +72,29 @@ inline uint32_t sample_rank_for(uint64_t opt_rank, uint32_t k, uint64_t S, uint3
     return r;
 }
 
+// ---- the segments of a long dense row (va_select.hip) ------------------------------------------
+// A long row is bound by its one workgroup: the passes over the row are serial, and a batch of few
+// queries leaves most of the chip idle.  Rows past kSegRow keys are cut into segments of at least
+// kSegKeys keys (16 k for large k, so that the winners are a small part of the row), each segment's
+// top-k selected by a workgroup of its own and the winners merged (20,000 keys, one query: 31 ->
+// 12 us; a whole search of 49,999 x 300, Q = 37 138 -> 59 us with the dense path).
+constexpr uint32_t kSegRow = 8192, kSegKeys = 4096;
+struct SegmentPlan {
+    uint32_t n = 0;    // segments (0 or 1: the row is selected whole)
+    uint32_t len = 0;  // keys of each; the last segment takes what is left, at least one key
+};
+// The segments of a row of n keys.  Their count follows from their rounded-up length: the floor of
+// n over the least length would leave segments that begin past the row (n past 4096^2).
+inline SegmentPlan select_segments(uint32_t n, uint32_t k) {
+    if (n <= kSegRow) return {};
+    const uint32_t want = n / std::max<uint32_t>(kSegKeys, 16u * k);
+    if (want <= 1) return {};
+    const uint32_t len = uint32_t((uint64_t(n) + want - 1) / want);
+    return {uint32_t((uint64_t(n) + len - 1) / len), len};
+}
+// (key, id) pairs of scratch per row (0: no segments)
+inline uint64_t select_scratch(uint32_t n, uint32_t k) { return uint64_t(select_segments(n, k).n) * k; }
+
 // ---- the device fallback (va_fallback.hpp) ------------------------------------------------------
 constexpr int kFbPasses = 5;
 constexpr uint32_t kFbGrid = 1024;  // workgroups per pass (4 waves each)

@@ -99,28 +99,17 @@ va_status launch_select(va_context* ctx, const SelectArgs& a) {
     return VA_OK;
 }
 
-// A long row is bound by its one workgroup: the passes over the row are serial, and a batch of few
-// queries leaves most of the chip idle.  Rows past kSegRow keys are cut into segments of at least
-// kSegKeys keys (16 k for large k, so that the winners are a small part of the row), each segment's
-// top-k selected by a workgroup of its own and the winners merged (20,000 keys, one query: 31 ->
-// 12 us; a whole search of 49,999 x 300, Q = 37 138 -> 59 us with the dense path).
-constexpr uint32_t kSegRow = 8192, kSegKeys = 4096;
-uint32_t select_segments(uint32_t n, uint32_t k) {
-    if (n <= kSegRow) return 0;
-    return n / std::max(kSegKeys, 16u * k);
-}
-
 va_status launch_select_dense(va_context* ctx, const SelectArgs& a, uint32_t* wkey, uint32_t* wid) {
-    const uint32_t nseg = select_segments(a.n, a.k);
-    if (nseg <= 1) return launch_select(ctx, a);
+    const SegmentPlan seg = select_segments(a.n, a.k);
+    if (seg.n <= 1) return launch_select(ctx, a);
     SelectArgs p;
     p.keys = a.keys;
     p.ld = a.ld;
     p.n = a.n;
-    p.rows = a.rows * nseg;
+    p.rows = a.rows * seg.n;
     p.k = a.k;
-    p.seg = (a.n + nseg - 1) / nseg;
-    p.nseg = nseg;
+    p.seg = seg.len;
+    p.nseg = seg.n;
     p.key_bits = a.key_bits;
     p.out_idx = wid;
     p.out_key = wkey;
@@ -128,8 +117,8 @@ va_status launch_select_dense(va_context* ctx, const SelectArgs& a, uint32_t* wk
     SelectArgs m = a;
     m.keys = wkey;
     m.ids = wid;
-    m.ld = int64_t(nseg) * a.k;
-    m.n = nseg * a.k;
+    m.ld = int64_t(seg.n) * a.k;
+    m.n = seg.n * a.k;
     return launch_select(ctx, m);
 }
 
