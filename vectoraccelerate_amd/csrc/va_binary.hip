@@ -183,15 +183,16 @@ __global__ __launch_bounds__(256) void hamming_scan_wide_kernel(HamArgs a) {
 namespace hmf {
 constexpr int NW = 8, WR = 32, TN = NW * WR;
 constexpr int PA = NW * WR * 4;  // per-wave row popcounts
-// staged passes per wave: fewer where a smaller tile then fits two workgroups per CU
-constexpr int lcap(int NB) { return NB == 8 ? 80 : 48; }
-constexpr int stage(int NB) { return NW * lcap(NB) * 12; }
+// Staged passes per wave, {query in the tile, distance} and row id: two words each, so that 128
+// queries of 24 words still fit two workgroups per CU.  One append stages up to a whole wave's passes.
+constexpr int LCAP = 80, STAGE = NW * LCAP * 8;
+static_assert(LCAP >= 64, "a flush must leave room for a whole wave's passes");
 // resident queries, chunk-major: 16-byte chunk c (of W) of query r of 32 NB at c * 512 NB + r * 16, so
 // the fragments of all query blocks of one k-step lie within a 16-bit DS offset of one address
 constexpr int qbytes(int W, int NB) { return 32 * NB * 16 * W; }
 constexpr int rows_bytes(int W) { return NW * WR * (W + 1) * 4; }  // per-wave row words, rows W + 1 apart
 constexpr size_t lds_bytes(int W, int NB) {
-    return size_t(qbytes(W, NB)) + stage(NB) + PA + 32 * NB * 4 + rows_bytes(W);
+    return size_t(qbytes(W, NB)) + STAGE + PA + 32 * NB * 4 + rows_bytes(W);
 }
 }  // namespace hmf
 
@@ -220,7 +221,7 @@ template <int W, int NB>
 __global__ __launch_bounds__(512, NB == 8 ? 2 : 4) void hamming_mfma_kernel(HamArgs a, uint32_t R) {
     using namespace hmf;
     constexpr int HW = W / 2;  // words per lane half = k-steps per tile
-    constexpr int TQ = 32 * NB, QB = qbytes(W, NB), STAGE = stage(NB), PB = TQ * 4, LCAP = lcap(NB);
+    constexpr int TQ = 32 * NB, QB = qbytes(W, NB), PB = TQ * 4;
     constexpr int CS = TQ * 16;  // bytes per chunk of all resident queries
     extern __shared__ __attribute__((aligned(16))) char lds8[];
     const int tid = threadIdx.x;
@@ -305,18 +306,18 @@ __global__ __launch_bounds__(512, NB == 8 ? 2 : 4) void hamming_mfma_kernel(HamA
     auto rd_q = [&](int st, int u) { return *reinterpret_cast<const i32x4h*>(qrd + qz + st * (2 * CS) + u * 512); };
 
     // ---- filter epilogue ------------------------------------------------------------------
-    uint32_t* s_qi = reinterpret_cast<uint32_t*>(lds8 + QB) + wave * 3 * LCAP;
-    uint32_t* s_key = s_qi + LCAP;
-    uint32_t* s_id = s_key + LCAP;
+    uint32_t* s_qk = reinterpret_cast<uint32_t*>(lds8 + QB) + wave * 2 * LCAP;  // query | distance << 8
+    uint32_t* s_id = s_qk + LCAP;
+    static_assert(TQ <= 256, "a staged pass holds its query in a byte");
     uint32_t lc = 0;  // staged passes (wave-uniform)
     auto flush = [&]() {
         for (uint32_t b0 = 0; b0 < lc; b0 += 64) {
             const uint32_t e = b0 + uint32_t(lane);
             if (e < lc) {
-                const uint32_t qi = s_qi[e];
+                const uint32_t qk = s_qk[e], qi = q0 + (qk & 255u);
                 const uint32_t pos = atomicAdd(a.cnt + qi, 1u);
                 if (pos < a.cap) {
-                    a.cand_key[int64_t(qi) * a.cap + pos] = s_key[e];
+                    a.cand_key[int64_t(qi) * a.cap + pos] = qk >> 8;
                     a.cand_id[int64_t(qi) * a.cap + pos] = s_id[e];
                 }
             }
@@ -351,8 +352,7 @@ __global__ __launch_bounds__(512, NB == 8 ? 2 : 4) void hamming_mfma_kernel(HamA
             if (p) {
                 const uint32_t e =
                     lc + __builtin_amdgcn_mbcnt_hi(uint32_t(mk >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(mk), 0u));
-                s_qi[e] = q0 + ql;
-                s_key[e] = uint32_t(s_pb[ql] + 1024.0f - 2.0f * sv);  // |q| + |x| - 2 a.b, exact
+                s_qk[e] = ql | uint32_t(s_pb[ql] + 1024.0f - 2.0f * sv) << 8;  // |q| + |x| - 2 a.b, exact
                 s_id[e] = r0 + roff + 4 * uint32_t(hh);
             }
             lc += n;
