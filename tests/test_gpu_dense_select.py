@@ -24,7 +24,11 @@ def _select(ctx, v, k, mode):
 
 
 @pytest.mark.parametrize("rows,n,k", [(1, 8192, 10), (1, 8193, 10), (3, 12289, 1), (2, 100_003, 100), (1, 65_537, 1024),
-                                      (600, 9000, 7), (5, 1500, 129), (4, 128, 128), (2, 40, 60)])
+                                      (600, 9000, 7), (5, 1500, 129), (4, 128, 128), (2, 40, 60),
+                                      # the lowest id among the ties of the smallest key; rows read from
+                                      # memory, cut (k = 32) and whole (more of them than half the CUs)
+                                      (3, 100, 1), (140, 26_000, 1), (140, 26_000, 32), (140, 26_000, 33),
+                                      (140, 9000, 33), (400, 17_000, 300)])
 @pytest.mark.parametrize("kind", ["spread", "ties", "crowded"])
 @pytest.mark.parametrize("mode", [0, 1])
 def test_select_rows(ctx, oracle, rows, n, k, kind, mode):

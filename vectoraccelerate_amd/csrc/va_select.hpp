@@ -80,8 +80,8 @@ __device__ inline void find_bin_wide(const uint32_t* hist, uint32_t nb, uint32_t
 
 // Adds this lane's item to bin d of the histogram when m.  Keys of one search crowd into few bins
 // (ties, excluded rows, Hamming distances), and 64 lanes incrementing one LDS word serialise: the
-// bins of the first two lanes still waiting are each added once for all lanes that share them, the
-// rest one by one.
+// bin of the first lane, and where eight lanes or more share it that of the first one left, are each
+// added once for all lanes that share them, the rest one by one.
 __device__ __forceinline__ void hist_add(uint32_t* hist, bool m, uint32_t d) {
     uint64_t rest = __ballot(m);
     const uint32_t lane = threadIdx.x & 63;
@@ -93,8 +93,36 @@ __device__ __forceinline__ void hist_add(uint32_t* hist, bool m, uint32_t d) {
         const uint64_t same = __ballot(m && d == f) & rest;
         if (lane == uint32_t(l)) atomicAdd(&hist[f], uint32_t(__popcll(same)));
         rest &= ~same;
+        if (__popcll(same) < 8) break;
     }
     if ((rest >> lane) & 1ull) atomicAdd(&hist[d], 1u);
+}
+
+// The need-th smallest of the few <= SEL_FEW values in lds.whist; need and eq as radix_kth's.  (The
+// loop's reads are independent: unrolled, they are not one LDS latency each.)
+__device__ inline uint32_t kth_of_few(RadixLds& lds, uint32_t few, uint32_t& need, uint32_t& eq) {
+    const uint32_t tid = threadIdx.x, want = need;
+    if (tid < few) {
+        const uint32_t v = lds.whist[tid];
+        uint32_t below = 0, same = 0;
+#pragma unroll 8
+        for (uint32_t j = 0; j < few; ++j) {
+            const uint32_t o = lds.whist[j];
+            below += o < v;
+            same += o == v;
+        }
+        if (below < want && want <= below + same) {  // (every item equal to the answer writes the same)
+            lds.lo = v;
+            lds.before = below;
+            lds.bin = same;
+        }
+    }
+    __syncthreads();
+    const uint32_t t = lds.lo;
+    need = want - lds.before;
+    eq = lds.bin;
+    __syncthreads();
+    return t;
 }
 
 // The need-th smallest value of the items for_vals(f) runs f(value, taken) over, all within
@@ -134,27 +162,7 @@ __device__ inline uint32_t radix_kth(RadixLds& lds, ForVals&& for_vals, uint32_t
                 if (taken && ((v - base) >> left) == prefix) lds.whist[atomicAdd(&lds.cnt, 1u)] = v;
             });
             __syncthreads();
-            const uint32_t few = eq, want = need;
-            if (uint32_t(tid) < few) {
-                const uint32_t v = lds.whist[tid];
-                uint32_t below = 0, same = 0;
-                for (uint32_t j = 0; j < few; ++j) {
-                    const uint32_t o = lds.whist[j];
-                    below += o < v;
-                    same += o == v;
-                }
-                if (below < want && want <= below + same) {  // (every item equal to the answer writes the same)
-                    lds.lo = v;
-                    lds.before = below;
-                    lds.bin = same;
-                }
-            }
-            __syncthreads();
-            const uint32_t t = lds.lo;
-            need = want - lds.before;
-            eq = lds.bin;
-            __syncthreads();
-            return t;
+            return kth_of_few(lds, eq, need, eq);
         }
     }
     return base + prefix;
@@ -162,7 +170,8 @@ __device__ inline uint32_t radix_kth(RadixLds& lds, ForVals&& for_vals, uint32_t
 
 // The need-th smallest key of for_keys(f): mn and mx are the smallest and largest of this thread's
 // keys.  The histograms start below the leading bits that all keys share: nearby distances have
-// equal top bits, and bins of those bits alone would count everything in one bin.
+// equal top bits, and bins of those bits alone would count everything in one bin.  The smallest key
+// needs none (eq is then left at "more than one": its ties were not counted).
 template <int NT, class ForKeys>
 __device__ inline uint32_t kth_key(RadixLds& lds, ForKeys&& for_keys, uint32_t mn, uint32_t mx, uint32_t& need,
                                    uint32_t& eq) {
@@ -182,6 +191,10 @@ __device__ inline uint32_t kth_key(RadixLds& lds, ForKeys&& for_keys, uint32_t m
     }
     __syncthreads();
     const uint32_t lo = lds.lo, hi = lds.hi;
+    if (need == 1) {
+        eq = 2;
+        return lo;
+    }
     return radix_kth<NT>(lds, [&](auto&& f) { for_keys([&](uint32_t k) { f(k, true); }); }, lo,
                          hi == lo ? 0u : 32u - uint32_t(__builtin_clz(hi - lo)), need, eq);
 }
@@ -249,7 +262,7 @@ __device__ void select_row(const SelectArgs& a, uint32_t row, SelectLds<KTH>& ld
         __syncthreads();
     }
     const uint32_t K = a.k < n ? a.k : n;
-    // f(key) over the row; rows read from memory load eight keys per thread before using them,
+    // f(key, i) over the row; rows read from memory load eight keys per thread before using them,
     // so a long row's pass is not one load latency per key
     auto for_keys = [&](auto&& f) {
         uint32_t i = uint32_t(tid);
@@ -259,9 +272,9 @@ __device__ void select_row(const SelectArgs& a, uint32_t row, SelectLds<KTH>& ld
 #pragma unroll
                 for (int j = 0; j < 8; ++j) v[j] = rv.key(i + uint32_t(j) * NT);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) f(v[j]);
+                for (int j = 0; j < 8; ++j) f(v[j], i + uint32_t(j) * NT);
             }
-        for (; i < n; i += NT) f(rv.key(i));
+        for (; i < n; i += NT) f(rv.key(i), i);
     };
 
     uint32_t T = 0xFFFFFFFFu, Tid = 0xFFFFFFFFu;
@@ -270,28 +283,47 @@ __device__ void select_row(const SelectArgs& a, uint32_t row, SelectLds<KTH>& ld
         // ---- phase 1: k-th smallest key ---------------------------------------------
         uint32_t need = K, eq = n;
         if (a.key_bits <= SEL_BITS) {
-            T = radix_kth<NT>(lds, [&](auto&& f) { for_keys([&](uint32_t k) { f(k, true); }); }, 0u, a.key_bits, need, eq);
+            T = radix_kth<NT>(lds, [&](auto&& f) { for_keys([&](uint32_t k, uint32_t) { f(k, true); }); }, 0u, a.key_bits,
+                              need, eq);
         } else {
-            if (!CACHED)
-                for_keys([&](uint32_t k) {
+            // A row read from memory: a pass for its keys' range pays where they lie close together (the
+            // winners and candidates of earlier steps); other rows start from the top bits.
+            if (!CACHED && !rv.ids && K > 1) {
+                mn = 0u;
+                mx = 0xFFFFFFFFu;
+            } else if (!CACHED) {
+                for_keys([&](uint32_t k, uint32_t) {
                     mn = min(mn, k);
                     mx = max(mx, k);
                 });
-            T = kth_key<NT>(lds, for_keys, mn, mx, need, eq);
+            }
+            T = kth_key<NT>(lds, [&](auto&& f) { for_keys([&](uint32_t k, uint32_t) { f(k); }); }, mn, mx, need, eq);
         }
         if (KTH || a.out_kth) {
             if (tid == 0) a.out_kth[orow] = T;
             return;
         }
         // ---- phase 2: among key == T take the `need` lowest ids ----------------------
-        if (need < eq)
+        if (need < eq && need == 1) {  // the lowest id
+            for_keys([&](uint32_t k, uint32_t i) {
+                if (k == T) Tid = min(Tid, rv.id(i));
+            });
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) Tid = min(Tid, uint32_t(__shfl_xor(int(Tid), off)));
+            __syncthreads();  // (lds.lo may still be read)
+            if (tid == 0) lds.lo = 0xFFFFFFFFu;
+            __syncthreads();
+            if ((tid & 63) == 0) atomicMin(&lds.lo, Tid);
+            __syncthreads();
+            Tid = lds.lo;
+        } else if (need < eq)
             Tid = radix_kth<NT>(
                 lds,
                 [&](auto&& f) {
-                    for (uint32_t i = tid; i < n; i += NT) {
-                        const bool t = rv.key(i) == T;
+                    for_keys([&](uint32_t k, uint32_t i) {
+                        const bool t = k == T;
                         f(t ? rv.id(i) : 0u, t);
-                    }
+                    });
                 },
                 0u, 32u, need, eq);
     } else if (a.out_kth) {
@@ -304,8 +336,7 @@ __device__ void select_row(const SelectArgs& a, uint32_t row, SelectLds<KTH>& ld
     if constexpr (KTH) return;  // threshold launches always have out_kth (returned above)
     if (tid == 0) s_cnt = 0;
     __syncthreads();
-    for (uint32_t i = tid; i < n; i += NT) {
-        const uint32_t k = rv.key(i);
+    for_keys([&](uint32_t k, uint32_t i) {
         if (take_all || k < T || k == T) {
             const uint32_t id = rv.id(i);
             if (take_all || k < T || id <= Tid) {
@@ -316,7 +347,7 @@ __device__ void select_row(const SelectArgs& a, uint32_t row, SelectLds<KTH>& ld
                 }
             }
         }
-    }
+    });
     __syncthreads();
     const uint32_t cnt = s_cnt < SEL_BUF ? s_cnt : SEL_BUF;
     // slot r of the output: winner (wk, wid), or missing
@@ -337,11 +368,14 @@ __device__ void select_row(const SelectArgs& a, uint32_t row, SelectLds<KTH>& ld
     if (cnt <= SEL_FEW) {
         // few winners: each finds its slot by comparing itself with all of them
         if (uint32_t(tid) < cnt) {
+            // (no branches in the loop: its reads then go out together, not one LDS latency each)
             const uint32_t wk = okey[tid], wid = oid[tid];
+            const uint64_t w = uint64_t(wk) << 32 | wid;
             uint32_t r = 0;
+#pragma unroll 8
             for (uint32_t j = 0; j < cnt; ++j) {
-                const uint32_t kj = okey[j], ij = oid[j];
-                r += kj < wk || (kj == wk && (ij < wid || (ij == wid && j < uint32_t(tid))));
+                const uint64_t o = uint64_t(okey[j]) << 32 | oid[j];
+                r += uint32_t(o < w) + (uint32_t(o == w) & uint32_t(j < uint32_t(tid)));
             }
             if (r < K) put(r, true, wk, wid);
         }
