@@ -127,9 +127,13 @@ int main() {
         }
         for (uint32_t n : lens)
             for (uint32_t k : ks) {
-                const SegmentPlan s = select_segments(n, k);
-                CHECK(u128(select_scratch(n, k)) == u128(s.n) * k, "select_scratch n=%u k=%u", n, k);
+                const SegmentPlan s = select_segments(n, k, 1, 256);
                 if (n <= kSegRow) CHECK(s.n == 0, "short row cut n=%u", n);
+                for (uint32_t rows : {128u, 129u, 100000u}) {  // many rows: the same segments, or none for a large k
+                    const SegmentPlan m = select_segments(n, k, rows, 256);
+                    const bool whole = rows > 128 && k > kSegManyK;
+                    CHECK(whole ? m.n == 0 : m.n == s.n && m.len == s.len, "rows=%u n=%u k=%u", rows, n, k);
+                }
                 if (s.n <= 1) {
                     CHECK(s.n == 0 && n / std::max(kSegKeys, 16u * k) <= 1 + (n <= kSegRow), "uncut row n=%u k=%u", n, k);
                     continue;

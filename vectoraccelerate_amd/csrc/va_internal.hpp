@@ -502,9 +502,10 @@ struct SelectArgs {
 constexpr uint32_t kZeroWords = 64;
 constexpr uint32_t kFbSync = 8;
 va_status launch_select(va_context* ctx, const SelectArgs& a);
-// Top-k of dense rows whose winners per segment go through wkey / wid (select_scratch(n, k) words
-// per row each; unused with one segment).
-va_status launch_select_dense(va_context* ctx, const SelectArgs& a, uint32_t* wkey, uint32_t* wid);
+// Top-k of dense rows, each cut as seg says; the segments' winners go through wkey / wid (seg.n k
+// words per row each).
+va_status launch_select_dense(va_context* ctx, const SelectArgs& a, const SegmentPlan& seg, uint32_t* wkey,
+                              uint32_t* wid);
 
 // assign[i] = the nearest centroid of row i by L2^2 (ties -> lower centroid) on the fp32 MFMA
 // distance kernel with the argmin epilogue; best is N words of scratch

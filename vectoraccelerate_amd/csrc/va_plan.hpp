@@ -77,23 +77,24 @@ inline uint32_t sample_rank_for(uint64_t opt_rank, uint32_t k, uint64_t S, uint3
 // queries leaves most of the chip idle.  Rows past kSegRow keys are cut into segments of at least
 // kSegKeys keys (16 k for large k, so that the winners are a small part of the row), each segment's
 // top-k selected by a workgroup of its own and the winners merged (20,000 keys, one query: 31 ->
-// 12 us; a whole search of 49,999 x 300, Q = 37 138 -> 59 us with the dense path).
-constexpr uint32_t kSegRow = 8192, kSegKeys = 4096;
+// 12 us; a whole search of 49,999 x 300, Q = 37 138 -> 59 us with the dense path).  Rows enough to
+// fill the chip by themselves are cut only for a small k, where the segments' winners cost next to
+// nothing (whole selections, cut / whole: 1,000 rows of 30,000 keys, k = 10 148 / 156 us, 100
+// 202 / 179, 600 351 / 219; 3,000 of 10,000, k = 10 148 / 199; 128 of 120,000, k = 50 104 / 109).
+constexpr uint32_t kSegRow = 8192, kSegKeys = 4096, kSegManyK = 32;
 struct SegmentPlan {
     uint32_t n = 0;    // segments (0 or 1: the row is selected whole)
     uint32_t len = 0;  // keys of each; the last segment takes what is left, at least one key
 };
-// The segments of a row of n keys.  Their count follows from their rounded-up length: the floor of
+// The segments of each of `rows` rows of n keys on cus CUs.  Their count follows from their rounded-up length: the floor of
 // n over the least length would leave segments that begin past the row (n past 4096^2).
-inline SegmentPlan select_segments(uint32_t n, uint32_t k) {
-    if (n <= kSegRow) return {};
+inline SegmentPlan select_segments(uint32_t n, uint32_t k, uint32_t rows, uint32_t cus) {
+    if (n <= kSegRow || (k > kSegManyK && rows > cus / 2)) return {};
     const uint32_t want = n / std::max<uint32_t>(kSegKeys, 16u * k);
     if (want <= 1) return {};
     const uint32_t len = uint32_t((uint64_t(n) + want - 1) / want);
     return {uint32_t((uint64_t(n) + len - 1) / len), len};
 }
-// (key, id) pairs of scratch per row (0: no segments)
-inline uint64_t select_scratch(uint32_t n, uint32_t k) { return uint64_t(select_segments(n, k).n) * k; }
 
 // ---- the device fallback (va_fallback.hpp) ------------------------------------------------------
 constexpr int kFbPasses = 5;

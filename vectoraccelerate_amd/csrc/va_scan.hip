@@ -211,7 +211,8 @@ va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t
         // small database: dense keys in query chunks + select
         const uint64_t per_q = uint64_t(N) * 4;
         uint32_t qc = uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(Q, dense_budget(ctx) / per_q)));
-        const uint64_t win = qc * select_scratch(N, k);  // winners of the rows' segments
+        const SegmentPlan seg = select_segments(N, k, qc, uint32_t(ctx->num_cus));
+        const uint64_t win = uint64_t(qc) * seg.n * k;  // winners of the rows' segments
         Scratch s(ctx);
         VA_CHECK_STATUS(s.reserve(Scratch::round(uint64_t(qc) * per_q) + Scratch::round(win * 4) * 2));
         uint32_t* keys = s.carve<uint32_t>(uint64_t(qc) * N);
@@ -231,7 +232,7 @@ va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t
             if (out.f) a.out_f = out.f + int64_t(q0) * k;
             if (out.i32) a.out_i32 = out.i32 + int64_t(q0) * k;
             if (out.key) a.out_key = out.key + int64_t(q0) * k;
-            VA_CHECK_STATUS(launch_select_dense(ctx, a, wkey, wid));
+            VA_CHECK_STATUS(launch_select_dense(ctx, a, seg, wkey, wid));
         }
         return pm.finish(false, false);
     }

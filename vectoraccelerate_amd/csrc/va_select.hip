@@ -74,9 +74,13 @@ va_status launch_select(va_context* ctx, const SelectArgs& a) {
     if (a.k > SEL_BUF) return fail(ctx, VA_ERR_INVALID_ARG, "k=%u exceeds the maximum %u", a.k, SEL_BUF);
     // Candidate lists are mostly far below their capacity, which sizes the LDS copy: past 8K
     // entries a large copy would leave one workgroup per CU, so such rows are read from memory
-    // (L2-resident lists) by many workgroups at once instead.
+    // (L2-resident lists) by many workgroups at once instead; and so are dense rows of that length
+    // when not all of them would be on the chip at once (1,000 rows of 16,384 keys, k = 600
+    // 321 -> 126 us; 600 of 8,193, which are, 70 from their copies, 78 without).
     const uint32_t n = a.nseg ? a.seg : a.n;
-    const bool cache = n <= kSelCache && !((a.counts || a.out_kth) && n > 8192);
+    constexpr uint32_t kLds = 160 * 1024;
+    const bool resident = a.rows <= uint64_t(ctx->num_cus) * (kLds / (n * 4ull + sizeof(SelectLds<false>)));
+    const bool cache = n <= 8192 || (n <= kSelCache && !a.counts && !a.out_kth && resident);
     const size_t lds = size_t(cache ? std::max<uint32_t>(n, 1) : (a.counts ? kSelList : 0)) * 4;
     auto go = [&](auto kern, int threads) -> va_status {
         if (lds > 48 * 1024)
@@ -99,8 +103,8 @@ va_status launch_select(va_context* ctx, const SelectArgs& a) {
     return VA_OK;
 }
 
-va_status launch_select_dense(va_context* ctx, const SelectArgs& a, uint32_t* wkey, uint32_t* wid) {
-    const SegmentPlan seg = select_segments(a.n, a.k);
+va_status launch_select_dense(va_context* ctx, const SelectArgs& a, const SegmentPlan& seg, uint32_t* wkey,
+                              uint32_t* wid) {
     if (seg.n <= 1) return launch_select(ctx, a);
     SelectArgs p;
     p.keys = a.keys;
@@ -136,7 +140,8 @@ va_status va_topk_select(va_context* ctx, const float* values, uint32_t num_rows
     va::DeviceGuard g(ctx->device);
     const uint64_t total = uint64_t(num_rows) * num_elements;
     va::Scratch s(ctx);
-    const uint64_t win = num_rows * va::select_scratch(num_elements, k);
+    const va::SegmentPlan seg = va::select_segments(num_elements, k, num_rows, uint32_t(ctx->num_cus));
+    const uint64_t win = uint64_t(num_rows) * seg.n * k;
     VA_CHECK_STATUS(s.reserve(va::Scratch::round(total * 4) + va::Scratch::round(win * 4) * 2));
     uint32_t* keys = s.carve<uint32_t>(total);
     uint32_t* wkey = s.carve<uint32_t>(win);
@@ -155,7 +160,7 @@ va_status va_topk_select(va_context* ctx, const float* values, uint32_t num_rows
     a.out_idx = out_idx;
     a.out_f = out_values;
     a.key_kind = mode == VA_SELECT_MAX ? 1 : 0;
-    return va::launch_select_dense(ctx, a, wkey, wid);
+    return va::launch_select_dense(ctx, a, seg, wkey, wid);
 }
 
 va_status va_topk_merge(va_context* ctx, const uint32_t* a_idx, const float* a_dist, const uint32_t* b_idx,
