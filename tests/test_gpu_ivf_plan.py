@@ -1,4 +1,5 @@
-"""The inverted-list search's plan at the edges of its one-launch form (probes, pairs, lists) and of the
+"""The inverted-list search's plan at the edges of its one-launch form (probes, pairs, lists), of its one
+workgroup (with lists that end within the last of several) and of the
 tile groups that a batch can need, long lists shared out among the waves of the 16-query tiles (their
 stages overflow), with the probes a caller may pass (repeated, out of range): against
 the oracle, and the screened scan against the fp32 list scan bit for bit."""
@@ -16,6 +17,8 @@ pytestmark = pytest.mark.gpu
                                               (40, 32, 4000, 32, 8, 5), (40, 32, 4000, 33, 8, 5), (64, 32, 6000, 64, 64, 10),
                                               (65, 32, 6000, 63, 65, 10), (64, 32, 6000, 65, 64, 3),
                                               (8192, 16, 20_000, 5, 20, 10), (8193, 16, 20_000, 5, 20, 10),
+                                              (2048, 16, 20_000, 70, 65, 10), (2049, 16, 20_000, 70, 65, 10),
+                                              (20_001, 16, 60_000, 70, 8, 10), (20_001, 9, 60_000, 500, 9, 10),
                                               (30, 768, 3000, 128, 2, 10), (30, 768, 3000, 129, 2, 10), (5, 33, 700, 9, 3, 10),
                                               (3, 64, 30_000, 4, 2, 100), (2, 128, 70_001, 16, 2, 1)])
 @pytest.mark.parametrize("odd_probes", [False, True])

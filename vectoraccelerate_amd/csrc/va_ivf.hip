@@ -1432,7 +1432,9 @@ struct DevPlan {
     uint32_t* qfill = nullptr;  // [C] fill cursors
     uint32_t* qlist = nullptr;  // [Q x np] (the first qoff[C] are used)
     uint32_t* pre = nullptr;    // [2][kGroups][C + 1]
+    uint32_t* part = nullptr;   // [plan_blocks(C)][kPlanSums] sums of the workgroups' lists
 };
+constexpr int kPlanSums = 2 * kGroups + 1;  // queries, tiles per pass and group
 
 __global__ __launch_bounds__(256) void plan_probes_kernel(DevPlan p) {
     const uint32_t q = blockIdx.x;
@@ -1479,16 +1481,26 @@ __device__ inline void plan_tiles(const DevPlan& p, int pass, uint32_t nq, uint3
     tiles = (nq == 0 || rows == 0) ? 0u : ((nq + TQ - 1) / TQ) * ((rows + TN - 1) / TN);
 }
 
-// The lists' query offsets and every group's tile prefixes, one workgroup: each thread sums its run
-// of lists, one scan of all sums at once (wave shuffles, then the waves' totals), and each thread
-// walks its run again.  ONE (few probes over few lists): the probes are counted before and the query
-// lists filled after, with the counters in LDS, so the whole plan is one launch (six of them took 38 us
-// of a search of 16 queries).
+// The lists' query offsets and every group's tile prefixes: each thread sums its run of lists, one
+// scan of all sums at once (wave shuffles, then the waves' totals), and each thread walks its run
+// again.  PLAN_ONE (few probes over few lists): one workgroup; the probes are counted before and the
+// query lists filled after, with the counters in LDS, so the whole plan is one launch (six of them took
+// 38 us of a search of 16 queries).  Otherwise plan_blocks(C) workgroups take equal runs of lists: with
+// more than one, PLAN_SUMS leaves each one's sums in p.part for the PLAN_LISTS launch behind it.
 constexpr uint32_t kPlanOneLists = 8192, kPlanOnePairs = 4096, kPlanOneProbes = 64;
-template <bool ONE>
+enum PlanMode : int { PLAN_ONE, PLAN_SUMS, PLAN_LISTS };
+// One workgroup up to kPlanBlockLists lists, where it is as fast as the two launches; past that its
+// threads walk many lists each, one after the other.  Whole searches of 500,000 rows, 32 probes, one
+// workgroup / many: 64-d, Q = 129 2,048 lists 195 / 194 us, 4,096 208 / 195, 16,384 339 / 216, 65,536
+// 905 / 280; 65,536 lists, Q = 1 718 / 102, Q = 1,024 1,420 / 800; the fp32 scan (33-d, five tile shapes
+// weighed per list), 65,536 lists, Q = 129 1,180 / 525.
+constexpr uint32_t kPlanBlockLists = 2048;
+inline uint32_t plan_blocks(uint32_t C) { return C <= kPlanBlockLists ? 1u : (C + 1023) / 1024; }
+template <PlanMode MODE>
 __global__ __launch_bounds__(1024) void plan_lists_kernel(DevPlan p) {
-    constexpr int A = 2 * kGroups + 1;
-    __shared__ uint32_t s_tot[16][A];
+    constexpr bool ONE = MODE == PLAN_ONE;
+    constexpr int A = kPlanSums;
+    __shared__ uint32_t s_tot[16][A], s_base[A];
     __shared__ uint32_t s_cnt[ONE ? kPlanOneLists : 1];
     const uint32_t t = threadIdx.x, lane = t & 63, w = t >> 6;
     const uint32_t pairs = p.Q * p.np;  // (ONE: at most kPlanOnePairs)
@@ -1504,8 +1516,9 @@ __global__ __launch_bounds__(1024) void plan_lists_kernel(DevPlan p) {
         }
         __syncthreads();
     }
-    const uint32_t per = (p.C + 1023) / 1024;
-    const uint32_t b0 = min(p.C, t * per), b1 = min(p.C, b0 + per);
+    const uint32_t per = uint32_t((p.C + 1024ull * gridDim.x - 1) / (1024ull * gridDim.x));
+    const uint64_t first = (uint64_t(blockIdx.x) * 1024 + t) * per;
+    const uint32_t b0 = uint32_t(min(uint64_t(p.C), first)), b1 = uint32_t(min(uint64_t(p.C), first + per));
     // f(list, queries, per pass: group, tiles)
     auto walk = [&](auto&& f) {
         for (uint32_t l = b0; l < b1; ++l) {
@@ -1541,10 +1554,27 @@ __global__ __launch_bounds__(1024) void plan_lists_kernel(DevPlan p) {
         if (lane == 63) s_tot[w][i] = v;
         run[i] = v - own;
     }
+    if (MODE == PLAN_LISTS && t < uint32_t(A)) {  // the workgroups before this one
+        uint32_t sum = 0;
+#pragma unroll 8
+        for (uint32_t b = 0; b < blockIdx.x; ++b) sum += p.part[b * A + t];
+        s_base[t] = sum;
+    }
     __syncthreads();
+    if constexpr (MODE == PLAN_SUMS) {
+        if (t < uint32_t(A)) {
+            uint32_t sum = 0;
+            for (uint32_t i = 0; i < 16; ++i) sum += s_tot[i][t];
+            p.part[blockIdx.x * A + t] = sum;
+        }
+        return;
+    }
     for (uint32_t i = 0; i < w; ++i)
 #pragma unroll
         for (int j = 0; j < A; ++j) run[j] += s_tot[i][j];
+    if constexpr (MODE == PLAN_LISTS)
+#pragma unroll
+        for (int j = 0; j < A; ++j) run[j] += s_base[j];
     uint32_t* const pre = p.pre;
     const int64_t ld = int64_t(p.C) + 1;
     auto put = [&](uint32_t l) {
@@ -1562,7 +1592,7 @@ __global__ __launch_bounds__(1024) void plan_lists_kernel(DevPlan p) {
         }
         add(nq, g0, t0, g1, t1);
     });
-    if (t == 1023) put(p.C);  // (the last thread's sums end at the totals)
+    if (t == 1023 && blockIdx.x == gridDim.x - 1) put(p.C);  // (the last thread's sums end at the totals)
     if constexpr (ONE) {
         __syncthreads();
         for (uint32_t i = t; i < pairs; i += 1024) {
@@ -1579,14 +1609,19 @@ bool plan_is_one(const DevPlan& p) {
 // Enqueues the device plan (probes -> lists -> tile prefixes); cleared: p.qcnt holds zeros.
 va_status plan_on_device(va_context* ctx, const DevPlan& p, bool cleared) {
     if (plan_is_one(p)) {
-        plan_lists_kernel<true><<<dim3(1), dim3(1024), 0, ctx->stream>>>(p);
+        plan_lists_kernel<PLAN_ONE><<<dim3(1), dim3(1024), 0, ctx->stream>>>(p);
         VA_CHECK_LAUNCH(ctx);
         return VA_OK;
     }
     if (!cleared) VA_CHECK_STATUS(fill_u32(ctx, p.qcnt, p.C, 0));
     plan_probes_kernel<<<dim3(p.Q), dim3(256), 0, ctx->stream>>>(p);
     VA_CHECK_LAUNCH(ctx);
-    plan_lists_kernel<false><<<dim3(1), dim3(1024), 0, ctx->stream>>>(p);
+    const uint32_t blocks = plan_blocks(p.C);
+    if (blocks > 1) {
+        plan_lists_kernel<PLAN_SUMS><<<dim3(blocks), dim3(1024), 0, ctx->stream>>>(p);
+        VA_CHECK_LAUNCH(ctx);
+    }
+    plan_lists_kernel<PLAN_LISTS><<<dim3(blocks), dim3(1024), 0, ctx->stream>>>(p);
     VA_CHECK_LAUNCH(ctx);
     const uint64_t pairs = uint64_t(p.Q) * p.np;
     plan_fill_kernel<<<dim3(uint32_t(std::min<uint64_t>(4096, (pairs + 255) / 256))), dim3(256), 0, ctx->stream>>>(p);
@@ -2012,6 +2047,7 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
                         Scratch::round(uint64_t(Q) * Dp * 2) + Scratch::round(pairs * 4) * 2 +
                         Scratch::round(uint64_t(C) * 4) * 2 + Scratch::round((uint64_t(C) + 1) * 4) +
                         Scratch::round(uint64_t(2 * kGroups) * (uint64_t(C) + 1) * 4) +
+                        Scratch::round(uint64_t(plan_blocks(C)) * kPlanSums * 4) +
                         Scratch::round(uint64_t(Q) * cand * 4) * 3 + Scratch::round(uint64_t(Q) * rcap * 4) * 3 +
                         fb_bytes(Q, id_span, k, ivf->N) +
                         (ivf_big_applies(ctx, Q, Dp) ? Scratch::round(pairs * 16) + Scratch::round(pairs * 8) : 0);
@@ -2049,6 +2085,7 @@ va_status ivf_scan_screened(va_context* ctx, const va_ivf* ivf, const float* que
     dp.qfill = s.carve<uint32_t>(C);
     dp.qoff = s.carve<uint32_t>(uint64_t(C) + 1);
     dp.pre = s.carve<uint32_t>(uint64_t(2 * kGroups) * (uint64_t(C) + 1));
+    dp.part = s.carve<uint32_t>(uint64_t(plan_blocks(C)) * kPlanSums);
     float* cdot = s.carve<float>(uint64_t(Q) * cand);  // becomes the keys of the upper bounds
     uint32_t* clo = s.carve<uint32_t>(uint64_t(Q) * cand);
     uint32_t* cpos = s.carve<uint32_t>(uint64_t(Q) * cand);
@@ -2401,6 +2438,7 @@ va_status ivf_scan_masked(va_context* ctx, const va_ivf* ivf, const float* queri
     const size_t need = Scratch::round(uint64_t(Q) * 4) * 3 + Scratch::round(256) + Scratch::round(pairs * 4) * 2 +
                         Scratch::round(uint64_t(C) * 4) * 2 + Scratch::round((uint64_t(C) + 1) * 4) +
                         Scratch::round(uint64_t(2 * va::kGroups) * (uint64_t(C) + 1) * 4) +
+                        Scratch::round(uint64_t(va::plan_blocks(C)) * va::kPlanSums * 4) +
                         Scratch::round(uint64_t(Q) * cand * 4) * 2 + va::fb_bytes(Q, id_span, k, ivf->N);
     VA_CHECK_STATUS(s.reserve(need));
     uint32_t* thr = s.carve<uint32_t>(Q);
@@ -2420,6 +2458,7 @@ va_status ivf_scan_masked(va_context* ctx, const va_ivf* ivf, const float* queri
     dp.qfill = s.carve<uint32_t>(C);
     dp.qoff = s.carve<uint32_t>(uint64_t(C) + 1);
     dp.pre = s.carve<uint32_t>(uint64_t(2 * va::kGroups) * (uint64_t(C) + 1));
+    dp.part = s.carve<uint32_t>(uint64_t(va::plan_blocks(C)) * va::kPlanSums);
     uint32_t* ckey = s.carve<uint32_t>(uint64_t(Q) * cand);
     uint32_t* cid = s.carve<uint32_t>(uint64_t(Q) * cand);
     va::FbArgs fb = va::fb_carve(s, Q, id_span, k, ivf->N);
