@@ -132,3 +132,24 @@ def test_sampled_scans_of_small_batches(ctx, oracle, Q, k):
     check_topk(L2SQ, q, x, k, *host[0], *oracle.flat_topk(L2SQ, q, x, k))
     check_topk_exact(*host[1], *oracle.i8_topk(qc, xc, k))
     check_topk_exact(host[2][0], host[2][1].view(np.uint32), *oracle.hamming_topk(qb, xb, k))
+
+
+@pytest.mark.parametrize("Q,N,D", [(40, 74_678, 2048), (40, 74_679, 2048), (9, 1_000_000, 1732), (9, 1_000_000, 1736)])
+def test_filter_streamed_or_gemm(ctx, Q, N, D):
+    """Either side of the line between the streamed filter pass and the GEMM's, at Q past and below 32: the
+    same keys, those of the all-pairs GEMM bit for bit (ties to the lower id)."""
+    import torch
+
+    k = 20
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    x, q = torch.randn(N, D, device="cuda", generator=gen), torch.randn(Q, D, device="cuda", generator=gen)
+    i, d = ctx.empty((Q, k), torch.int32), ctx.empty((Q, k), torch.float32)
+    m = ctx.empty((Q, N), torch.float32)
+    ctx.order_after_torch()
+    ctx.check(ctx.lib.va_fused_topk(ctx.handle, L2SQ, q.data_ptr(), x.data_ptr(), Q, N, D, k, i.data_ptr(), d.data_ptr()),
+              "va_fused_topk")
+    ctx.check(ctx.lib.va_l2_all_pairs(ctx.handle, q.data_ptr(), x.data_ptr(), m.data_ptr(), Q, N, D, 0), "l2")
+    ctx.synchronize()
+    want, ids = m.sort(dim=1, stable=True)
+    np.testing.assert_array_equal(d.cpu().numpy(), want[:, :k].cpu().numpy())
+    np.testing.assert_array_equal(i.cpu().numpy(), ids[:, :k].to(torch.int32).cpu().numpy())

@@ -628,12 +628,23 @@ __global__ __launch_bounds__(256, R > 4 ? 1 : 2) void dist_stream_kernel(DistArg
 // or so few GEMM tiles that the chip would be mostly idle (past that the GEMM's tiles read the rows
 // once for up to 128 queries: 500,000 x 768, Q = 40 595 us on them, 810 streamed; 4,096 x 768 centroids,
 // Q = 1,024 86 and 110), every offset within a tile below 2^31.
-bool stream_ok(const va_context* ctx, const DistArgs& a, int wq, int wn) {
+// Every wave reads its 32 queries again for each tile of rows, which costs a filter pass over many long
+// rows more than the GEMM's shared stages and latency: about (Q - 6) per value of a row against a fixed
+// 60 to 150 us.  Whole searches, streamed / GEMM, us: 2M x 768, Q = 8 1,457 / 1,399, 16 1,642 / 1,429, 32
+// 1,992 / 1,432; 500,000 x 768, Q = 16 454 / 407, 32 542 / 411; 1M x 512, Q = 16 519 / 543, 32 621 / 547;
+// 130,000 x 768, Q = 64 271 / 185.  Short rows (2M x 100, Q = 32 316 / 390; 1M x 300, Q = 24 420 / 439) and
+// rows the GEMM cannot load as 16-byte pieces (1M x 513, Q = 32 848 / 1,044) are streamed.
+constexpr uint32_t kStreamDims = 384;
+constexpr uint64_t kStreamWork = 5'200'000'000ull;
+bool stream_ok(const va_context* ctx, const DistArgs& a, int wq, int wn, bool vec) {
     if (a.wq || a.wn || a.plan.pre || a.gather || a.qrow || a.ids || (a.out != OUT_KEYS && a.out != OUT_FILTER)) return false;
     if (a.op != OP_L2SQ && a.op != OP_L2 && a.op != OP_COS_DIST && a.op != OP_NEG_DOT) return false;
     if (uint64_t(ceil_div(a.N, 32)) * ceil_div(a.Q, 32) >= (1ull << 31)) return false;
     if (uint64_t(31) * uint64_t(a.ldq) * 4 + uint64_t(a.D) * 4 > kDmaMaxBytes ||
         uint64_t(31) * uint64_t(a.ldx) * 4 + uint64_t(a.D) * 4 > kDmaMaxBytes)
+        return false;
+    if (vec && a.out == OUT_FILTER && a.Q > 6 && a.D >= kStreamDims &&
+        uint64_t(a.N) * a.D >= kStreamWork / (a.Q - 6))
         return false;
     if (a.Q <= 32) return true;
     const uint64_t waves = uint64_t(ceil_div(a.N, 32)) * ceil_div(a.Q, 32);
@@ -679,7 +690,7 @@ va_status launch_dist(va_context* ctx, const DistArgs& a) {
     }
     const int wq = a.wq ? a.wq : (a.Q <= 32 ? 1 : (a.Q <= 64 ? 2 : 4));
     const int wn = a.wn ? a.wn : 4 / wq;
-    if (stream_ok(ctx, a, wq, wn))
+    if (stream_ok(ctx, a, wq, wn, vec))
         return a.out == OUT_KEYS ? launch_stream<OUT_KEYS>(ctx, a) : launch_stream<OUT_FILTER>(ctx, a);
 #define VA_DIST_CASE(W, N, O) \
     if (wq == W && wn == N && a.out == O) return launch_shape<W, N, O>(ctx, a, vec);
