@@ -488,6 +488,7 @@ struct SelectArgs {
     uint32_t min_count = 0;
     // every key is below 2^key_bits (Hamming distances: a few bits)
     uint32_t key_bits = 32;
+    bool spread = false;  // the keys are not expected to lie close together
     // segmented rows (dense keys only): selection row r takes keys [seg (r % nseg), + seg) of dense
     // row r / nseg; `rows` counts segments, ids are columns of the dense row; every segment begins
     // within the row (select_segments)

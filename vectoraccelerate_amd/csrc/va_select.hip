@@ -76,7 +76,7 @@ va_status launch_select(va_context* ctx, const SelectArgs& a) {
     // entries a large copy would leave one workgroup per CU, so such rows are read from memory
     // (L2-resident lists) by many workgroups at once instead; and so are dense rows of that length
     // when not all of them would be on the chip at once (1,000 rows of 16,384 keys, k = 600
-    // 321 -> 126 us; 600 of 8,193, which are, 70 from their copies, 78 without).
+    // 321 -> 118 us; 600 of 8,193, which are, 70 from their copies, 78 without).
     const uint32_t n = a.nseg ? a.seg : a.n;
     constexpr uint32_t kLds = 160 * 1024;
     const bool resident = a.rows <= uint64_t(ctx->num_cus) * (kLds / (n * 4ull + sizeof(SelectLds<false>)));
@@ -115,6 +115,7 @@ va_status launch_select_dense(va_context* ctx, const SelectArgs& a, const Segmen
     p.seg = seg.len;
     p.nseg = seg.n;
     p.key_bits = a.key_bits;
+    p.spread = a.spread;
     p.out_idx = wid;
     p.out_key = wkey;
     VA_CHECK_STATUS(launch_select(ctx, p));
@@ -123,6 +124,7 @@ va_status launch_select_dense(va_context* ctx, const SelectArgs& a, const Segmen
     m.ids = wid;
     m.ld = int64_t(seg.n) * a.k;
     m.n = seg.n * a.k;
+    m.spread = false;
     return launch_select(ctx, m);
 }
 
@@ -160,6 +162,7 @@ va_status va_topk_select(va_context* ctx, const float* values, uint32_t num_rows
     a.out_idx = out_idx;
     a.out_f = out_values;
     a.key_kind = mode == VA_SELECT_MAX ? 1 : 0;
+    a.spread = true;
     return va::launch_select_dense(ctx, a, seg, wkey, wid);
 }
 

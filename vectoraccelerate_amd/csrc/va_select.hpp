@@ -286,9 +286,11 @@ __device__ void select_row(const SelectArgs& a, uint32_t row, SelectLds<KTH>& ld
             T = radix_kth<NT>(lds, [&](auto&& f) { for_keys([&](uint32_t k, uint32_t) { f(k, true); }); }, 0u, a.key_bits,
                               need, eq);
         } else {
-            // A row read from memory: a pass for its keys' range pays where they lie close together (the
-            // winners and candidates of earlier steps); other rows start from the top bits.
-            if (!CACHED && !rv.ids && K > 1) {
+            // A row read from memory: a pass for its keys' range pays where they lie close together, as
+            // distances and the winners of segments do (a sample of 20,000 L2^2 distances, 200 queries:
+            // 14 us, 19 without).  A caller's values may lie anywhere and start from the top bits (3,000
+            // rows of 30,000 N(0, 1) values, k = 600: 589 us, 648 with it).
+            if (!CACHED && a.spread && K > 1) {
                 mn = 0u;
                 mx = 0xFFFFFFFFu;
             } else if (!CACHED) {
