@@ -57,6 +57,7 @@ def parse():
     p.add_argument("--no-extra", action="store_true", help="headline only (no L2 top-10 extra)")
     p.add_argument("--copy-calibration", action="store_true",
                    help="first run a plain 1 GiB device copy (reference point for rocprofv3 FETCH/WRITE_SIZE)")
+    p.add_argument("--details", metavar="FILE", help="also write the whole measurement, texts and breakdowns, to FILE")
     return p.parse_args()
 
 
@@ -917,6 +918,29 @@ def run_small_768(ctx, a):
     return res
 
 
+# phase breakdowns and the like: in the --details file only
+_DETAILS = {"phases_ms", "power_limited_ceiling", "scan_timings"}
+
+
+def digest(v):
+    """The figures of a measurement to five digits, without its texts and breakdowns: with them the
+    printed line was 22 KB, more than a reader of a log's last 12,000 characters gets whole."""
+    if isinstance(v, dict):
+        return {k: digest(x) for k, x in v.items() if not isinstance(x, str) and k not in _DETAILS}
+    return float(f"{v:.5g}") if isinstance(v, float) else v
+
+
+def emit(a, line) -> None:
+    """Prints the one result line; --details FILE gets it with everything that was measured."""
+    if a.details:
+        with open(a.details, "w") as f:
+            json.dump(line, f, indent=1)
+    for key in ("cpu_baseline", "roofline"):  # (the headline's own keep their texts)
+        if line.get(key):
+            line[key] = {k: v for k, v in line[key].items() if k not in _DETAILS}
+    print(json.dumps({**line, "extra": digest(line["extra"])}), flush=True)
+
+
 def main() -> int:
     a = parse()
     if a.gpus != 1:
@@ -943,7 +967,7 @@ def main() -> int:
         extra["mfma_ceiling"] = ceil
     if a.workload == "ceiling":
         ctx.close()
-        print(json.dumps({"metric": METRIC, "value": None, "extra": extra}), flush=True)
+        emit(a, {"metric": METRIC, "value": None, "extra": extra})
         return 0
     if a.workload in ("all", "small"):
         extra["small_batches_1Mx768"] = run_small_768(ctx, a)
@@ -969,7 +993,7 @@ def main() -> int:
         with_hbm_ceiling(c2, ceil)
     ctx.close()
     if c2 is None:
-        print(json.dumps({"metric": METRIC, "value": None, "extra": extra}), flush=True)
+        emit(a, {"metric": METRIC, "value": None, "extra": extra})
         return 0
     cpu_base = c2.pop("cpu_baseline", None)
     roof = with_ceiling(c2.pop("roofline"), ceil, "fp16" if c2["phases_ms"].get("screened") else "fp32")
@@ -996,7 +1020,7 @@ def main() -> int:
         "cpu_baseline": cpu_base,
         "extra": {"configs1_cosine_top100": c2, **extra},
     }
-    print(json.dumps(line), flush=True)
+    emit(a, line)
     return 0
 
 
