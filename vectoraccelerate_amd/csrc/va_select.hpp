@@ -202,9 +202,10 @@ __device__ inline uint32_t kth_key(RadixLds& lds, ForKeys&& for_keys, uint32_t m
 // Exact top-k of one row (every thread of an NT-thread workgroup calls it; a caller that selects
 // several rows in turn puts a barrier between them).  KTH: threshold mode only (a.out_kth
 // set): no winners buffer, so a cached row of up to 16K keys leaves room for two workgroups per CU.
-// CACHED: the row's keys are copied to s_row (LDS) first.
+// CACHED: the row's keys are copied to s_row (LDS) first.  Inlined by force: a call copies a (232
+// bytes) to each lane's private memory, also in a fallback that finds nothing to do.
 template <int NT, bool CACHED, bool KTH>
-__device__ void select_row(const SelectArgs& a, uint32_t row, SelectLds<KTH>& lds, uint32_t* s_row) {
+__device__ __forceinline__ void select_row(const SelectArgs& a, uint32_t row, SelectLds<KTH>& lds, uint32_t* s_row) {
     uint32_t& s_cnt = lds.cnt;
     uint32_t *const okey = lds.okey, *const oid = lds.oid;
     const int tid = threadIdx.x;
