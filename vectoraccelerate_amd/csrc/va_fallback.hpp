@@ -525,28 +525,40 @@ __device__ inline void fb_consume(const FbArgs& a, int pass, FbSlot& sl, uint32_
         }
     }
 }
-// The phases of a fallback kernel: pass(p, share) runs the workgroup's share of pass p (work items
-// share, share + gridDim.x, ... of the launch; no barrier inside).
+// Workgroups that take shares of a launch whose passes have `items` work items: one per four items
+// (one per wave), at least one, at most the grid; the others leave at once.
+__device__ inline uint32_t fb_workers(uint64_t items) {
+    return uint32_t(max(uint64_t(1), min(uint64_t(gridDim.x), (items + 3) / 4)));
+}
+// The phases of a fallback kernel, by its G = fb_workers workgroups: pass(p, share) runs the workgroup's
+// share of pass p (work items share, share + G, ...; no barrier inside).  A pass has G shares, the
+// phases between them one per slot (at most G): their work is a slot's, and a share costs two atomics
+// on words that all workgroups wait on.  Few listed queries of many, us a search with seven launches /
+// 1,024 shares in every phase / now: 21,548 x 64 bits, 2 of 276 676 / 1,235 / 630; 180,202 x 768, 1 of 200
+// 2,324 / 2,625 / 2,303; 194,587 x 8 (a pass is a few us), 1 of 200 411 / 944 / 619.
 template <class Pass>
-__device__ inline void fb_phases(const FbArgs& a, const SelectArgs& sel, uint32_t n, Pass&& pass) {
+__device__ inline void fb_phases(const FbArgs& a, const SelectArgs& sel, uint32_t n, uint32_t G, Pass&& pass) {
     __shared__ uint32_t s_word;
     __shared__ SelectLds<false> s_sel;
-    const uint32_t G = gridDim.x;
+    if (blockIdx.x >= G) return;
+    const uint32_t R = min(n, G);  // shares of the even phases
     for (;;) {
         if (threadIdx.x == 0) s_word = atomicAdd(a.sync + FBS_TICKET, 1u);
         __syncthreads();
-        const uint32_t phase = s_word / G, share = s_word % G;
+        const uint32_t two = s_word / (R + G), rest = s_word % (R + G);
+        const uint32_t phase = 2 * two + (rest >= R ? 1u : 0u), share = rest >= R ? rest - R : rest;
+        const uint32_t shares = phase & 1 ? G : R;
         if (phase >= kFbPhases) return;
         if (phase > 0) {
             if (threadIdx.x == 0) {
                 while (!__hip_atomic_load(a.sync + FBS_READY + phase - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                    __builtin_amdgcn_s_sleep(1);
+                    __builtin_amdgcn_s_sleep(4);
                 __threadfence();  // what the phase before wrote is visible to the workgroup
             }
             __syncthreads();
         }
         if (phase == kFbPhases - 1) {
-            for (uint32_t s = share; s < n; s += G) {
+            for (uint32_t s = share; s < n; s += shares) {
                 select_row<256, false, false>(sel, s, s_sel, nullptr);
                 __syncthreads();
             }
@@ -555,7 +567,7 @@ __device__ inline void fb_phases(const FbArgs& a, const SelectArgs& sel, uint32_
         const int p = int(phase - 1) / 2;  // of phases past the clear
         uint32_t* done;                    // shares of the phase done
         if (phase == 0) {
-            const uint64_t step = uint64_t(G) * 256, i0 = uint64_t(share) * 256 + threadIdx.x;
+            const uint64_t step = uint64_t(shares) * 256, i0 = uint64_t(share) * 256 + threadIdx.x;
             for (uint64_t i = i0; i < uint64_t(n) * kFbKeyBins; i += step) a.hist[i] = 0;
             for (uint64_t i = i0; i < uint64_t(n) * kFbTieBins; i += step) a.tidh[i] = 0;
             for (uint64_t i = i0; i < uint64_t(n) * 8; i += step) a.st[i] = 0;
@@ -566,7 +578,7 @@ __device__ inline void fb_phases(const FbArgs& a, const SelectArgs& sel, uint32_
             if (p < 4 || a.sync[FBS_TIES]) pass(p, share);
             done = a.done + p;
         } else {
-            for (uint32_t s = share; s < n; s += G) fb_resolve(a, p, s);
+            for (uint32_t s = share; s < n; s += shares) fb_resolve(a, p, s);
             done = a.sync + FBS_RESOLVED + p;
         }
         // the last workgroup to finish the phase publishes it (nobody waits here)
@@ -574,7 +586,7 @@ __device__ inline void fb_phases(const FbArgs& a, const SelectArgs& sel, uint32_
         __syncthreads();
         if (threadIdx.x == 0) {
             __threadfence();
-            if (atomicAdd(done, 1u) == G - 1)
+            if (atomicAdd(done, 1u) == shares - 1)
                 __hip_atomic_store(a.sync + FBS_READY + phase, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
@@ -587,8 +599,8 @@ __global__ __launch_bounds__(256) void fb_kernel(P p, FbArgs a, SelectArgs sel) 
     const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5;
     const uint32_t ngr = (n + 31) / 32, ntl = (a.N + 31) / 32;
     const uint64_t items = uint64_t(ngr) * ntl;
-    const uint32_t nw = gridDim.x * 4;
-    fb_phases(a, sel, n, [&](int pass, uint32_t share) {
+    const uint32_t G = fb_workers(items), nw = G * 4;
+    fb_phases(a, sel, n, G, [&](int pass, uint32_t share) {
         for (uint64_t it = uint64_t(share) * 4 + (threadIdx.x >> 6); it < items; it += nw) {
             const uint32_t g = uint32_t(it / ntl), t = uint32_t(it % ntl);
             const uint32_t s = g * 32 + l32;

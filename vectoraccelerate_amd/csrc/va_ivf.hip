@@ -1826,8 +1826,8 @@ __global__ __launch_bounds__(256) void fb_ivf_kernel(FbIvf v, FbArgs a, SelectAr
     if (n == 0) return;  // nothing overflowed: every workgroup leaves at once
     const int lane = threadIdx.x & 63;
     const uint64_t items = uint64_t(n) * v.np * v.tmax;
-    const uint32_t nw = gridDim.x * 4;
-    fb_phases(a, sel, n, [&](int pass, uint32_t share) {
+    const uint32_t G = fb_workers(items), nw = G * 4;
+    fb_phases(a, sel, n, G, [&](int pass, uint32_t share) {
         for (uint64_t it = uint64_t(share) * 4 + (threadIdx.x >> 6); it < items; it += nw) {
             const uint32_t t = uint32_t(it % v.tmax);
             const uint64_t sp = it / v.tmax;
