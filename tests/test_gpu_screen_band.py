@@ -86,3 +86,26 @@ def test_long_lists(ctx, Q, rank_of_k, gone):
         for o in options:
             ctx.set_option(o, 0)
         ix.close()
+
+
+@pytest.mark.parametrize("Q,k,gone,sample", [(40, 200, True, 4096), (40, 400, True, 16_384), (256, 1000, True, 16_384),
+                                             (40, 1000, False, 4096), (32, 1000, True, 4096)])
+def test_sample_of_middling_batches(ctx, Q, k, gone, sample):
+    """With deletions the lists hold about k N / S rows: middling batches keep the larger sample where
+    those would be long."""
+    N, D = 60_000, 32
+    rng = np.random.default_rng(Q + k)
+    x = rng.standard_normal((N, D)).astype(np.float32)
+    q = rng.standard_normal((Q, D)).astype(np.float32)
+    live = np.arange(N, dtype=np.uint32)
+    ix = _Index(ctx, x)
+    try:
+        if gone:
+            rows = rng.choice(N, N // 50, replace=False)
+            _remove(ctx, ix, rows, False)
+            live = np.delete(live, rows)
+        gi, gd, t = ix.search(L2SQ, q, k)
+        assert t["screened"] == 2 and t["sample_rows"] == sample, t
+        _same((gi, gd), _fp32_scan(ctx, L2SQ, q, x[live], k), live)
+    finally:
+        ix.close()

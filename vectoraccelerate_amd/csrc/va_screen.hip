@@ -1629,12 +1629,17 @@ va_status screen_prepare_queries(va_context* ctx, const float* q, uint32_t Q, ui
 // candidates that it is 2% slower than N/64; for 100,000 rows and 100 queries 4,096 rows instead
 // of 16,384 take the sample from 27 to 20 us.)  With excluded rows the threshold is the sample's k-th
 // bound itself, which lets through k N / S rows: long lists for N/256 (1M x 384, k = 10,
-// 1,000 deleted, Q = 32: 418 -> 310 us).
+// 1,000 deleted, Q = 32: 418 -> 310 us), and for middling batches where that passes kMaskedList
+// (max(16384, N/64) rows / max(4096, N/64), us, 1 % deleted: 30,000 x 64, Q = 220, k = 200 116 / 105,
+// 1000 138 / 149; 100,000 x 384, Q = 100, k = 200 159 / 157, 500 180 / 204; 400,000 x 384, Q = 220,
+// k = 200 356 / 388, 1000 520 / 782).
+constexpr uint64_t kMaskedList = 4096;
 ScanPlan screen_plan(const va_context* ctx, const ScreenInput& in, uint32_t k) {
     const bool small = in.Q <= kSmallBatchMax, middling = in.Q <= kSmallGminMax && in.N > kMinSample;
-    if (in.xh && (small || middling) && !ctx->opt_sample_rows)
-        return plan_scan_for(dense_budget(ctx), std::max<uint64_t>(4096, in.N / (small && !in.masked ? 256 : 64)),
-                             ctx->opt_candidate_cap, in.Q, in.N, k);
+    const uint64_t S = std::max<uint64_t>(4096, in.N / (small && !in.masked ? 256 : 64));
+    const bool long_lists = in.masked && !small && uint64_t(k) * in.N > kMaskedList * S;
+    if (in.xh && (small || middling) && !long_lists && !ctx->opt_sample_rows)
+        return plan_scan_for(dense_budget(ctx), S, ctx->opt_candidate_cap, in.Q, in.N, k);
     return plan_scan(ctx, in.Q, in.N, k);
 }
 
