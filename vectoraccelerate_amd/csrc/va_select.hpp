@@ -328,7 +328,7 @@ __device__ __forceinline__ void select_row(const SelectArgs& a, uint32_t row, Se
                         f(t ? rv.id(i) : 0u, t);
                     });
                 },
-                0u, 32u, need, eq);
+                0u, rv.ids ? 32u : 32u - uint32_t(__builtin_clz(n - 1)), need, eq);  // (columns: below n)
     } else if (a.out_kth) {
         // fewer items than k: every key passes
         if (tid == 0) a.out_kth[orow] = 0xFFFFFFFFu;
