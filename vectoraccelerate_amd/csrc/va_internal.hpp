@@ -498,8 +498,8 @@ struct SelectArgs {
     uint32_t* zero_cnt = nullptr;
     uint32_t* zero_words = nullptr;
 };
-// Overflow words of a scan (one carve): [0] queries listed for the fallback, [1] longest rerank
-// list, [kFbSync ..) the fallback's phase words (va_fallback.hpp).  Cleared before the scan.
+// Overflow words of a scan (one carve): [0] queries listed for the fallback, [kFbSync ..) the
+// fallback's phase words (va_fallback.hpp).  Cleared before the scan.
 constexpr uint32_t kZeroWords = 64;
 constexpr uint32_t kFbSync = 8;
 va_status launch_select(va_context* ctx, const SelectArgs& a);
@@ -562,11 +562,9 @@ struct ScanOutputs {
 // keys[r * ld + j] = kAbsentKey for the rows + j * stride (j < cols) that skip excludes
 va_status mask_dense_keys(va_context* ctx, uint32_t* keys, uint32_t rows, uint32_t cols, int64_t ld, uint32_t row0,
                           uint32_t stride, const uint8_t* skip);
-// keys[r * ld + i] (and keys2, when given) = kAbsentKey for the excluded ids[r * ld + i],
-// i < min(counts[r], cap); with id_map the list holds positions p and the row id is id_map[p]
-va_status mask_list_keys(va_context* ctx, uint32_t* keys, uint32_t* keys2, const uint32_t* ids, const uint32_t* counts,
-                         uint32_t rows, uint32_t cap, int64_t ld, const uint8_t* skip,
-                         const uint32_t* id_map = nullptr);
+// keys[r * ld + i] = kAbsentKey for the excluded ids[r * ld + i], i < min(counts[r], cap)
+va_status mask_list_keys(va_context* ctx, uint32_t* keys, const uint32_t* ids, const uint32_t* counts, uint32_t rows,
+                         uint32_t cap, int64_t ld, const uint8_t* skip);
 
 va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t N, uint32_t k,
                           const ScanOutputs& out);

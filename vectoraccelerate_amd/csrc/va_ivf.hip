@@ -2477,7 +2477,7 @@ va_status ivf_scan_masked(va_context* ctx, const va_ivf* ivf, const float* queri
     VA_CHECK_STATUS(va::fill_u32(ctx, thr, Q, 0xFFFFFFFFu));
     VA_CHECK_STATUS(va::fill_u32(ctx, cnt, Q, 0));
     VA_CHECK_STATUS(va::run_planned_pass(ctx, dp, 0, queries, ivf, thr, cnt, ckey, cid, uint32_t(cap_s)));
-    VA_CHECK_STATUS(va::mask_list_keys(ctx, ckey, nullptr, cid, cnt, Q, uint32_t(cap_s), int64_t(cap_s), skip));
+    VA_CHECK_STATUS(va::mask_list_keys(ctx, ckey, cid, cnt, Q, uint32_t(cap_s), int64_t(cap_s), skip));
     {
         va::SelectArgs a;
         a.keys = ckey;
@@ -2496,7 +2496,7 @@ va_status ivf_scan_masked(va_context* ctx, const va_ivf* ivf, const float* queri
     VA_CHECK_STATUS(pm.mark(1));
     VA_CHECK_STATUS(va::run_planned_pass(ctx, dp, 1, queries, ivf, thr, cnt, ckey, cid, uint32_t(cap)));
     VA_CHECK_STATUS(pm.mark(2));
-    VA_CHECK_STATUS(va::mask_list_keys(ctx, ckey, nullptr, cid, cnt, Q, uint32_t(cap), int64_t(cap), skip));
+    VA_CHECK_STATUS(va::mask_list_keys(ctx, ckey, cid, cnt, Q, uint32_t(cap), int64_t(cap), skip));
     va::SelectArgs base;
     base.k = k;
     base.out_idx = out_idx;

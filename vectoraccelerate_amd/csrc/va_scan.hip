@@ -30,19 +30,15 @@ __global__ void mask_dense_kernel(uint32_t* keys, uint32_t cols, int64_t ld, uin
         if (skip[row0 + uint64_t(j) * stride]) k[j] = kAbsentKey;
 }
 
-__global__ void mask_list_kernel(uint32_t* keys, uint32_t* keys2, const uint32_t* __restrict__ ids,
+__global__ void mask_list_kernel(uint32_t* keys, const uint32_t* __restrict__ ids,
                                  const uint32_t* __restrict__ counts, uint32_t cap, int64_t ld,
-                                 const uint8_t* __restrict__ skip, const uint32_t* __restrict__ id_map) {
+                                 const uint8_t* __restrict__ skip) {
     const uint32_t r = blockIdx.y;
     const uint32_t n = min(counts[r], cap);
     for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
         const int64_t o = int64_t(r) * ld + i;
-        uint32_t id = ids[o];
-        if (id != kSentinel && id_map) id = id_map[id];
-        if (id != kSentinel && skip[id]) {
-            keys[o] = kAbsentKey;
-            if (keys2) keys2[o] = kAbsentKey;
-        }
+        const uint32_t id = ids[o];
+        if (id != kSentinel && skip[id]) keys[o] = kAbsentKey;
     }
 }
 
@@ -59,16 +55,14 @@ va_status mask_dense_keys(va_context* ctx, uint32_t* keys, uint32_t rows, uint32
     return VA_OK;
 }
 
-va_status mask_list_keys(va_context* ctx, uint32_t* keys, uint32_t* keys2, const uint32_t* ids, const uint32_t* counts,
-                         uint32_t rows, uint32_t cap, int64_t ld, const uint8_t* skip, const uint32_t* id_map) {
+va_status mask_list_keys(va_context* ctx, uint32_t* keys, const uint32_t* ids, const uint32_t* counts, uint32_t rows,
+                         uint32_t cap, int64_t ld, const uint8_t* skip) {
     if (!skip || rows == 0 || cap == 0) return VA_OK;
     const uint32_t bx = std::min<uint32_t>(16, (cap + 255) / 256);
     for (uint32_t r0 = 0; r0 < rows; r0 += 65535) {
         const uint32_t nr = std::min<uint32_t>(65535, rows - r0);
-        mask_list_kernel<<<dim3(bx, nr), dim3(256), 0, ctx->stream>>>(keys + int64_t(r0) * ld,
-                                                                     keys2 ? keys2 + int64_t(r0) * ld : nullptr,
-                                                                     ids + int64_t(r0) * ld, counts + r0, cap, ld, skip,
-                                                                     id_map);
+        mask_list_kernel<<<dim3(bx, nr), dim3(256), 0, ctx->stream>>>(keys + int64_t(r0) * ld, ids + int64_t(r0) * ld,
+                                                                     counts + r0, cap, ld, skip);
         VA_CHECK_LAUNCH(ctx);
     }
     return VA_OK;
@@ -300,7 +294,7 @@ va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t
     VA_CHECK_STATUS(pm.mark(1));
     VA_CHECK_STATUS(kp.filter(thr, cnt, ckey, cid, uint32_t(cap)));
     VA_CHECK_STATUS(pm.mark(2));
-    VA_CHECK_STATUS(mask_list_keys(ctx, ckey, nullptr, cid, cnt, Q, uint32_t(cap), int64_t(cap), out.skip));
+    VA_CHECK_STATUS(mask_list_keys(ctx, ckey, cid, cnt, Q, uint32_t(cap), int64_t(cap), out.skip));
     ctx->last_scan.scan_launches = 1;
     ctx->last_scan.sample_rows = uint32_t(S);
     ctx->last_scan.candidate_cap = uint32_t(cap);

@@ -1652,7 +1652,7 @@ bool screen_applies(const va_context* ctx, const ScreenInput& in, uint32_t k) {
     const ScanPlan plan = screen_plan(ctx, in, k);
     if (plan.direct) return false;
     // a small batch over a small index: every exact key at once (two or three launches) instead of
-    // the screen's twelve (5,000 x 128, Q = 1: 54 -> 19 us)
+    // the screen's eight (5,000 x 128, Q = 1: 54 us with what were twelve then, 17 dense)
     if (in.xh && in.Q <= kSmallBatchMax && in.N <= kMinSample && !ctx->opt_sample_rows && !ctx->opt_candidate_cap &&
         !ctx->opt_sample_rank && ctx->opt_screen != 2)
         return false;
