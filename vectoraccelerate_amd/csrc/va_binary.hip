@@ -314,23 +314,18 @@ __global__ __launch_bounds__(512, NB == 8 ? 2 : 4) void hamming_mfma_kernel(HamA
         for (uint32_t b0 = 0; b0 < lc; b0 += 64) {
             const uint32_t e = b0 + uint32_t(lane);
             const uint32_t qk = e < lc ? s_qk[e] : 256u, qi = q0 + (qk & 255u);
-            // One atomic for the passes of a query that has many of them here (runs of equal rows; 300,000
-            // x 512 bits in 50 runs, Q = 21: 64 atomics on one counter took the scan from 26 us to 1.1 ms)
-            uint64_t rest = __ballot(e < lc);
-            uint32_t pos = 0;
-            while (rest) {
-                const int l = __builtin_ctzll(rest);
-                const uint32_t f = uint32_t(__builtin_amdgcn_readlane(int(qk & 255u), l));
-                const uint64_t same = __ballot((qk & 255u) == f) & rest;
-                if (__popcll(same) < 8) break;
-                uint32_t base = 0;
-                if (lane == l) base = atomicAdd(a.cnt + qi, uint32_t(__popcll(same)));
-                base = uint32_t(__builtin_amdgcn_readlane(int(base), l));
-                if ((same >> lane) & 1ull) pos = base + uint32_t(__popcll(same & ((1ull << lane) - 1)));
-                rest &= ~same;
-            }
-            if ((rest >> lane) & 1ull) pos = atomicAdd(a.cnt + qi, 1u);
-            if (e < lc) {
+            // One atomic where all passes are one query's (runs of equal rows; 300,000 x 512 bits in 50 runs,
+            // Q = 21: 64 atomics on one counter were 1.1 ms of scan, now 0.26).  A loop over the queries that
+            // share a flush costs the kernel registers: 24 words, Q = 100 spilled more, 533 us a search of 10M
+            // rows on an idle card instead of 495.
+            const bool in = e < lc;
+            const uint64_t same = __ballot(in && (qk & 255u) == uint32_t(__builtin_amdgcn_readfirstlane(int(qk & 255u))));
+            const bool many = __popcll(same) >= 8 && same == __ballot(in);
+            uint32_t pos = __builtin_amdgcn_mbcnt_hi(uint32_t(same >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(same), 0u));
+            uint32_t base = 0;
+            if (in && (!many || pos == 0)) base = atomicAdd(a.cnt + qi, many ? uint32_t(__popcll(same)) : 1u);
+            pos = many ? pos + uint32_t(__builtin_amdgcn_readfirstlane(int(base))) : base;
+            if (in) {
                 if (pos < a.cap) {
                     a.cand_key[int64_t(qi) * a.cap + pos] = qk >> 8;
                     a.cand_id[int64_t(qi) * a.cap + pos] = s_id[e];
