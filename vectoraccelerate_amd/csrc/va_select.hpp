@@ -128,14 +128,26 @@ __device__ inline uint32_t kth_of_few(RadixLds& lds, uint32_t few, uint32_t& nee
 // The need-th smallest value of the items for_vals(f) runs f(value, taken) over, all within
 // [base, base + 2^bits): histograms of up to 11 bits at a time, from the top, until the bin that
 // holds it has at most SEL_FEW items (the tail of a spread of distances: usually after the
-// first), which are ranked directly.  need becomes its rank among the items equal to it, eq
-// their number.  Every thread of an NT-thread workgroup calls it.
+// first), which are ranked directly; eq, the number of items taken, at once where that few.  need
+// becomes its rank among the items equal to it, eq their number.  Every thread of an NT-thread
+// workgroup calls it.
 template <int NT, class ForVals>
 __device__ inline uint32_t radix_kth(RadixLds& lds, ForVals&& for_vals, uint32_t base, uint32_t bits, uint32_t& need,
                                      uint32_t& eq) {
     const int tid = threadIdx.x;
     uint32_t prefix = 0;
     uint32_t left = bits;
+    // (1,024 threads are for long rows: there the path would only cost registers, and past 80 SGPRs a CU
+    // holds one such workgroup instead of two)
+    if (NT <= 256 && left && eq <= SEL_FEW) {
+        if (tid == 0) lds.cnt = 0;
+        __syncthreads();
+        for_vals([&](uint32_t v, bool taken) {
+            if (taken) lds.whist[atomicAdd(&lds.cnt, 1u)] = v;
+        });
+        __syncthreads();
+        return kth_of_few(lds, eq, need, eq);
+    }
     while (left) {
         const uint32_t w = left < SEL_BITS ? left : SEL_BITS, sh = left - w, nb = 1u << w;
         for (uint32_t b = tid; b < nb; b += NT) lds.whist[b] = 0;
