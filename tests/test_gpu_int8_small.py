@@ -35,3 +35,10 @@ def test_small_scan(ctx, oracle, D, Q, N, k, sample):
     finally:
         ctx.set_option(_lib.VA_OPT_SAMPLE_ROWS, 0)
     check_topk_exact(i.cpu().numpy().view(np.uint32), d.cpu().numpy(), *oracle.i8_topk(q, x, k))
+
+
+@pytest.mark.parametrize("D", [20, 64, 512, 528])
+@pytest.mark.parametrize("Q,N", [(32, 500), (33, 2047), (64, 2048), (65, 4095), (128, 4096)])
+def test_dense_keys_of_few_rows(ctx, oracle, D, Q, N):
+    """Either side of the lines below which the LDS-tiled kernel takes the dense keys."""
+    test_small_scan(ctx, oracle, D, Q, N, 7, 0)

@@ -1240,9 +1240,15 @@ bool i8_vec(const I8Args& a) {
 
 va_status launch_i8(va_context* ctx, const I8Args& a, bool filter) {
     if (a.Q == 0 || a.N == 0) return VA_OK;
-    const bool small = i8_small_ok(a);
-    if (small && a.Q <= kI8SmallQueries) return launch_i8_small(ctx, a, filter);
     const bool vec = i8_vec(a);
+    // The dense keys of few rows are too few wave tiles for the streaming kernel, whose workgroups each
+    // bring all queries into LDS first: the LDS-tiled kernel takes them.  Whole searches, k = 3, streamed
+    // / tiled, us: 300 x 64, Q = 57 18.7 / 17.7; 1,000 x 64, Q = 57 27.4 / 20.2, 128 30.2 / 21.6; 1,000 x 512,
+    // Q = 100 35.0 / 23.9; 4,095 x 512, Q = 128 34.1 / 24.5; 2,000 x 1024, Q = 57 27.6 / 29.9.
+    const bool few_rows = (vec || a.D <= 32) && !filter && a.Q > 32 && a.Q <= kI8SmallQueries &&
+                          (a.Q > 64 ? a.N < 4096 : a.N < 2048 && a.D <= 512);
+    const bool small = !few_rows && i8_small_ok(a);
+    if (small && a.Q <= kI8SmallQueries) return launch_i8_small(ctx, a, filter);
     if (filter && resq16_ok(a, vec)) return launch_i8_resq16(ctx, a);
     if (filter && resq_ok(a, vec)) return launch_i8_resq(ctx, a);
 #ifndef VA_I8_DMA
