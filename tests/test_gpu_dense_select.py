@@ -153,3 +153,26 @@ def test_filter_streamed_or_gemm(ctx, Q, N, D):
     want, ids = m.sort(dim=1, stable=True)
     np.testing.assert_array_equal(d.cpu().numpy(), want[:, :k].cpu().numpy())
     np.testing.assert_array_equal(i.cpu().numpy(), ids[:, :k].to(torch.int32).cpu().numpy())
+
+
+@pytest.mark.parametrize("N,Q,k,dense", [(400_003, 1, 10, True), (400_003, 1, 300, False), (400_003, 4, 600, True),
+                                         (900_001, 4, 300, False)])
+def test_dense_or_sampled(ctx, oracle, N, Q, k, dense):
+    """Either side of the line in the winners that one workgroup would merge per row: exact."""
+    import torch
+
+    g = np.random.default_rng(N + k)
+    x = g.integers(0, 2**32, (N, 2), dtype=np.uint64).astype(np.uint32)
+    q = g.integers(0, 2**32, (Q, 2), dtype=np.uint64).astype(np.uint32)
+    xd, qd = ctx.buffer(x.view(np.int32)), ctx.buffer(q.view(np.int32))
+    i, d = ctx.empty((Q, k), torch.int32), ctx.empty((Q, k), torch.int32)
+    ctx.order_after_torch()
+    ctx.set_profiling(True)
+    try:
+        ctx.check(ctx.lib.va_hamming_topk(ctx.handle, qd.data_ptr(), xd.data_ptr(), Q, N, 2, k, i.data_ptr(), d.data_ptr()),
+                  "va_hamming_topk")
+        t = ctx.last_scan_timings()
+    finally:
+        ctx.set_profiling(False)
+    assert (t["sample_rows"] == 0) == dense, t
+    check_topk_exact(i.cpu().numpy().view(np.uint32), d.cpu().numpy().view(np.uint32), *oracle.hamming_topk(q, x, k))

@@ -178,7 +178,16 @@ uint32_t sample_rank(const va_context* ctx, uint32_t k, uint64_t S, uint32_t N, 
 // Measured per search, k = 10, dense against sampled: fp32 768-d, 50,000 rows, Q = 8 57 / 83 us,
 // Q = 40 (2M pairs) 107 / 129, 200,000 rows, Q = 40 (8M) 290 / 286; int8 512-d, 20,000 rows, Q = 160
 // (3.2M) 53 / 56, 50,000 rows, Q = 160 (8M) 89 / 68; PQ, 500,000 rows, Q = 8 (4M) 80 / 83.
+// One workgroup merges the winners of a long row's segments, about n k / max(4096, 16 k) of them, which
+// for a large k takes longer than a sample and a filter pass; those take longer with Q k.  us, dense /
+// sampled (one board): Hamming 256-bit, Q = 1, 300,000 rows, k = 100 40 / 41, 300 63 / 52; 3.9M rows, k = 100
+// 124 / 62, 500 261 / 83; Q = 4, 600,000 rows, k = 300 93 / 74, 1000 101 / 116; int8 64-d, 900,000 rows, Q = 1,
+// k = 200 71 / 54; Q = 4, k = 1000 104 / 115; fp32 64-d, 3.9M rows, Q = 1, k = 10 290 / 298, 200 393 / 306.
 constexpr uint64_t kDensePairs = 4ull << 20;
+static bool dense_pays(const va_context* ctx, uint32_t Q, uint32_t N, uint32_t k) {
+    const uint64_t winners = uint64_t(select_segments(N, k, Q, uint32_t(ctx->num_cus)).n) * k;
+    return uint64_t(Q) * N <= kDensePairs && winners <= 10240 + 16ull * Q * k;
+}
 va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t N, uint32_t k,
                           const ScanOutputs& out) {
     SelectArgs base;
@@ -195,8 +204,8 @@ va_status exact_topk_scan(va_context* ctx, KeyProducer& kp, uint32_t Q, uint32_t
     const bool automatic = !ctx->opt_candidate_cap && !ctx->opt_sample_rows && !ctx->opt_sample_rank;
     const ScanPlan plan = plan_scan(ctx, Q, N, k);
     const uint64_t S = plan.S;
-    const bool direct = plan.direct || (automatic && uint64_t(Q) * N <= kDensePairs &&
-                                        uint64_t(Q) * N * 4 <= dense_budget(ctx));
+    const bool direct =
+        plan.direct || (automatic && dense_pays(ctx, Q, N, k) && uint64_t(Q) * N * 4 <= dense_budget(ctx));
     ScanPhaseMarks pm(ctx);
     ctx->last_scan = va_scan_timings{};
     VA_CHECK_STATUS(pm.mark(0));
