@@ -131,8 +131,15 @@ __global__ __launch_bounds__(kThreads, 2) void i8_small_kernel(I8Args a) {
 #pragma unroll
                     for (int v = 0; v < 4; ++v)
                         pass |= uint32_t((acc[m][n][v] >= cut[n]) & (16u * m + 4u * g + v < rc)) << (4 * m + v);
-                if (q >= a.Q || !pass) continue;
-                uint32_t pos = atomicAdd(a.cnt + q, uint32_t(__popc(pass)));
+                if (q >= a.Q) pass = 0;
+                // one atomic for the four lanes of a query: their places in lane order
+                const uint32_t c = uint32_t(__popc(pass));
+                const uint32_t c16 = uint32_t(__shfl_xor(int(c), 16)), pair = c + c16;
+                const uint32_t other = uint32_t(__shfl_xor(int(pair), 32));
+                uint32_t pos = 0;
+                if (g == 0 && pair + other) pos = atomicAdd(a.cnt + q, pair + other);
+                pos = uint32_t(__shfl(int(pos), int(r16))) + (g & 1 ? c16 : 0u) + (g & 2 ? other : 0u);
+                if (!pass) continue;
 #pragma unroll
                 for (int m = 0; m < MB; ++m)
 #pragma unroll
